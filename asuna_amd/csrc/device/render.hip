@@ -647,25 +647,42 @@ __device__ __forceinline__ void initStack(Stack& st, int* lds, float* ldsT, cons
 // one contiguous slice per XCD; a wave drains the slice of its own XCD
 // first, then helps with the others, so each XCD's L2 serves one run of the
 // pixel-ordered queue instead of rays from the whole image.
+//
+// The fetch counters are device-scope atomics, resolved beyond the XCD's L2
+// one at a time, so waves that cannot get rays stay away from them: wave j
+// of an XCD takes no part when the first fetches of the waves before it
+// cover the slice (surplus).  With every wave of the 2048-block grid adding
+// to all eight counters, a launch with next to no rays lasted 124 us and a
+// fused one 156 us: a 96 x 64 render of the box at 1 spp 1530 -> 530 us;
+// launches with rays for every wave are unchanged (5.2 M triangles, 1080p,
+// 16 spp: 30.4 ms).  Reading a counter before adding to it when a wave goes
+// over to a further slice made that frame slower (33 ms): waves then help
+// other XCDs sooner and share their L2 less.
 struct ChunkFetch {
   uint32_t* ctr;  // first fetch counter (queue order) or first slice counter (XCD)
   uint32_t count;
   uint32_t slice, home, k;
   uint32_t lo, hi;
+  bool surplus;  // the XCD's earlier waves cover the slice with their first fetches
   __device__ __forceinline__ void slicesFor(uint32_t s) {
     lo = s * slice;
     hi = lo < count ? min(count, lo + slice) : lo;
   }
 };
-template <bool XCD>
+// CH: queue entries of a wave's first fetch.
+template <bool XCD, uint32_t CH = 64>
 __device__ __forceinline__ void chunkInit(ChunkFetch& f, uint32_t* ctr, uint32_t count) {
   f.ctr = ctr;
   f.count = count;
   f.k = 0;
+  f.surplus = false;
   if (XCD) {
     f.slice = (count + kXcds - 1) / kXcds;
     f.home = blockIdx.x % kXcds;
     f.slicesFor(f.home);
+    // slices differ in length only at the queue's end, so the rule looks at the longest; wave 0 stays while there are rays
+    const uint32_t j = (blockIdx.x / kXcds) * (kTraceBlock / 64) + (threadIdx.x >> 6);
+    f.surplus = uint64_t(j) * CH >= f.slice;
   } else {
     f.slice = count;
     f.home = 0;
@@ -677,12 +694,14 @@ __device__ __forceinline__ void chunkInit(ChunkFetch& f, uint32_t* ctr, uint32_t
 // atomic fetch; false when the queue is drained.
 template <bool XCD, uint32_t CH = 64>
 __device__ __forceinline__ bool chunkNext(ChunkFetch& f, int lane, uint32_t& start) {
+  if (f.surplus) return false;
   for (;;) {
     uint32_t s = XCD ? (f.home + f.k) % kXcds : 0u;
+    const uint32_t len = f.hi - f.lo;
     uint32_t base = 0;
     if (lane == 0) base = atomicAdd(f.ctr + (XCD ? s * 32u : 0u), CH);
     base = __shfl(base, 0);
-    if (base < f.hi - f.lo) {
+    if (base < len) {
       start = f.lo + base;
       return true;
     }
@@ -812,10 +831,10 @@ __device__ __forceinline__ bool fetchIdle(ChunkFetch& f, bool idle, int lane, bo
   const uint32_t rank = uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
   for (;;) {
     const uint32_t sl = (f.home + f.k) % kXcds;
+    const uint32_t len = f.hi - f.lo;
     uint32_t base = 0;
     if (lane == 0) base = atomicAdd(f.ctr + sl * 32u, n);
     base = __shfl(base, 0);
-    const uint32_t len = f.hi - f.lo;
     if (base < len) {
       idx = f.lo + base + rank;
       bool got = idle && idx < f.hi;
@@ -841,7 +860,7 @@ __device__ __forceinline__ void extendDynLoop(const SceneView& sc, const Wavefro
   const float4 *qo = w.rayO[cur], *qd = w.rayD[cur];
   ChunkFetch f;
   chunkInit<true>(f, &w.ctr[kXcdCtr], count);
-  bool active = false, drained = false;
+  bool active = false, drained = f.surplus;
   uint32_t slot = 0;
   TRay r;
   DynState s;
@@ -1145,7 +1164,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(8, 
   const float4 *qo = w.rayO[cur], *qd = w.rayD[cur];
   uint32_t nN = 0, nT = 0;
   ChunkFetch f;
-  chunkInit<true>(f, &w.ctr[kXcdCtr], count);
+  chunkInit<true, FETCH>(f, &w.ctr[kXcdCtr], count);
   uint32_t start;
   while (chunkNext<true, FETCH>(f, lane, start)) {
    for (uint32_t sub = start; sub < start + FETCH && sub < f.hi; sub += 64) {
@@ -1299,7 +1318,7 @@ __device__ __forceinline__ void shadowDynLoop(const SceneView& sc, const Wavefro
                                               uint32_t& nNodes, uint32_t& nTris) {
   ChunkFetch f;
   chunkInit<true>(f, &w.ctr[kXcdCtr + kXcds * 32], w.ctr[2]);
-  bool active = false, drained = false;
+  bool active = false, drained = f.surplus;
   int pid = -1;
   uint32_t slot = 0;
   float tmax = 0.0f;
@@ -1465,7 +1484,7 @@ __device__ __forceinline__ void extend2LLoop(const SceneView& sc, const Wavefron
   const float4 *qo = w.rayO[cur], *qd = w.rayD[cur];
   ChunkFetch f;
   chunkInit<true>(f, &w.ctr[kXcdCtr], count);
-  bool active = false, drained = false;
+  bool active = false, drained = f.surplus;
   uint32_t slot = 0;
   TRay rw, ro;
   Walk2L s;
@@ -1573,7 +1592,7 @@ __device__ __forceinline__ void shadow2LLoop(const SceneView& sc, const Wavefron
   const uint32_t count = w.ctr[2];
   ChunkFetch f;
   chunkInit<true>(f, &w.ctr[kXcdCtr + kXcds * 32], count);
-  bool active = false, drained = false;
+  bool active = false, drained = f.surplus;
   uint32_t slot = 0;
   int pid = 0;
   float tmax = 0.f;

@@ -153,3 +153,27 @@ def test_autotune_picks_a_candidate_and_keeps_results(renderer, multishot_scene)
     renderer.render_shots(list(cams), list(pcs), 2, graphs=False)
     for i in range(8):
         np.testing.assert_array_equal(tuned[i], renderer.read_shot(i, 0))
+
+
+@pytest.mark.parametrize("two_level", [False, True])
+@pytest.mark.parametrize("w,h", [(1, 1), (9, 7), (16, 4), (73, 7), (64, 64), (65, 63), (256, 130)])
+def test_small_queues_are_traced_whole(renderer, box_scene, w, h, two_level):
+    """Waves that earlier waves' first fetches leave without rays stay away
+    from the queue: at queue lengths around one ray, one wave (64), one wave
+    per XCD slice (512) and one 256-ray camera fetch per slice, every ray is
+    still traced, as the queue-order scheme (which has no such rule) does."""
+    s = A.HostScene(box_scene)
+    renderer.upload(s)
+    renderer.build()
+    cam = A.camera_lookat(w, h, 60.0, (0.0, 0.0, 2.5), (0.0, 0.0, 0.0))
+    _, pc = s.shot(0)
+    renderer.set_film(w, h)
+    ref_st = renderer.render(cam, pc, 0, 2, traversal=1)
+    ref = [renderer.read(i) for i in (0, 1, 8)]
+    if two_level:
+        renderer.build(two_level=True)
+    renderer.set_film(w, h)
+    st = renderer.render(cam, pc, 0, 2)
+    assert st["extension_rays"] == ref_st["extension_rays"] and st["shadow_rays"] == ref_st["shadow_rays"]
+    for a, b in zip(ref, [renderer.read(i) for i in (0, 1, 8)]):
+        np.testing.assert_array_equal(a, b)
