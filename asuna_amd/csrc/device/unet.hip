@@ -4,24 +4,31 @@
 // Every 3x3 convolution is an implicit GEMM on v_mfma_f32_16x16x32_bf16
 // (BF16 operands, FP32 accumulation):
 //   forward      Y[p][co]  = b[co] + sum_tap sum_ci X[p + d(tap)][ci] W[tap][co][ci]
-//                GEMM rows = pixels, cols = cout, K = 9 x cin
+//                GEMM rows = cout, cols = pixels, K = 9 x cin
 //   backward-x   dX[p][ci] = sum_tap sum_co dY[p - d(tap)][co] W[tap][co][ci]
-//                GEMM rows = pixels, cols = cin, K = 9 x cout
+//                the same kernels on dY with the taps reversed and the roles
+//                of cin and cout exchanged in the packed weights
 //   backward-w   dW[tap][co][ci] = sum_p dY[p][co] X[p + d(tap)][ci]
-//                GEMM rows = cout, cols = cin, K = pixels (split over waves;
+//                GEMM rows = cout, cols = cin, K = pixels (split over blocks;
 //                each split writes its partial sums, which a second kernel
-//                adds in split order, so gradients are reproducible)
+//                adds in a fixed order, so gradients are reproducible)
 // Activations are NHWC BF16 with the channel count padded to a multiple of
-// 32 (padding channels hold zeros and their weights stay zero), so an A or B
-// fragment row is one 16-byte load.  Decoder convolutions read their input
+// 32 (padding channels hold zeros and their weights stay zero), so an
+// operand row is one 16-byte load.  Decoder convolutions read their input
 // as two sources -- the half-resolution tensor below, nearest-upsampled on
 // the fly, then the skip tensor -- so neither the upsampled tensor nor the
-// concatenation is materialised.  Gradients are FP32.
+// concatenation is materialised.  Gradients are summed in FP32 and rounded to
+// BF16 once, where they are complete, as the operand of the next products;
+// bias gradients and the weight gradients' partial sums are FP32.
 //
 // MFMA 16x16x32 operand layout (lane l of 64, q = l / 16):
 //   A (16 x 32)  row l % 16, k = 8q .. 8q+7
 //   B (32 x 16)  col l % 16, k = 8q .. 8q+7
 //   D (16 x 16)  col l % 16, rows 4q .. 4q+3
+// With weights as A and pixels as B a lane ends with 4 channels of one pixel
+// per tile.  Row m of tile t (of a 32-channel group's two) is channel
+// 8 (m / 4) + 4 t + m % 4, so the lane's 8 values are channels 8q .. 8q+7 of
+// its pixel and a wave stores 16 pixels x 64 bytes without a transpose.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -39,699 +46,699 @@
 namespace {
 
 typedef __bf16 bf16;
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kLevels = 5;
 constexpr uint32_t kWidths[kLevels] = {32, 48, 64, 96, 128};
 constexpr uint32_t kInCh = 10, kOutCh = 3;
-constexpr int kMaxTiles = 14;  // 224 / 16: widest GEMM column count in 16-wide tiles
+constexpr int kNumLayers = 2 * kLevels + 2 * (kLevels - 1) + 1;
+constexpr uint32_t kMaxChunks = 7;  // 224 / 32: widest input in 32-channel chunks
 
 __host__ __device__ inline uint32_t pad32(uint32_t c) { return (c + 31) & ~31u; }
 
 struct Src {
-  const bf16* a;  // activations [N][h][w][C]
-  float* g;       // gradient, same shape (backward-x target)
+  const bf16* a;  // activations (or a gradient) [N][h][w][C]
   uint32_t C;     // stored channels (multiple of 32)
   uint32_t up;    // 1: half-resolution tensor read nearest-upsampled
+};
+
+// What a convolution computes: a layer's activations, the last layer's
+// prediction, or a backward-x product.
+enum ConvMode { kModeAct, kModeLast, kModeGrad };
+
+// Where a backward-x convolution's output goes, by the tensor its forward
+// convolution read.
+enum GradKind : uint32_t {
+  kGradFinal,  // the tensor's only reader: ReLU mask, BF16
+  kGradUp,     // read upsampled: sum of the 2 x 2 pixels, ReLU mask, BF16 at half resolution
+  kGradPool,   // a pooled tensor: a quarter to each of the 4 pixels of the unpooled one, added to
+               // its skip gradient, ReLU mask, BF16 at full resolution
+  kGradSkip,   // a skip tensor, whose pooled branch follows: FP32
+};
+struct GradDst {
+  uint32_t kind;
+  uint32_t C;       // channels of the tensor
+  bf16* g;          // its complete gradient, masked
+  const bf16* act;  // its activations (the mask)
+  float* skip;      // FP32 skip gradient (written by kGradSkip, read by kGradPool)
+  float* bPart;     // bias-gradient partial sums of the layer that made it: [pixel tile][C]
 };
 
 struct ConvArgs {
   Src s0, s1;  // s1.C == 0: one source
   uint32_t N, H, W;
-  uint32_t Cin, Cout;  // stored, multiples of 32
-  const bf16* Wf;      // [9][Cout][Cin]
-  const bf16* Wb;      // [9][Cin][Cout]
-  const float* bias;   // [Cout]
-  bf16* Y;             // BF16 output, or null
-  float* Yf;           // FP32 output (last layer), or null
-  const float* dY;     // output gradient (ReLU already applied)
-  float* upTmp;        // full-resolution gradient of an upsampled s0
-  float* dW;           // [9][Cout][Cin]
-  float* dB;           // [Cout]
-  float* wPart;        // backward-w partial sums [splits][9][Cout][Cin]
-  uint32_t relu;
-  uint32_t splits;     // backward-w pixel splits
+  uint32_t nCh, nCg;  // 32-channel input chunks and output groups
+  const bf16* Wp;     // packed weights [group][chunk][tap][2 tiles][64 lanes][8]
+  // forward
+  const float* bias;  // [32 nCg]
+  bf16* Y;            // BF16 output [N][H][W][32 nCg] after ReLU, or null: the last layer
+  bf16* pool;         // 2 x 2 average of Y, or null
+  float* Yf;          // last layer: FP32 prediction [pixel][4] (log space), or null
+  float* rgb;         // last layer: expm1 of it, [pixel][3], or null
+  float4* film;       // last layer: max(expm1, 0) as RGBA of the filmW x filmH part, or null
+  uint32_t filmW, filmH;
+  // backward-x: groups [0, cg0) belong to d0, the rest to d1
+  uint32_t cg0;
+  GradDst d0, d1;
 };
 
-__device__ inline void pixelOf(uint32_t p, uint32_t H, uint32_t W, uint32_t& n, int& y, int& x) {
-  x = int(p % W);
-  uint32_t t = p / W;
-  y = int(t % H);
-  n = t / H;
-}
-
-// 8 BF16 channels [c, c + 8) of the input at (n, y, x); zeros outside.
-__device__ inline bf16x8 loadIn(const ConvArgs& a, uint32_t n, int y, int x, uint32_t c) {
+__device__ __forceinline__ bf16x8 zero8() {
   bf16x8 z;
   for (int i = 0; i < 8; ++i) z[i] = bf16(0.0f);
-  if (y < 0 || y >= int(a.H) || x < 0 || x >= int(a.W)) return z;
-  if (c < a.s0.C) {
-    size_t idx = a.s0.up ? ((size_t(n) * (a.H / 2) + uint32_t(y) / 2) * (a.W / 2) + uint32_t(x) / 2) * a.s0.C + c
-                         : ((size_t(n) * a.H + uint32_t(y)) * a.W + uint32_t(x)) * a.s0.C + c;
-    return *reinterpret_cast<const bf16x8*>(a.s0.a + idx);
-  }
-  c -= a.s0.C;
-  size_t idx = ((size_t(n) * a.H + uint32_t(y)) * a.W + uint32_t(x)) * a.s1.C + c;
-  return *reinterpret_cast<const bf16x8*>(a.s1.a + idx);
+  return z;
 }
 
-// One BF16 input value (backward-w B fragment); zero outside.
-__device__ inline float loadIn1(const ConvArgs& a, uint32_t n, int y, int x, uint32_t c) {
-  if (y < 0 || y >= int(a.H) || x < 0 || x >= int(a.W)) return 0.f;
-  if (c < a.s0.C) {
-    size_t idx = a.s0.up ? ((size_t(n) * (a.H / 2) + uint32_t(y) / 2) * (a.W / 2) + uint32_t(x) / 2) * a.s0.C + c
-                         : ((size_t(n) * a.H + uint32_t(y)) * a.W + uint32_t(x)) * a.s0.C + c;
-    return float(a.s0.a[idx]);
-  }
-  c -= a.s0.C;
-  return float(a.s1.a[((size_t(n) * a.H + uint32_t(y)) * a.W + uint32_t(x)) * a.s1.C + c]);
+// One 32-channel chunk of one image of a convolution's input (uniform over
+// the block: sources hold whole chunks).
+struct ChunkSrc {
+  const bf16* p;
+  uint32_t C, w, up;  // channels per pixel, pixels per row, coordinate shift
+};
+__device__ __forceinline__ ChunkSrc chunkSrc(const Src& s0, const Src& s1, uint32_t H, uint32_t W, uint32_t n, uint32_t ch) {
+  const bool first = 32 * ch < s0.C;
+  const Src& s = first ? s0 : s1;
+  ChunkSrc k;
+  k.C = s.C, k.up = s.up, k.w = W >> s.up;
+  k.p = s.a + size_t(n) * (H >> s.up) * k.w * s.C + (32 * ch - (first ? 0u : s0.C));
+  return k;
+}
+// 8 BF16 channels [c, c + 8) of the chunk at pixel (y, x); zeros outside the H x W image.
+__device__ __forceinline__ u32x4 loadIn(const ChunkSrc& k, uint32_t H, uint32_t W, int y, int x, uint32_t c) {
+  u32x4 v = {0, 0, 0, 0};
+  if (uint32_t(y) < H && uint32_t(x) < W)
+    v = *reinterpret_cast<const u32x4*>(k.p + (uint64_t((uint32_t(y) >> k.up) * k.w + (uint32_t(x) >> k.up)) * k.C + c));
+  return v;
 }
 
-// ------------------------------------------------------------- forward
-// Block: 4 waves, each computing PG groups of 16 output pixels for all NT
-// 16-wide output channel tiles; a wave loads each weight fragment once per
-// (tap, 32-channel step) and uses it for its PG pixel groups.
-template <int NT, int PG>
-__global__ __launch_bounds__(256) void kConvFwd(ConvArgs a) {
-  const uint32_t P = a.N * a.H * a.W;
-  const uint32_t lane = threadIdx.x & 63, q = lane >> 4, r16 = lane & 15;
-  const uint32_t p0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (16 * PG);
-  uint32_t n[PG];
-  int y[PG], x[PG];
-  bool pin[PG];
+// The value of the lane whose index differs in bit 0 (the horizontally
+// neighbouring pixel of a pair).
+__device__ __forceinline__ float pairLane(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xf, 0xf, true));
+}
+
+// Bias, activation, store and what follows a convolution, for ROWS pixels
+// (n, y0 .. y0 + ROWS - 1, x) of the lane and the 8 channels 32 cg + 8q + j
+// (y0 even, ROWS = 2, lane pairs hold even and odd x).  All lanes of the wave
+// call it; pixels outside the image are dropped here.  bs: the lane's sums
+// of the complete gradient (backward).
+template <int ROWS, ConvMode MODE>
+__device__ __forceinline__ void emit(const ConvArgs& a, uint32_t cg, uint32_t n, int y0, int x, uint32_t q,
+                                     float (&v)[ROWS][8], float (&bs)[8]) {
+  const int H = int(a.H), W = int(a.W);
+  if (MODE != kModeGrad) {
+    const uint32_t C = 32 * a.nCg, c0 = 32 * cg + 8 * q;
+    float b[8];
+    *reinterpret_cast<float4*>(b) = *reinterpret_cast<const float4*>(a.bias + c0);
+    *reinterpret_cast<float4*>(b + 4) = *reinterpret_cast<const float4*>(a.bias + c0 + 4);
+    if (MODE == kModeLast) {  // channels 0..2, no ReLU
+#pragma unroll 1
+      for (int i = 0; i < ROWS; ++i) {
+        const int y = y0 + i;
+        if (q || cg || y >= H || x >= W) continue;
+        const size_t p = (size_t(n) * a.H + y) * a.W + x;
+        const float f0 = (i ? v[ROWS - 1][0] : v[0][0]) + b[0], f1 = (i ? v[ROWS - 1][1] : v[0][1]) + b[1],
+                    f2 = (i ? v[ROWS - 1][2] : v[0][2]) + b[2];
+        if (a.Yf) *reinterpret_cast<float4*>(a.Yf + 4 * p) = make_float4(f0, f1, f2, 0.f);
+        if (a.rgb) a.rgb[3 * p] = expm1f(f0), a.rgb[3 * p + 1] = expm1f(f1), a.rgb[3 * p + 2] = expm1f(f2);
+        if (a.film && y < int(a.filmH) && x < int(a.filmW))
+          a.film[size_t(y) * a.filmW + x] =
+              make_float4(fmaxf(expm1f(f0), 0.f), fmaxf(expm1f(f1), 0.f), fmaxf(expm1f(f2), 0.f), 1.f);
+      }
+      return;
+    }
 #pragma unroll
-  for (int g = 0; g < PG; ++g) {
-    const uint32_t p = p0 + 16 * g + r16;
-    pin[g] = p < P;
-    n[g] = 0, y[g] = 0, x[g] = 0;
-    if (pin[g]) pixelOf(p, a.H, a.W, n[g], y[g], x[g]);
-  }
-  f32x4 acc[PG][NT];
+    for (int i = 0; i < ROWS; ++i) {
+      bf16x8 o;
 #pragma unroll
-  for (int g = 0; g < PG; ++g)
+      for (int j = 0; j < 8; ++j) {
+        o[j] = bf16(fmaxf(v[i][j] + b[j], 0.f));
+        v[i][j] = float(o[j]);
+      }
+      const int y = y0 + i;
+      if (y < H && x < W) *reinterpret_cast<bf16x8*>(a.Y + ((size_t(n) * a.H + y) * a.W + x) * C + c0) = o;
+    }
+    if (a.pool) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[g][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int tap = 0; tap < 9; ++tap) {
-    const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-    const bf16* wt = a.Wf + size_t(tap) * a.Cout * a.Cin;
-    for (uint32_t c0 = 0; c0 < a.Cin; c0 += 32) {
-      const bf16* wr = wt + c0 + 8 * q;
-      bf16x8 B[NT];
+      for (int i = 0; i < ROWS; i += 2) {
+        bf16x8 o;
 #pragma unroll
-      for (int t = 0; t < NT; ++t) B[t] = *reinterpret_cast<const bf16x8*>(wr + size_t(16 * t + r16) * a.Cin);
-#pragma unroll
-      for (int g = 0; g < PG; ++g) {
-        bf16x8 A;
-        if (pin[g]) {
-          A = loadIn(a, n[g], y[g] + dy, x[g] + dx, c0 + 8 * q);
-        } else {
-          for (int i = 0; i < 8; ++i) A[i] = bf16(0.0f);
+        for (int j = 0; j < 8; ++j) {
+          const float right0 = pairLane(v[i][j]), right1 = pairLane(v[i + 1][j]);
+          o[j] = bf16(0.25f * (v[i][j] + right0 + v[i + 1][j] + right1));
         }
-#pragma unroll
-        for (int t = 0; t < NT; ++t) acc[g][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B[t], acc[g][t], 0, 0, 0);
+        const int y = y0 + i;
+        if (!(x & 1) && y < H && x < W)
+          *reinterpret_cast<bf16x8*>(a.pool + ((size_t(n) * (a.H / 2) + y / 2) * (a.W / 2) + x / 2) * C + c0) = o;
       }
     }
+    return;
   }
+  const GradDst& d = cg < a.cg0 ? a.d0 : a.d1;
+  const uint32_t c0 = 32 * (cg < a.cg0 ? cg : cg - a.cg0) + 8 * q;
+  auto put = [&](size_t e, const float (&g)[8]) {  // masked gradient of elements e .. e + 7
+    const bf16x8 act = *reinterpret_cast<const bf16x8*>(d.act + e);
+    bf16x8 o;
 #pragma unroll
-  for (int g = 0; g < PG; ++g)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const uint32_t co = 16 * t + r16;
-      const float b = a.bias[co];
-      for (int r = 0; r < 4; ++r) {
-        const uint32_t pp = p0 + 16 * g + 4 * q + r;
-        if (pp >= P) continue;
-        float v = acc[g][t][r] + b;
-        if (a.relu) v = fmaxf(v, 0.f);
-        if (a.Y) a.Y[size_t(pp) * a.Cout + co] = bf16(v);
-        if (a.Yf) a.Yf[size_t(pp) * a.Cout + co] = v;
-      }
+    for (int j = 0; j < 8; ++j) {
+      const float m = float(act[j]) > 0.f ? g[j] : 0.f;
+      o[j] = bf16(m);
+      bs[j] += m;
     }
-}
-
-// Tiled forward convolution for the large levels: a block stages an
-// (8 + 2) x (TC + 2) pixel input tile with its halo (all input channels,
-// zeros outside the image) in LDS with coalesced 16-byte loads, then each
-// of its four waves computes 2 rows x TC columns of output pixels (TC / 8
-// groups of 16) for all NT output tiles, reading A fragments from LDS.
-// Pixel stride in LDS: Cin + 8 BF16, which spreads the 16 lanes of a
-// fragment over the banks.
-constexpr int kTileRows = 8;
-template <int NT, int TC>
-__global__ __launch_bounds__(256) void kConvFwdTile(ConvArgs a) {
-  extern __shared__ __align__(16) bf16 tile[];
-  const uint32_t Cin = a.Cin, stride = Cin + 8;
-  const uint32_t tilesX = (a.W + TC - 1) / TC, tilesY = (a.H + kTileRows - 1) / kTileRows;
-  const uint32_t tx0 = (blockIdx.x % tilesX) * TC, ty0 = ((blockIdx.x / tilesX) % tilesY) * kTileRows;
-  const uint32_t n = blockIdx.x / (tilesX * tilesY);
-  // stage: (kTileRows + 2) x (TC + 2) pixels x Cin channels, 8 channels per thread-step
-  const uint32_t chunks = Cin / 8, tw = TC + 2, total = (kTileRows + 2) * tw * chunks;
-  for (uint32_t k = threadIdx.x; k < total; k += 256) {
-    const uint32_t c8 = k % chunks, pix = k / chunks;
-    const int yy = int(ty0) - 1 + int(pix / tw), xx = int(tx0) - 1 + int(pix % tw);
-    *reinterpret_cast<bf16x8*>(tile + pix * stride + 8 * c8) = loadIn(a, n, yy, xx, 8 * c8);
-  }
-  __syncthreads();
-  constexpr int G = TC / 8;  // 16-pixel groups per wave: 2 rows x TC columns
-  const uint32_t lane = threadIdx.x & 63, q = lane >> 4, r16 = lane & 15, wv = threadIdx.x >> 6;
-  f32x4 acc[G][NT];
-#pragma unroll
-  for (int g = 0; g < G; ++g)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) acc[g][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int tap = 0; tap < 9; ++tap) {
-    const int dy = tap / 3, dx = tap % 3;  // tile coordinates are offset by the halo
-    const bf16* wt = a.Wf + size_t(tap) * a.Cout * Cin;
-    for (uint32_t c0 = 0; c0 < Cin; c0 += 32) {
-      const bf16* wr = wt + c0 + 8 * q;
-      bf16x8 B[NT];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) B[t] = *reinterpret_cast<const bf16x8*>(wr + size_t(16 * t + r16) * Cin);
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const uint32_t row = 2 * wv + uint32_t(g) / (TC / 16), col = (uint32_t(g) % (TC / 16)) * 16 + r16;
-        const bf16x8 A =
-            *reinterpret_cast<const bf16x8*>(tile + ((row + dy) * tw + col + dx) * stride + c0 + 8 * q);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) acc[g][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B[t], acc[g][t], 0, 0, 0);
-      }
-    }
-  }
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    const uint32_t y = ty0 + 2 * wv + uint32_t(g) / (TC / 16);
-    if (y >= a.H) continue;
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const uint32_t co = 16 * t + r16;
-      const float b = a.bias[co];
-      for (int r = 0; r < 4; ++r) {
-        const uint32_t x = tx0 + (uint32_t(g) % (TC / 16)) * 16 + 4 * q + r;
-        if (x >= a.W) continue;
-        const size_t pp = (size_t(n) * a.H + y) * a.W + x;
-        float v = acc[g][t][r] + b;
-        if (a.relu) v = fmaxf(v, 0.f);
-        if (a.Y) a.Y[pp * a.Cout + co] = bf16(v);
-        if (a.Yf) a.Yf[pp * a.Cout + co] = v;
-      }
-    }
-  }
-}
-
-// K-chunked tiled forward convolution for the large levels: a block owns
-// an 8-row x 32-column output tile and walks the input channels in chunks
-// of 32.  Per chunk it stages in LDS, with coalesced 16-byte loads, the
-// chunk of its (8 + 2) x (32 + 2) input tile with the halo (zeros outside
-// the image), and the chunk's weights of all cout for TG taps at a time
-// (all 9 for two output tiles, 3 for four, keeping a block under 64 KB);
-// each wave computes 2 rows x 32 columns (4 groups of 16 pixels) for all
-// NT output tiles with every MFMA operand read from LDS.  Row stride in
-// LDS: 40 BF16 (80 bytes), which spreads a fragment's 16 lanes over the
-// banks.
-constexpr int kChunkRows = 8, kChunkCols = 32, kChunkStride = 40;
-// taps whose weights a block stages in LDS at a time: 3 (a smaller LDS
-// share, hence more resident blocks, pays for the two extra barriers; 9
-// taps for 32-channel layers measured 4 % slower, 1 tap slower still)
-template <int NT> constexpr int chunkTaps() { return 3; }
-// 64 output channels: 3 waves per SIMD (160 VGPRs without spills, where the
-// unconstrained 192 allow 2; the LDS share allows 3): 1.386 -> 1.338 ms per
-// 1080p frame, output unchanged.
-template <int NT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 4 ? 3 : 1, NT == 4 ? 3 : 8))) void kConvFwdChunk(
-    ConvArgs a) {
-  extern __shared__ __align__(16) bf16 lds[];
-  constexpr uint32_t tw = kChunkCols + 2, tpix = (kChunkRows + 2) * tw;
-  constexpr uint32_t Cout = 16 * NT, TG = chunkTaps<NT>();
-  bf16* tile = lds;                       // tpix x kChunkStride
-  bf16* wts = lds + tpix * kChunkStride;  // TG x Cout x kChunkStride
-  const uint32_t tilesX = (a.W + kChunkCols - 1) / kChunkCols, tilesY = (a.H + kChunkRows - 1) / kChunkRows;
-  const uint32_t tx0 = (blockIdx.x % tilesX) * kChunkCols, ty0 = ((blockIdx.x / tilesX) % tilesY) * kChunkRows;
-  const uint32_t n = blockIdx.x / (tilesX * tilesY);
-  const uint32_t lane = threadIdx.x & 63, q = lane >> 4, r16 = lane & 15, wv = threadIdx.x >> 6;
-  f32x4 acc[4][NT];
-#pragma unroll
-  for (int g = 0; g < 4; ++g)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) acc[g][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (uint32_t c0 = 0; c0 < a.Cin; c0 += 32) {
-    if (c0) __syncthreads();  // the previous chunk's fragments are consumed
-    for (uint32_t k = threadIdx.x; k < tpix * 4; k += 256) {
-      const uint32_t c8 = k & 3, pix = k >> 2;
-      const int yy = int(ty0) - 1 + int(pix / tw), xx = int(tx0) - 1 + int(pix % tw);
-      *reinterpret_cast<bf16x8*>(tile + pix * kChunkStride + 8 * c8) = loadIn(a, n, yy, xx, c0 + 8 * c8);
-    }
-    for (uint32_t t0 = 0; t0 < 9; t0 += TG) {
-      if (t0) __syncthreads();  // the previous tap group's fragments are consumed
-      for (uint32_t k = threadIdx.x; k < TG * Cout * 4; k += 256) {
-        const uint32_t c8 = k & 3, row = k >> 2;  // row = (tap - t0) * Cout + co
-        *reinterpret_cast<bf16x8*>(wts + row * kChunkStride + 8 * c8) =
-            *reinterpret_cast<const bf16x8*>(a.Wf + (size_t(t0) * Cout + row) * a.Cin + c0 + 8 * c8);
-      }
-      __syncthreads();
-#pragma unroll 3
-      for (uint32_t tl = 0; tl < TG; ++tl) {
-        const uint32_t tap = t0 + tl, dy = tap / 3, dx = tap % 3;  // tile coordinates are offset by the halo
-        bf16x8 B[NT];
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-          B[t] = *reinterpret_cast<const bf16x8*>(wts + (tl * Cout + 16 * t + r16) * kChunkStride + 8 * q);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const uint32_t row = 2 * wv + uint32_t(g) / 2, col = (uint32_t(g) % 2) * 16 + r16;
-          const bf16x8 A =
-              *reinterpret_cast<const bf16x8*>(tile + ((row + dy) * tw + col + dx) * kChunkStride + 8 * q);
-#pragma unroll
-          for (int t = 0; t < NT; ++t) acc[g][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B[t], acc[g][t], 0, 0, 0);
-        }
-      }
-    }
-  }
-  if (a.Y) {
-    // BF16 output through LDS: each lane holds 4 pixels of one channel per
-    // fragment; the block's 256 x Cout tile is written to LDS pixel-major and
-    // stored as 16-byte runs of 8 channels (whole tile rows are contiguous
-    // in NHWC memory)
-    constexpr uint32_t OS = Cout + 8;  // bf16 per pixel in LDS (the pad spreads banks)
-    bf16* ot = lds;
-    __syncthreads();  // every wave is done with the tile and the weights
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const uint32_t co = 16 * t + r16;
-        const float b = a.bias[co];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const uint32_t px = (2 * wv + uint32_t(g) / 2) * kChunkCols + (uint32_t(g) % 2) * 16 + 4 * q + r;
-          float v = acc[g][t][r] + b;
-          if (a.relu) v = fmaxf(v, 0.f);
-          ot[px * OS + co] = bf16(v);
-        }
-      }
-    __syncthreads();
-    constexpr uint32_t C8 = Cout / 8;
-    for (uint32_t k = threadIdx.x; k < kChunkRows * kChunkCols * C8; k += 256) {
-      const uint32_t px = k / C8, c8 = k % C8;
-      const uint32_t y = ty0 + px / kChunkCols, x = tx0 + px % kChunkCols;
-      if (y < a.H && x < a.W)
-        *reinterpret_cast<bf16x8*>(a.Y + ((size_t(n) * a.H + y) * a.W + x) * Cout + 8 * c8) =
-            *reinterpret_cast<const bf16x8*>(ot + px * OS + 8 * c8);
-    }
-  }
-  if (a.Yf) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const uint32_t y = ty0 + 2 * wv + uint32_t(g) / 2;
-      if (y >= a.H) continue;
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const uint32_t co = 16 * t + r16;
-        const float b = a.bias[co];
-        for (int r = 0; r < 4; ++r) {
-          const uint32_t x = tx0 + (uint32_t(g) % 2) * 16 + 4 * q + r;
-          if (x >= a.W) continue;
-          const size_t pp = (size_t(n) * a.H + y) * a.W + x;
-          float v = acc[g][t][r] + b;
-          if (a.relu) v = fmaxf(v, 0.f);
-          a.Yf[pp * Cout + co] = v;
-        }
-      }
-    }
-  }
-}
-template <int NT> constexpr size_t chunkLds() {
-  const size_t staged =
-      (size_t(kChunkRows + 2) * (kChunkCols + 2) + size_t(chunkTaps<NT>()) * 16 * NT) * kChunkStride * sizeof(bf16);
-  const size_t outTile = size_t(kChunkRows) * kChunkCols * (16 * NT + 8) * sizeof(bf16);
-  return staged > outTile ? staged : outTile;
-}
-static_assert(chunkLds<2>() <= 65536 && chunkLds<4>() <= 65536, "chunked convolution LDS above 64 KB");
-static_assert(chunkLds<2>() >= size_t(kChunkRows) * kChunkCols * (32 + 8) * sizeof(bf16) &&
-                  chunkLds<4>() >= size_t(kChunkRows) * kChunkCols * (64 + 8) * sizeof(bf16),
-              "chunked convolution LDS below its output tile");
-
-// Persistent forward convolution for 32 -> 32-channel layers on large
-// levels.  The weights of all 9 taps stay in LDS for the block's lifetime;
-// the block walks output tiles of 8 rows x 32 columns (tile = blockIdx.x +
-// k * gridDim.x), and while its waves run the MFMAs of one tile, each
-// thread's loads of the next tile's input (with the halo) are in flight into
-// registers, then written to the one LDS tile buffer once the current tile's
-// fragments and output are consumed.  Per output tile and fragment the taps
-// are accumulated in the order kConvFwdChunk uses, so the output is the
-// same bit for bit.
-constexpr uint32_t kP32Tile = (kChunkRows + 2) * (kChunkCols + 2);     // input pixels per tile
-constexpr uint32_t kP32Loads = (kP32Tile * 4 + 255) / 256;             // 16-byte loads per thread
-constexpr size_t kP32Lds = (size_t(9) * 32 + kP32Tile) * kChunkStride * sizeof(bf16);
-static_assert(kP32Lds <= 65536, "persistent convolution LDS above 64 KB");
-static_assert(size_t(kP32Tile) * kChunkStride >= size_t(kChunkRows) * kChunkCols * (32 + 8),
-              "persistent convolution tile buffer below its output tile");
-constexpr uint32_t kP32BlocksPerCU = 3;  // 50 KB of LDS each
-
-__global__ __launch_bounds__(256) void kConvFwd32(ConvArgs a, uint32_t tiles) {
-  extern __shared__ __align__(16) bf16 lds[];
-  constexpr uint32_t tw = kChunkCols + 2;
-  bf16* wts = lds;                             // 9 x 32 x kChunkStride: [tap][co][ci]
-  bf16* tile = lds + 9 * 32 * kChunkStride;    // kP32Tile x kChunkStride
-  const uint32_t tilesX = (a.W + kChunkCols - 1) / kChunkCols, tilesY = (a.H + kChunkRows - 1) / kChunkRows;
-  const uint32_t lane = threadIdx.x & 63, q = lane >> 4, r16 = lane & 15, wv = threadIdx.x >> 6;
-  for (uint32_t k = threadIdx.x; k < 9 * 32 * 4; k += 256) {
-    const uint32_t c8 = k & 3, row = k >> 2;  // row = tap * 32 + co
-    *reinterpret_cast<bf16x8*>(wts + row * kChunkStride + 8 * c8) =
-        *reinterpret_cast<const bf16x8*>(a.Wf + size_t(row) * 32 + 8 * c8);
-  }
-  bf16x8 pre[kP32Loads];
-  auto fetch = [&](uint32_t t) {
-    const uint32_t tx0 = (t % tilesX) * kChunkCols, ty0 = ((t / tilesX) % tilesY) * kChunkRows;
-    const uint32_t n = t / (tilesX * tilesY);
-#pragma unroll
-    for (uint32_t j = 0; j < kP32Loads; ++j) {
-      const uint32_t k = threadIdx.x + 256 * j;
-      if (k < kP32Tile * 4) {
-        const uint32_t c8 = k & 3, pix = k >> 2;
-        const int yy = int(ty0) - 1 + int(pix / tw), xx = int(tx0) - 1 + int(pix % tw);
-        pre[j] = loadIn(a, n, yy, xx, 8 * c8);
-      }
-    }
+    *reinterpret_cast<bf16x8*>(d.g + e) = o;
   };
-  auto put = [&]() {
+  if (d.kind == kGradUp) {
 #pragma unroll
-    for (uint32_t j = 0; j < kP32Loads; ++j) {
-      const uint32_t k = threadIdx.x + 256 * j;
-      if (k < kP32Tile * 4) *reinterpret_cast<bf16x8*>(tile + (k >> 2) * kChunkStride + 8 * (k & 3)) = pre[j];
+    for (int i = 0; i < ROWS; i += 2) {
+      float s[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s[j] = v[i][j] + pairLane(v[i][j]) + v[i + 1][j] + pairLane(v[i + 1][j]);
+      const int y = y0 + i;
+      if (!(x & 1) && y < H && x < W) put(((size_t(n) * (a.H / 2) + y / 2) * (a.W / 2) + x / 2) * d.C + c0, s);
     }
-  };
-  uint32_t t = blockIdx.x;
-  if (t < tiles) {
-    fetch(t);
-    put();
-  }
-  __syncthreads();  // the weights and the first tile are in LDS
-  for (; t < tiles; t += gridDim.x) {
-    const uint32_t next = t + gridDim.x;
-    if (next < tiles) fetch(next);  // in flight during this tile's MFMAs
-    const uint32_t tx0 = (t % tilesX) * kChunkCols, ty0 = ((t / tilesX) % tilesY) * kChunkRows;
-    const uint32_t n = t / (tilesX * tilesY);
-    f32x4 acc[4][2];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) acc[g][0] = acc[g][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 3
-    for (uint32_t tap = 0; tap < 9; ++tap) {
-      const uint32_t dy = tap / 3, dx = tap % 3;  // tile coordinates are offset by the halo
-      bf16x8 B[2];
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-        B[c] = *reinterpret_cast<const bf16x8*>(wts + (tap * 32 + 16 * c + r16) * kChunkStride + 8 * q);
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const uint32_t row = 2 * wv + uint32_t(g) / 2, col = (uint32_t(g) % 2) * 16 + r16;
-        const bf16x8 A = *reinterpret_cast<const bf16x8*>(tile + ((row + dy) * tw + col + dx) * kChunkStride + 8 * q);
-#pragma unroll
-        for (int c = 0; c < 2; ++c) acc[g][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B[c], acc[g][c], 0, 0, 0);
-      }
-    }
-    __syncthreads();  // every wave is done with the tile's fragments
-    if (a.Y) {
-      // BF16 output through the tile buffer, stored as 16-byte runs (as kConvFwdChunk)
-      constexpr uint32_t OS = 32 + 8;
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          const uint32_t co = 16 * c + r16;
-          const float b = a.bias[co];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const uint32_t px = (2 * wv + uint32_t(g) / 2) * kChunkCols + (uint32_t(g) % 2) * 16 + 4 * q + r;
-            float v = acc[g][c][r] + b;
-            if (a.relu) v = fmaxf(v, 0.f);
-            tile[px * OS + co] = bf16(v);
-          }
-        }
-      __syncthreads();
-      for (uint32_t k = threadIdx.x; k < kChunkRows * kChunkCols * 4; k += 256) {
-        const uint32_t px = k >> 2, c8 = k & 3;
-        const uint32_t y = ty0 + px / kChunkCols, x = tx0 + px % kChunkCols;
-        if (y < a.H && x < a.W)
-          *reinterpret_cast<bf16x8*>(a.Y + ((size_t(n) * a.H + y) * a.W + x) * 32 + 8 * c8) =
-              *reinterpret_cast<const bf16x8*>(tile + px * OS + 8 * c8);
-      }
-      __syncthreads();  // the output tile is read out
-    }
-    if (a.Yf) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const uint32_t y = ty0 + 2 * wv + uint32_t(g) / 2;
-        if (y >= a.H) continue;
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          const uint32_t co = 16 * c + r16;
-          const float b = a.bias[co];
-          for (int r = 0; r < 4; ++r) {
-            const uint32_t x = tx0 + (uint32_t(g) % 2) * 16 + 4 * q + r;
-            if (x >= a.W) continue;
-            const size_t pp = (size_t(n) * a.H + y) * a.W + x;
-            float v = acc[g][c][r] + b;
-            if (a.relu) v = fmaxf(v, 0.f);
-            a.Yf[pp * 32 + co] = v;
-          }
-        }
-      }
-    }
-    if (next < tiles) put();
-    __syncthreads();  // the next tile is in LDS
-  }
-}
-
-template <int NT>
-static void convFwdFor(const ConvArgs& a, size_t P, hipStream_t s) {
-  if (P >= (size_t(1) << 16) && NT == 2 && a.Cin == 32) {
-    // large levels, 32 -> 32 channels: the persistent kernel with all taps' weights in LDS
-    const uint32_t tiles = a.N * ((a.H + kChunkRows - 1) / kChunkRows) * ((a.W + kChunkCols - 1) / kChunkCols);
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        cus <= 0)
-      cus = 256;
-    const uint32_t grid = std::min<uint32_t>(tiles, kP32BlocksPerCU * uint32_t(cus));
-    kConvFwd32<<<grid, 256, kP32Lds, s>>>(a, tiles);
     return;
   }
-  if (P >= (size_t(1) << 16) && NT <= 4) {
-    // large levels: the K-chunked LDS kernel (input tile and weights of each 32-channel chunk in LDS)
-    const uint32_t tiles = a.N * ((a.H + kChunkRows - 1) / kChunkRows) * ((a.W + kChunkCols - 1) / kChunkCols);
-    kConvFwdChunk<NT><<<tiles, 256, chunkLds<NT>(), s>>>(a);
-    return;
-  }
-  if (P >= (size_t(1) << 18) && a.Cin <= 128) {
-    // large levels with wide outputs: the LDS-tiled kernel (32-column tiles up to 64 input channels, else 16)
-    const bool wide = a.Cin <= 64;
-    const uint32_t TC = wide ? 32 : 16;
-    const uint32_t tiles = a.N * ((a.H + kTileRows - 1) / kTileRows) * ((a.W + TC - 1) / TC);
-    const size_t lds = size_t(kTileRows + 2) * (TC + 2) * (a.Cin + 8) * sizeof(bf16);
-    if (wide) kConvFwdTile<NT, 32><<<tiles, 256, lds, s>>>(a);
-    else kConvFwdTile<NT, 16><<<tiles, 256, lds, s>>>(a);
-    return;
-  }
-  // more pixel groups per wave on larger levels (and narrower layers); small
-  // levels keep one so that the grid still fills the chip
-  if (P >= (size_t(1) << 20) && NT <= 2) kConvFwd<NT, 4><<<uint32_t((P + 255) / 256), 256, 0, s>>>(a);
-  else if (P >= (size_t(1) << 16)) kConvFwd<NT, 2><<<uint32_t((P + 127) / 128), 256, 0, s>>>(a);
-  else kConvFwd<NT, 1><<<uint32_t((P + 63) / 64), 256, 0, s>>>(a);
-}
-static bool launchConvFwd(const ConvArgs& a, size_t P, hipStream_t s) {
-  switch (a.Cout) {
-    case 32: convFwdFor<2>(a, P, s); return true;
-    case 64: convFwdFor<4>(a, P, s); return true;
-    case 96: convFwdFor<6>(a, P, s); return true;
-    case 128: convFwdFor<8>(a, P, s); return true;
-    default: return false;
-  }
-}
-
-// ---------------------------------------------------------- backward-x
-// Same tiling with the roles of cin and cout exchanged; gradients are
-// added (+=) into s0.g (or upTmp when s0 is upsampled) and s1.g.
-__global__ __launch_bounds__(256) void kConvBwdX(ConvArgs a) {
-  const uint32_t P = a.N * a.H * a.W;
-  const uint32_t lane = threadIdx.x & 63, q = lane >> 4, r16 = lane & 15;
-  const uint32_t p0 = blockIdx.x * 64 + (threadIdx.x >> 6) * 16;
-  const uint32_t p = p0 + r16;
-  const bool pin = p < P;
-  uint32_t n = 0;
-  int y = 0, x = 0;
-  if (pin) pixelOf(p, a.H, a.W, n, y, x);
-  const uint32_t nt = a.Cin / 16;
-  f32x4 acc[kMaxTiles];
-  for (int t = 0; t < kMaxTiles; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int tap = 0; tap < 9; ++tap) {
-    const int yy = y - (tap / 3 - 1), xx = x - (tap % 3 - 1);
-    const bool in = pin && yy >= 0 && yy < int(a.H) && xx >= 0 && xx < int(a.W);
-    const size_t src = in ? ((size_t(n) * a.H + uint32_t(yy)) * a.W + uint32_t(xx)) * a.Cout : 0;
-    const bf16* wt = a.Wb + size_t(tap) * a.Cin * a.Cout;
-    for (uint32_t c0 = 0; c0 < a.Cout; c0 += 32) {
-      bf16x8 A;
-      if (in) {
-        const float4* g = reinterpret_cast<const float4*>(a.dY + src + c0 + 8 * q);
-        float4 g0 = g[0], g1 = g[1];
-        A[0] = bf16(g0.x), A[1] = bf16(g0.y), A[2] = bf16(g0.z), A[3] = bf16(g0.w);
-        A[4] = bf16(g1.x), A[5] = bf16(g1.y), A[6] = bf16(g1.z), A[7] = bf16(g1.w);
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    const int y = y0 + i;
+    if (y >= H || x >= W) continue;
+    if (d.kind == kGradPool) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const size_t e = ((size_t(n) * (2 * a.H) + 2 * y + k / 2) * (2 * a.W) + 2 * x + k % 2) * d.C + c0;
+        float s[8];
+        *reinterpret_cast<float4*>(s) = *reinterpret_cast<const float4*>(d.skip + e);
+        *reinterpret_cast<float4*>(s + 4) = *reinterpret_cast<const float4*>(d.skip + e + 4);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s[j] += 0.25f * v[i][j];
+        put(e, s);
+      }
+    } else {
+      const size_t e = ((size_t(n) * a.H + y) * a.W + x) * d.C + c0;
+      if (d.kind == kGradFinal) {
+        put(e, v[i]);
       } else {
-        for (int i = 0; i < 8; ++i) A[i] = bf16(0.0f);
-      }
-      const bf16* wr = wt + c0 + 8 * q;
-#pragma unroll
-      for (int t = 0; t < kMaxTiles; ++t) {
-        if (uint32_t(t) < nt) {
-          bf16x8 B = *reinterpret_cast<const bf16x8*>(wr + size_t(16 * t + r16) * a.Cout);
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, acc[t], 0, 0, 0);
-        }
+        *reinterpret_cast<float4*>(d.skip + e) = make_float4(v[i][0], v[i][1], v[i][2], v[i][3]);
+        *reinterpret_cast<float4*>(d.skip + e + 4) = make_float4(v[i][4], v[i][5], v[i][6], v[i][7]);
       }
     }
   }
+}
+
+// Sums the lanes' bias-gradient parts over the wave's 16 pixel columns (a
+// fixed tree) into row[8q + j].
+__device__ __forceinline__ void waveBias(float (&bs)[8], uint32_t q, uint32_t r16, float* row) {
 #pragma unroll
-  for (int t = 0; t < kMaxTiles; ++t) {
-    if (uint32_t(t) >= nt) continue;
-    const uint32_t ci = 16 * t + r16;
-    for (int r = 0; r < 4; ++r) {
-      const uint32_t pp = p0 + 4 * q + r;
-      if (pp >= P) continue;
-      float* dst;
-      if (ci < a.s0.C) dst = (a.s0.up ? a.upTmp : a.s0.g) + size_t(pp) * a.s0.C + ci;
-      else dst = a.s1.g + size_t(pp) * a.s1.C + (ci - a.s0.C);
-      *dst += acc[t][r];
+  for (int j = 0; j < 8; ++j) {
+    float s = bs[j];
+    s += __shfl_xor(s, 1);
+    s += __shfl_xor(s, 2);
+    s += __shfl_xor(s, 4);
+    s += __shfl_xor(s, 8);
+    if (r16 == 0) row[8 * q + j] = s;
+  }
+}
+// Writes a 32-channel group's bias-gradient sums of one pixel tile (thread c
+// of 32; rows: the waves' sums, added in wave order).
+__device__ __forceinline__ void tileBias(const ConvArgs& a, uint32_t cg, uint32_t tile, uint32_t c, const float* rows,
+                                         uint32_t nRows) {
+  const GradDst& d = cg < a.cg0 ? a.d0 : a.d1;
+  if (d.kind == kGradSkip) return;
+  float s = 0.f;
+  for (uint32_t w = 0; w < nRows; ++w) s += rows[32 * w + c];
+  d.bPart[size_t(tile) * d.C + 32 * (cg < a.cg0 ? cg : cg - a.cg0) + c] = s;
+}
+
+// Convolution from LDS, for levels with work for the whole chip: a block of
+// 4 waves owns a tile of 2R rows x 32 columns (CW = 1: four pixel waves) or
+// 2R x 16 columns (CW = 2: two pixel waves for each of two output groups)
+// and walks the input in chunks of 32 channels.  Per chunk it holds in LDS
+// the input tile with its halo (64 bytes per pixel) and the chunk's weights
+// of its output groups, in fragment order (a fragment is 1 KB in lane order).
+// Each wave computes R rows x 16 columns x 32 channels: an input fragment
+// (one row, one column shift) is read once and feeds the three taps of its
+// column shift, i.e. up to 6 MFMAs, so that per chunk a wave reads 3 (R + 2)
+// input and 18 weight fragments for 18 R MFMAs and the matrix cores, not
+// the LDS, are the limit (R = 8: 48 KB of LDS reads, 384 cycles of the CU's
+// 128 bytes per cycle, against 576 matrix cycles per SIMD).  The loads of the
+// next chunk (or the next tile's first) are in flight in registers during
+// the MFMAs.  Blocks are persistent; with one chunk the weights stay in LDS.
+//
+// A pixel's four 16-byte slots are swizzled by its column (slot ^ column / 4),
+// which spreads a fragment's 16 pixels over all banks and leaves the
+// row's offset an immediate.
+template <int R, int CW> struct ConvTile {
+  static constexpr uint32_t PW = 4 / CW;              // pixel waves
+  static constexpr uint32_t TR = 2 * R, TC = CW == 1 ? 32 : 16;
+  static constexpr uint32_t P = (TR + 2) * (TC + 2);  // staged pixels
+  static constexpr uint32_t LX = (P * 4 + 255) / 256;           // 16-byte input loads per thread
+  static constexpr uint32_t LW = (CW * 18 * 64 + 255) / 256;    // weight loads per thread
+  static constexpr size_t lds = size_t(P) * 64 + size_t(CW) * 18 * 1024;
+};
+template <int R, int CW, int NT, ConvMode MODE>
+__global__ __launch_bounds__(256, R == 8 ? 2 : 3) void kConvLds(ConvArgs a, uint32_t tilesX, uint32_t tilesY, uint32_t items) {
+  using T = ConvTile<R, CW>;
+  extern __shared__ __align__(16) bf16 lds[];
+  __shared__ float sB[4 * 32];
+  bf16* tile = lds;               // [T::P][4 slots][8]
+  bf16* wts = lds + T::P * 32;    // [CW][9 taps][2][64][8]
+  const uint32_t tid = threadIdx.x, lane = tid & 63, q = lane >> 4, r16 = lane & 15, wv = tid >> 6;
+  const uint32_t cw = wv / T::PW, pw = wv % T::PW;
+  const uint32_t row0 = CW == 1 ? (pw >> 1) * R : pw * R, col0 = CW == 1 ? (pw & 1) * 16 : 0;
+  const uint32_t cgb = a.nCg / CW;  // gridDim.x is a multiple: a block keeps its output groups
+  uint32_t item = blockIdx.x;
+  const uint32_t cgBase = (item % cgb) * CW;
+  u32x4 px[T::LX], pwt[T::LW];
+  auto origin = [&](uint32_t it, uint32_t& n, int& ty, int& tx) {
+    const uint32_t t = it / cgb;
+    tx = int((t % tilesX) * T::TC);
+    ty = int(((t / tilesX) % tilesY) * T::TR);
+    n = t / (tilesX * tilesY);
+  };
+  // the thread index through an opaque copy: the staging coordinates are recomputed where they are used instead of
+  // being held in registers through the loops (10 loads of 2 coordinates spilled 100 registers)
+  auto fresh = [&]() {
+    uint32_t t = tid;
+    asm volatile("" : "+v"(t));
+    return t;
+  };
+  auto fetch = [&](uint32_t it, uint32_t ch, bool weights) {
+    const uint32_t tid = fresh();
+    uint32_t n;
+    int ty, tx;
+    origin(it, n, ty, tx);
+    const ChunkSrc src = chunkSrc(a.s0, a.s1, a.H, a.W, n, ch);
+#pragma unroll
+    for (uint32_t j = 0; j < T::LX; ++j) {
+      const uint32_t k = tid + 256 * j, pix = k >> 2;
+      if (k < T::P * 4) {
+        const int y = ty - 1 + int(pix / (T::TC + 2)), x = tx - 1 + int(pix % (T::TC + 2));
+        px[j] = loadIn(src, a.H, a.W, y, x, 8 * (k & 3));
+      }
     }
+    if (weights) {
+#pragma unroll
+      for (uint32_t j = 0; j < T::LW; ++j) {
+        const uint32_t k = tid + 256 * j, g = k / (18 * 64), f = k % (18 * 64);
+        if (k < CW * 18 * 64)
+          pwt[j] = *reinterpret_cast<const u32x4*>(a.Wp + ((size_t(cgBase + g) * a.nCh + ch) * (18 * 64) + f) * 8);
+      }
+    }
+  };
+  auto put = [&](bool weights) {
+    const uint32_t tid = fresh();
+#pragma unroll
+    for (uint32_t j = 0; j < T::LX; ++j) {
+      const uint32_t k = tid + 256 * j, pix = k >> 2, col = pix % (T::TC + 2);
+      if (k < T::P * 4) *reinterpret_cast<u32x4*>(tile + (pix * 4 + ((k & 3) ^ ((col >> 2) & 3))) * 8) = px[j];
+    }
+    if (weights) {
+#pragma unroll
+      for (uint32_t j = 0; j < T::LW; ++j) {
+        const uint32_t k = tid + 256 * j;
+        if (k < CW * 18 * 64) *reinterpret_cast<u32x4*>(wts + k * 8) = pwt[j];
+      }
+    }
+  };
+  const bf16* wAt = wts + (cw * 18 * 64 + lane) * 8;
+  bool w = true;
+  fetch(item, 0, true);
+  for (;;) {
+    f32x4 acc[R][NT];
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (uint32_t ch = 0; ch < a.nCh; ++ch) {
+      __syncthreads();  // the previous chunk's fragments are consumed
+      put(w);
+      __syncthreads();
+      w = a.nCh > 1;
+      if (ch + 1 < a.nCh) fetch(item, ch + 1, w);
+      else if (item + gridDim.x < items) fetch(item + gridDim.x, 0, w);
+      __builtin_amdgcn_sched_barrier(0);  // the loads are issued before the MFMAs
+#pragma unroll 1  // unrolled, the reads of all three shifts are hoisted together and spill
+      for (int dx = 0; dx < 3; ++dx) {
+        const uint32_t col = col0 + r16 + dx;  // rows are immediate offsets from here
+        const bf16* xAt = tile + ((row0 * (T::TC + 2) + col) * 4 + (q ^ ((col >> 2) & 3))) * 8;
+        bf16x8 wf[3][NT];
+#pragma unroll
+        for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+          for (int t = 0; t < NT; ++t) wf[dy][t] = *reinterpret_cast<const bf16x8*>(wAt + ((dy * 3 + dx) * 2 + t) * 512);
+#pragma unroll
+        for (int r = 0; r < R + 2; ++r) {
+          const bf16x8 xf = *reinterpret_cast<const bf16x8*>(xAt + r * (T::TC + 2) * 32);
+#pragma unroll
+          for (int dy = 0; dy < 3; ++dy) {
+            const int o = r - dy;
+            if (o < 0 || o >= R) continue;
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+              acc[o][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[dy][t], xf, acc[o][t], 0, 0, 0);
+          }
+        }
+      }
+    }
+    uint32_t n;
+    int ty, tx;
+    origin(item, n, ty, tx);
+    float bs[8] = {};
+#pragma unroll
+    for (int i = 0; i < R; i += 2) {
+      __builtin_amdgcn_sched_barrier(0);
+      float v[2][8];
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[k][j] = j / 4 < NT ? acc[i + k][j / 4 < NT ? j / 4 : 0][j % 4] : 0.f;
+      emit<2, MODE>(a, cgBase + cw, n, ty + int(row0) + i, tx + int(col0 + r16), q, v, bs);
+    }
+    if (MODE == kModeGrad) {
+      waveBias(bs, q, r16, sB + 32 * wv);
+      __syncthreads();
+      if (tid < 32 * CW) tileBias(a, cgBase + tid / 32, item / cgb, tid & 31, sB + 32 * T::PW * (tid / 32), T::PW);
+    }
+    item += gridDim.x;
+    if (item >= items) break;
+  }
+}
+
+// Convolution of small levels, whose pixels do not fill the chip: a block
+// owns 4 rows x 16 columns x 32 output channels and has one wave per
+// 32-channel input chunk (K split over the waves), so a layer lasts about one
+// round trip to L2 instead of a serial walk over its chunks: a wave loads its
+// chunk's 18 weight and 18 input fragments straight from memory, all in
+// flight together, and the partial sums are added in chunk order in LDS.
+constexpr int kSplitRows = 4;
+template <ConvMode MODE>
+__global__ __launch_bounds__(64 * kMaxChunks) void kConvSplit(ConvArgs a, uint32_t tilesX, uint32_t tilesY) {
+  extern __shared__ __align__(16) float red[];  // [chunk][row][lane][8]
+  __shared__ float sB[2 * 32];
+  constexpr int R = kSplitRows;
+  const uint32_t tid = threadIdx.x, lane = tid & 63, q = lane >> 4, r16 = lane & 15, wv = tid >> 6;
+  const uint32_t cg = blockIdx.x % a.nCg, t0 = blockIdx.x / a.nCg;
+  const int tx = int((t0 % tilesX) * 16), ty = int(((t0 / tilesX) % tilesY) * R);
+  const uint32_t n = t0 / (tilesX * tilesY);
+  const int x = tx + int(r16);
+  bf16x8 xf[R + 2][3], wf[9][2];
+  const ChunkSrc src = chunkSrc(a.s0, a.s1, a.H, a.W, n, __builtin_amdgcn_readfirstlane(wv));
+#pragma unroll
+  for (int r = 0; r < R + 2; ++r)
+#pragma unroll
+    for (int dx = 0; dx < 3; ++dx) xf[r][dx] = __builtin_bit_cast(bf16x8, loadIn(src, a.H, a.W, ty + r - 1, x + dx - 1, 8 * q));
+  const bf16* wp = a.Wp + ((size_t(cg) * a.nCh + wv) * (18 * 64) + lane) * 8;
+#pragma unroll
+  for (int k = 0; k < 18; ++k) wf[k / 2][k % 2] = *reinterpret_cast<const bf16x8*>(wp + k * 512);
+  f32x4 acc[R][2];
+#pragma unroll
+  for (int i = 0; i < R; ++i) acc[i][0] = acc[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int tap = 0; tap < 9; ++tap)
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[tap][t], xf[i + tap / 3][tap % 3], acc[i][t], 0, 0, 0);
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) *reinterpret_cast<f32x4*>(red + ((wv * R + i) * 64 + lane) * 8 + 4 * t) = acc[i][t];
+  __syncthreads();
+  for (uint32_t pair = wv; pair < R / 2; pair += a.nCh) {
+    float v[2][8] = {};
+    for (uint32_t w = 0; w < a.nCh; ++w)
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const f32x4 p = *reinterpret_cast<const f32x4*>(red + ((w * R + 2 * pair + k) * 64 + lane) * 8 + 4 * t);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[k][4 * t + j] += p[j];
+        }
+    float bs[8] = {};
+    emit<2, MODE>(a, cg, n, ty + 2 * int(pair), x, q, v, bs);
+    if (MODE == kModeGrad) waveBias(bs, q, r16, sB + 32 * pair);
+  }
+  if (MODE == kModeGrad) {
+    __syncthreads();
+    if (tid < 32) tileBias(a, cg, t0, tid, sB, R / 2);
   }
 }
 
 // ---------------------------------------------------------- backward-w
-// One wave = one tap x (32 cout) x (32 cin) block over one pixel split;
-// 2 x 2 MFMA tiles per K step of 32 pixels.
-__global__ __launch_bounds__(256) void kConvBwdW(ConvArgs a) {
-  const uint32_t P = a.N * a.H * a.W;
-  const uint32_t lane = threadIdx.x & 63, q = lane >> 4, r16 = lane & 15;
-  const uint32_t task = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const uint32_t nco = a.Cout / 32, nci = a.Cin / 32;
-  const uint32_t nTasks = 9 * nco * nci * a.splits;
-  if (task >= nTasks) return;
-  uint32_t t = task;
-  const uint32_t split = t % a.splits;
-  t /= a.splits;
-  const uint32_t cib = t % nci;
-  t /= nci;
-  const uint32_t cob = t % nco;
-  const int tap = int(t / nco);
-  const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-  const uint32_t pBeg = uint32_t(uint64_t(P) * split / a.splits), pEnd = uint32_t(uint64_t(P) * (split + 1) / a.splits);
-  f32x4 acc[2][2];
-  for (int i = 0; i < 2; ++i)
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const uint32_t co0 = cob * 32 + r16, ci0 = cib * 32 + r16;
-  for (uint32_t pp = pBeg; pp < pEnd; pp += 32) {
-    bf16x8 A[2], B[2];
-    uint32_t p = pp + 8 * q;
-    uint32_t n = 0;
-    int y = 0, x = 0;
-    if (p < pEnd) pixelOf(p, a.H, a.W, n, y, x);
-    for (int k = 0; k < 8; ++k, ++p) {
-      float g0 = 0.f, g1 = 0.f, x0 = 0.f, x1 = 0.f;
-      if (p < pEnd) {
-        const float* gr = a.dY + size_t(p) * a.Cout;
-        g0 = gr[co0];
-        g1 = gr[co0 + 16];
-        x0 = loadIn1(a, n, y + dy, x + dx, ci0);
-        x1 = loadIn1(a, n, y + dy, x + dx, ci0 + 16);
-      }
-      A[0][k] = bf16(g0);
-      A[1][k] = bf16(g1);
-      B[0][k] = bf16(x0);
-      B[1][k] = bf16(x1);
-      if (++x == int(a.W)) {
-        x = 0;
-        if (++y == int(a.H)) y = 0, ++n;
+// A block (4 waves) owns the 9 taps of a 32 cout x 32 cin block of one
+// layer's weights and walks every splits-th pixel tile (TC columns, 256 / TC
+// rows).  A tile's output gradient and its input with the halo are staged in
+// LDS as they are in memory (64 bytes per pixel, loads of the next tile in
+// flight in registers); both operands need 8 consecutive pixels of one channel
+// per lane, which ds_read_b64_tr_b16 reads transposed (16 lanes read 4 pixels
+// x 16 channels), at any pixel offset, so the nine taps read the one staged
+// tile.  Each wave takes 2 of the tile's 8 steps of 32 pixels and keeps all 36
+// output tiles in registers: 20 fragments read for 36 MFMAs.  The waves' sums
+// are added in wave order through LDS.  (One wave per tap, 32 x 32 block and
+// split, gathering 2-byte values from memory, took 319 us per layer of a
+// batch of 8 x 128 x 128 on average; this takes 12.)
+struct BwdWArgs {
+  Src s0, s1;
+  const bf16* dY;  // [N][H][W][32 nCo], masked
+  uint32_t N, H, W, nCo, nCi, splits;
+  uint32_t tilesX, tilesY, tiles;
+  float* part;     // [splits][9][32 nCo][32 nCi]
+};
+template <int TC> struct BwdWTile {
+  static constexpr uint32_t TR = 256 / TC, P = (TR + 2) * (TC + 2);
+  static constexpr uint32_t LX = (P * 4 + 255) / 256;
+  static constexpr size_t lds = (size_t(P) + 256) * 64;
+};
+typedef __attribute__((address_space(3))) bf16x4* LdsTr;
+// 8 pixels (two groups of 4) x 16 channels, transposed: lane l holds channel l % 16.
+__device__ __forceinline__ bf16x8 readTr(const bf16* p0, const bf16* p1) {
+  const bf16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((LdsTr)(p0));
+  const bf16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((LdsTr)(p1));
+  return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+template <int TC>
+__global__ __launch_bounds__(256, 2) void kConvBwdW(BwdWArgs a) {
+  using T = BwdWTile<TC>;
+  static_assert(T::lds >= 4 * 9 * 1024, "the reduction reuses the staging space");
+  __shared__ __align__(16) bf16 lds[T::lds / 2];
+  bf16* xs = lds;              // [T::P][4 slots][8]
+  bf16* ys = lds + T::P * 32;  // [256][4 slots][8]
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const uint32_t pairs = a.nCo * a.nCi, split = blockIdx.x / pairs;
+  const uint32_t cob = (blockIdx.x % pairs) / a.nCi, cib = (blockIdx.x % pairs) % a.nCi;
+  u32x4 px[T::LX], py[4];
+  auto fresh = [&]() {  // as in kConvLds
+    uint32_t i = tid;
+    asm volatile("" : "+v"(i));
+    return i;
+  };
+  auto fetch = [&](uint32_t t) {
+    const uint32_t tid = fresh();
+    const int tx = int((t % a.tilesX) * TC), ty = int(((t / a.tilesX) % a.tilesY) * T::TR);
+    const uint32_t n = t / (a.tilesX * a.tilesY);
+    const ChunkSrc src = chunkSrc(a.s0, a.s1, a.H, a.W, n, cib);
+#pragma unroll
+    for (uint32_t j = 0; j < T::LX; ++j) {
+      const uint32_t k = tid + 256 * j, pix = k >> 2;
+      if (k < T::P * 4)
+        px[j] = loadIn(src, a.H, a.W, ty - 1 + int(pix / (TC + 2)), tx - 1 + int(pix % (TC + 2)), 8 * (k & 3));
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+      const uint32_t k = tid + 256 * j, pix = k >> 2;
+      const uint32_t y = uint32_t(ty) + pix / TC, x = uint32_t(tx) + pix % TC;
+      py[j] = u32x4{0, 0, 0, 0};
+      if (y < a.H && x < a.W)
+        py[j] = *reinterpret_cast<const u32x4*>(a.dY + ((size_t(n) * a.H + y) * a.W + x) * (32 * a.nCo) + 32 * cob + 8 * (k & 3));
+    }
+  };
+  // 16-byte slots swapped in halves by bit 3 of the column: the lane groups of one read use different banks
+  auto slot = [](uint32_t col, uint32_t s) { return s ^ (((col >> 3) & 1) << 1); };
+  auto put = [&]() {
+    const uint32_t tid = fresh();
+#pragma unroll
+    for (uint32_t j = 0; j < T::LX; ++j) {
+      const uint32_t k = tid + 256 * j, pix = k >> 2;
+      if (k < T::P * 4) *reinterpret_cast<u32x4*>(xs + (pix * 4 + slot(pix % (TC + 2), k & 3)) * 8) = px[j];
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+      const uint32_t k = tid + 256 * j, pix = k >> 2;
+      *reinterpret_cast<u32x4*>(ys + (pix * 4 + slot(pix, k & 3)) * 8) = py[j];
+    }
+  };
+  // The lane's addresses in the wave's first step of 32 pixels: pixel group h (of 4 pixels), channel tile c.  The second
+  // step and the taps' rows are immediate offsets.
+  const uint32_t kp = 8 * (lane >> 4) + ((lane & 15) >> 2), sub = lane & 3;
+  constexpr uint32_t stepRows = TC >= 32 ? 1 : 32 / TC;
+  uint32_t yAt[2][2], xAt[3][2][2];
+#pragma unroll
+  for (uint32_t h = 0; h < 2; ++h)
+#pragma unroll
+    for (uint32_t c = 0; c < 2; ++c) {
+      const uint32_t p = 64 * wv + kp + 4 * h, row = 2 * wv * stepRows + (kp + 4 * h) / TC;
+      yAt[h][c] = T::P * 32 + p * 32 + slot(p, 2 * c + (sub >> 1)) * 8 + (sub & 1) * 4;
+#pragma unroll
+      for (uint32_t dx = 0; dx < 3; ++dx) {
+        const uint32_t col = (kp + 4 * h) % TC + dx;
+        xAt[dx][h][c] = (row * (TC + 2) + col) * 32 + slot(col, 2 * c + (sub >> 1)) * 8 + (sub & 1) * 4;
       }
     }
-    for (int i = 0; i < 2; ++i)
-      for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[i], B[j], acc[i][j], 0, 0, 0);
-  }
-  // D: col = cin (l % 16), rows = cout 4q .. 4q+3; one slot per (split, weight)
-  float* dw = a.wPart + (size_t(split) * 9 + size_t(tap)) * a.Cout * a.Cin;
-  for (int i = 0; i < 2; ++i)
-    for (int j = 0; j < 2; ++j)
-      for (int r = 0; r < 4; ++r) {
-        const uint32_t co = cob * 32 + 16 * i + 4 * q + r, ci = cib * 32 + 16 * j + r16;
-        dw[size_t(co) * a.Cin + ci] = acc[i][j][r];
+  f32x4 acc[9][2][2];
+#pragma unroll
+  for (int k = 0; k < 9; ++k)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) acc[k][i][0] = acc[k][i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  uint32_t t = split;
+  if (t < a.tiles) fetch(t);
+  while (t < a.tiles) {
+    __syncthreads();
+    put();
+    __syncthreads();
+    t += a.splits;
+    if (t < a.tiles) fetch(t);
+#pragma unroll
+    for (uint32_t s = 0; s < 2; ++s) {
+      bf16x8 A[2];
+#pragma unroll
+      for (uint32_t c = 0; c < 2; ++c) A[c] = readTr(lds + yAt[0][c] + s * 1024, lds + yAt[1][c] + s * 1024);
+#pragma unroll
+      for (uint32_t tap = 0; tap < 9; ++tap) {
+        const uint32_t off = (s * stepRows + tap / 3) * (TC + 2) * 32;
+        if (tap % 3 == 0) __builtin_amdgcn_sched_barrier(0);  // later rows' reads would spill
+        bf16x8 B[2];
+#pragma unroll
+        for (uint32_t c = 0; c < 2; ++c) B[c] = readTr(lds + xAt[tap % 3][0][c] + off, lds + xAt[tap % 3][1][c] + off);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[tap][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[i], B[j], acc[tap][i][j], 0, 0, 0);
       }
+    }
+  }
+  // waves' sums in wave order, one (cout tile, cin tile) of the nine taps at a time
+  float* red = reinterpret_cast<float*>(lds);  // [4 waves][9 taps][64 lanes][4]
+  const uint32_t Co = 32 * a.nCo, Ci = 32 * a.nCi;
+  float* out = a.part + size_t(split) * 9 * Co * Ci;
+#pragma unroll
+  for (uint32_t ij = 0; ij < 4; ++ij) {
+    __syncthreads();
+#pragma unroll
+    for (uint32_t tap = 0; tap < 9; ++tap)
+      *reinterpret_cast<f32x4*>(red + ((wv * 9 + tap) * 64 + lane) * 4) = acc[tap][ij / 2][ij % 2];
+    __syncthreads();
+    for (uint32_t e = tid; e < 9 * 64; e += 256) {
+      f32x4 s = *reinterpret_cast<const f32x4*>(red + e * 4);
+      for (uint32_t w = 1; w < 4; ++w) s += *reinterpret_cast<const f32x4*>(red + (w * 9 * 64 + e) * 4);
+      const uint32_t tap = e / 64, l = e % 64;
+      const uint32_t co = 32 * cob + 16 * (ij / 2) + 4 * (l >> 4), ci = 32 * cib + 16 * (ij % 2) + (l & 15);
+#pragma unroll
+      for (uint32_t r = 0; r < 4; ++r) out[(size_t(tap) * Co + co + r) * Ci + ci] = s[r];
+    }
+  }
 }
 
-// dW[i] += the splits' partial sums, added in split order.
-__global__ void kReduceSplits(const float* part, uint32_t splits, size_t n, float* dW) {
-  const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+// ------------------------------------------------- parameters (all layers)
+// One layer's place in the parameter vector, the packed weights and the
+// gradient partial sums.
+struct LayerTab {
+  struct Row {
+    uint32_t CoS, CinS;             // stored channels
+    uint32_t co, ca, CaS, cin;      // real output, source-0 and input channels, stored source-0 channels
+    uint32_t wOff, bOff;            // FP32 parameters: W[9][CoS][CinS], bias[CoS]
+    uint32_t fOff;                  // packed BF16 weights (both layouts)
+    uint32_t rOff;                  // real-channel flat order
+    uint32_t splits, nbk;           // weight and bias partial sums per element
+    size_t wPart, bPart;            // their offsets in the partial-sum buffer
+  } r[kNumLayers];
+};
+// The layer that holds parameter i of the padded vector.
+__device__ __forceinline__ const LayerTab::Row& layerOf(const LayerTab& T, uint32_t i) {
+  int k = 0;
+  while (k + 1 < kNumLayers && i >= T.r[k + 1].wOff) ++k;
+  return T.r[k];
+}
+// Stores weight e of a layer in both fragment orders.  A fragment holds,
+// per lane, 8 input channels of one output row; row m of tile t of a
+// 32-channel output group is channel 8 (m / 4) + 4 t + m % 4.
+__device__ __forceinline__ uint32_t fragIndex(uint32_t out, uint32_t in, uint32_t nIn, uint32_t tap) {
+  const uint32_t g = out / 32, c = out % 32, t = (c / 4) & 1, m = 4 * (c / 8) + c % 4;
+  return ((((g * (nIn / 32) + in / 32) * 9 + tap) * 2 + t) * 64 + ((in % 32) / 8) * 16 + m) * 8 + in % 8;
+}
+__device__ __forceinline__ void packWeight(const LayerTab::Row& l, uint32_t e, float w, bf16* wf, bf16* wb) {
+  const uint32_t ci = e % l.CinS, co = (e / l.CinS) % l.CoS, tap = e / (l.CinS * l.CoS);
+  wf[l.fOff + fragIndex(co, ci, l.CinS, tap)] = bf16(w);
+  wb[l.fOff + fragIndex(ci, co, l.CoS, 8 - tap)] = bf16(w);  // backward-x: taps reversed, roles exchanged
+}
+__global__ __launch_bounds__(256) void kPackW(LayerTab T, const float* theta, uint32_t n, bf16* wf, bf16* wb) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
-  float s = 0.f;
-  for (uint32_t k = 0; k < splits; ++k) s += part[size_t(k) * n + i];
-  dW[i] += s;
+  const LayerTab::Row& l = layerOf(T, i);
+  if (i < l.bOff) packWeight(l, i - l.wOff, theta[i], wf, wb);
 }
 
-// Bias gradient in two fixed-order passes: block b sums dY over its 256
-// pixels for every channel (thread c, pixels in order), then one thread per
-// channel adds the block sums in block order.
-constexpr uint32_t kBiasChunk = 256;
-__global__ void kBiasPart(const float* dY, uint32_t P, uint32_t C, float* part) {
-  const uint32_t c = threadIdx.x;
-  if (c >= C) return;
-  const uint32_t p0 = blockIdx.x * kBiasChunk, p1 = min(P, p0 + kBiasChunk);
+// Parameter gradients from the partial sums, and (ADAM) the optimiser step
+// and the packed weights, for 32 parameters per block: eight groups of 32
+// threads each add an eighth of a parameter's partial sums in order, then the
+// groups' sums are added in group order.  One launch of 70 us for a batch of
+// 8 x 128 x 128, where per-layer reductions of weights (8 us) and biases (one
+// block, 41 us), the Adam pass and 19 packing launches took 1.1 ms.
+struct AdamArgs {
+  float *theta, *m, *v;
+  float lr, b1, b2, eps, c1, c2;
+};
+template <bool ADAM>
+__global__ __launch_bounds__(256) void kGradients(LayerTab T, const float* part, float* grad, AdamArgs o, bf16* wf, bf16* wb) {
+  __shared__ float red[8][32];
+  const uint32_t c = threadIdx.x & 31, g = threadIdx.x >> 5;
+  const uint32_t i = blockIdx.x * 32 + c;  // every layer's weights and biases are whole blocks of 32
+  const LayerTab::Row& l = layerOf(T, blockIdx.x * 32);
+  const bool isW = blockIdx.x * 32 < l.bOff;
+  const uint32_t e = isW ? i - l.wOff : i - l.bOff, n = isW ? l.splits : l.nbk;
+  const size_t stride = isW ? size_t(9) * l.CoS * l.CinS : l.CoS;
+  const float* p = part + (isW ? l.wPart : l.bPart) + e;
+  const uint32_t k0 = uint32_t(uint64_t(n) * g / 8), k1 = uint32_t(uint64_t(n) * (g + 1) / 8);
   float s = 0.f;
-  for (uint32_t p = p0; p < p1; ++p) s += dY[size_t(p) * C + c];
-  part[size_t(blockIdx.x) * C + c] = s;
+#pragma unroll 8
+  for (uint32_t k = k0; k < k1; ++k) s += p[k * stride];
+  red[g][c] = s;
+  __syncthreads();
+  if (g) return;
+  for (uint32_t k = 1; k < 8; ++k) s += red[k][c];
+  grad[i] = s;
+  if (ADAM) {
+    const float mi = o.b1 * o.m[i] + (1.f - o.b1) * s;
+    const float vi = o.b2 * o.v[i] + (1.f - o.b2) * s * s;
+    o.m[i] = mi;
+    o.v[i] = vi;
+    const float w = o.theta[i] - o.lr * (mi / o.c1) / (sqrtf(vi / o.c2) + o.eps);
+    o.theta[i] = w;
+    if (isW) packWeight(l, e, w, wf, wb);
+  }
 }
-__global__ void kBiasReduce(const float* part, uint32_t nb, uint32_t C, float* dB) {
-  const uint32_t c = threadIdx.x;
-  if (c >= C) return;
-  float s = 0.f;
-  for (uint32_t b = 0; b < nb; ++b) s += part[size_t(b) * C + c];
-  dB[c] += s;
+
+// Padded parameter vector -> real-channel flat order.
+__global__ __launch_bounds__(256) void kRealOrder(LayerTab T, const float* pad, float* real, uint32_t n) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  int k = 0;
+  while (k + 1 < kNumLayers && i >= T.r[k + 1].rOff) ++k;
+  const LayerTab::Row& l = T.r[k];
+  const uint32_t e = i - l.rOff, nw = 9 * l.co * l.cin;
+  if (e >= nw) {
+    real[i] = pad[l.bOff + (e - nw)];
+    return;
+  }
+  const uint32_t r = e % l.cin, co = (e / l.cin) % l.co, tap = e / (l.cin * l.co);
+  const uint32_t s = r < l.ca ? r : l.CaS + (r - l.ca);
+  real[i] = pad[l.wOff + (tap * l.CoS + co) * l.CinS + s];
 }
 
 // --------------------------------------------------------- elementwise
-__global__ void kReluMask(float* dY, const bf16* Y, size_t n) {
-  size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n && !(float(Y[i]) > 0.f)) dY[i] = 0.f;
-}
-
-__global__ void kPool(const bf16* in, bf16* out, uint32_t N, uint32_t H, uint32_t W, uint32_t C) {
-  size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const uint32_t h = H / 2, w = W / 2;
-  if (i >= size_t(N) * h * w * C) return;
-  uint32_t c = uint32_t(i % C);
-  size_t pix = i / C;
-  uint32_t x = uint32_t(pix % w), y = uint32_t((pix / w) % h), n = uint32_t(pix / (size_t(w) * h));
-  size_t b = ((size_t(n) * H + 2 * y) * W + 2 * x) * C + c;
-  float s = float(in[b]) + float(in[b + C]) + float(in[b + size_t(W) * C]) + float(in[b + size_t(W) * C + C]);
-  out[i] = bf16(0.25f * s);
-}
-
-// dIn[full] += dOut[half] / 4
-__global__ void kPoolBwd(const float* dOut, float* dIn, uint32_t N, uint32_t H, uint32_t W, uint32_t C) {
-  size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= size_t(N) * H * W * C) return;
-  uint32_t c = uint32_t(i % C);
-  size_t pix = i / C;
-  uint32_t x = uint32_t(pix % W), y = uint32_t((pix / W) % H), n = uint32_t(pix / (size_t(W) * H));
-  dIn[i] += 0.25f * dOut[((size_t(n) * (H / 2) + y / 2) * (W / 2) + x / 2) * C + c];
-}
-
-// dHalf += sum of the 2 x 2 full-resolution gradients (nearest upsampling)
-__global__ void kUpBwd(const float* tmp, float* dHalf, uint32_t N, uint32_t H, uint32_t W, uint32_t C) {
-  size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const uint32_t h = H / 2, w = W / 2;
-  if (i >= size_t(N) * h * w * C) return;
-  uint32_t c = uint32_t(i % C);
-  size_t pix = i / C;
-  uint32_t x = uint32_t(pix % w), y = uint32_t((pix / w) % h), n = uint32_t(pix / (size_t(w) * h));
-  size_t b = ((size_t(n) * H + 2 * y) * W + 2 * x) * C + c;
-  dHalf[i] += tmp[b] + tmp[b + C] + tmp[b + size_t(W) * C] + tmp[b + size_t(W) * C + C];
-}
-
 // Raw (P, 10) FP32 -> features (P, 32) BF16
 __global__ void kFeatures(const float* raw, bf16* x, uint32_t P) {
   size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -752,7 +759,7 @@ __global__ void kFeaturesFilm(const float4* rad, const float4* alb, const float4
   size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= size_t(Wp) * Hp) return;
   uint32_t px = uint32_t(i % Wp), py = uint32_t(i / Wp);
-  float f[kInCh] = {};
+  float f[16] = {};
   if (px < W && py < H) {
     size_t s = size_t(py) * W + px;
     float4 r = rad[s];
@@ -767,72 +774,55 @@ __global__ void kFeaturesFilm(const float4* rad, const float4* alb, const float4
     }
     if (dep) f[9] = log1pf(fmaxf(dep[s].x, 0.f));
   }
-  bf16* o = x + i * 32;
-  for (uint32_t c = 0; c < 32; ++c) o[c] = bf16(c < kInCh ? f[c] : 0.f);
-}
-
-__global__ void kFilmOut(const float* y, uint32_t C, uint32_t W, uint32_t H, uint32_t Wp, float4* out) {
-  size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= size_t(W) * H) return;
-  uint32_t px = uint32_t(i % W), py = uint32_t(i / W);
-  const float* v = y + (size_t(py) * Wp + px) * C;
-  out[i] = make_float4(fmaxf(expm1f(v[0]), 0.f), fmaxf(expm1f(v[1]), 0.f), fmaxf(expm1f(v[2]), 0.f), 1.f);
-}
-
-__global__ void kOutRgb(const float* y, uint32_t C, uint32_t P, float* rgb) {
-  size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= size_t(P) * 3) return;
-  rgb[i] = expm1f(y[(i / 3) * C + i % 3]);
-}
-
-// Mean L1 in log space; dY = sign / (3P).  One partial sum per block.
-__global__ __launch_bounds__(256) void kLoss(const float* y, uint32_t C, const float* target, uint32_t P, float* dY,
-                                             float* partial) {
-  __shared__ float red[256];
-  size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  float l = 0.f;
-  if (i < size_t(P) * C) {
-    uint32_t c = uint32_t(i % C);
-    size_t p = i / C;
-    float g = 0.f;
-    if (c < kOutCh) {
-      float d = y[i] - log1pf(fmaxf(target[p * kOutCh + c], 0.f));
-      l = fabsf(d);
-      g = (d > 0.f ? 1.f : (d < 0.f ? -1.f : 0.f)) / float(3.0 * double(P));
-    }
-    dY[i] = g;
+  bf16x8* o = reinterpret_cast<bf16x8*>(x + i * 32);
+  for (int k = 0; k < 2; ++k) {
+    bf16x8 v;
+    for (int j = 0; j < 8; ++j) v[j] = bf16(f[8 * k + j]);
+    o[k] = v;
   }
-  red[threadIdx.x] = l;
+  o[2] = o[3] = zero8();
+}
+
+// Mean L1 in log space: per pixel the gradient sign / (3P) of the three
+// channels as the last layer's BF16 output gradient, per block of 256 pixels
+// the partial loss and bias-gradient sums (trees of fixed order).
+__global__ __launch_bounds__(256) void kLoss(const float4* y, const float* target, uint32_t P, bf16* dY, float* partial,
+                                             float* bPart) {
+  __shared__ float4 red[256];
+  const uint32_t p = blockIdx.x * 256 + threadIdx.x;
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);  // gradients of the three channels, loss
+  if (p < P) {
+    const float4 v = y[p];
+    const float d[3] = {v.x - log1pf(fmaxf(target[3 * size_t(p)], 0.f)), v.y - log1pf(fmaxf(target[3 * size_t(p) + 1], 0.f)),
+                        v.z - log1pf(fmaxf(target[3 * size_t(p) + 2], 0.f))};
+    float g[3];
+    for (int c = 0; c < 3; ++c) {
+      s.w += fabsf(d[c]);
+      g[c] = (d[c] > 0.f ? 1.f : (d[c] < 0.f ? -1.f : 0.f)) / float(3.0 * double(P));
+    }
+    s.x = g[0], s.y = g[1], s.z = g[2];
+    bf16x8 o = zero8();
+    bf16x8* row = reinterpret_cast<bf16x8*>(dY + size_t(p) * 32);
+    row[1] = row[2] = row[3] = o;
+    o[0] = bf16(g[0]), o[1] = bf16(g[1]), o[2] = bf16(g[2]);
+    row[0] = o;
+  }
+  red[threadIdx.x] = s;
   __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (int(threadIdx.x) < s) red[threadIdx.x] += red[threadIdx.x + s];
+  for (int k = 128; k > 0; k >>= 1) {
+    if (int(threadIdx.x) < k) {
+      const float4 b = red[threadIdx.x + k];
+      float4& a = red[threadIdx.x];
+      a.x += b.x, a.y += b.y, a.z += b.z, a.w += b.w;
+    }
     __syncthreads();
   }
-  if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
-}
-
-__global__ void kAdam(float* w, const float* g, float* m, float* v, size_t n, float lr, float b1, float b2, float eps,
-                      float c1, float c2) {
-  size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float gi = g[i];
-  float mi = b1 * m[i] + (1.f - b1) * gi;
-  float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-}
-
-// FP32 master W[9][Cout][Cin] -> BF16 Wf (same layout) and Wb [9][Cin][Cout]
-__global__ void kPackW(const float* w, uint32_t Cout, uint32_t Cin, bf16* wf, bf16* wb) {
-  size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= size_t(9) * Cout * Cin) return;
-  uint32_t ci = uint32_t(i % Cin);
-  size_t t = i / Cin;
-  uint32_t co = uint32_t(t % Cout), tap = uint32_t(t / Cout);
-  bf16 v = bf16(w[i]);
-  wf[i] = v;
-  wb[(size_t(tap) * Cin + ci) * Cout + co] = v;
+  if (threadIdx.x == 0) partial[blockIdx.x] = red[0].w;
+  if (threadIdx.x < 32) {
+    const float4 r = red[0];
+    bPart[size_t(blockIdx.x) * 32 + threadIdx.x] =
+        threadIdx.x == 0 ? r.x : threadIdx.x == 1 ? r.y : threadIdx.x == 2 ? r.z : 0.f;
+  }
 }
 
 template <class T> struct Buf {
@@ -870,8 +860,10 @@ struct Layer {
 
 struct Act {
   uint32_t N, H, W, C;
+  int layer = -1;   // the layer that writes it
   Buf<bf16> a;
-  Buf<float> g;
+  Buf<bf16> g;      // training: its complete gradient, ReLU mask applied
+  Buf<float> skip;  // training: the skip branch's part of the gradient (encoder outputs)
   size_t count() const { return size_t(N) * H * W * C; }
 };
 
@@ -891,8 +883,10 @@ struct ash_denoiser {
   uint32_t N = 0, H = 0, W = 0;
   Act x, out;
   Act enc[kLevels][2], pooled[kLevels], dec[kLevels][2];
-  Buf<float> upTmp, outF, lossPart, raw, target, rgb;
-  Buf<float> wPart, bPart;  // backward-w and bias-gradient partial sums
+  Buf<float> outF, lossPart, raw, target, rgb;
+  Buf<float> part;  // weight and bias gradient partial sums of all layers
+  Buf<float> real;  // parameters or gradient in the real-channel order
+  int numCU = 256;
   bool wDirty = true;
 };
 
@@ -961,7 +955,7 @@ static size_t realCount(const ash_denoiser* d) {
   return n;
 }
 
-// padded device layout <-> real-channel flat order
+// real-channel flat order -> padded device layout
 static void toPadded(const ash_denoiser* d, const float* real, std::vector<float>& pad) {
   pad.assign(d->nParams, 0.f);
   size_t k = 0;
@@ -979,40 +973,43 @@ static void toPadded(const ash_denoiser* d, const float* real, std::vector<float
   }
 }
 
-static void fromPadded(const ash_denoiser* d, const std::vector<float>& pad, float* real) {
+// Every layer's offsets; the partial-sum fields are filled by the backward pass.
+static LayerTab layerTab(const ash_denoiser* d) {
+  LayerTab T;
+  std::memset(&T, 0, sizeof T);
   size_t k = 0;
-  for (auto& l : d->L) {
-    uint32_t cin = l.CaS + l.CbS, rin = l.ca + l.cb;
-    for (uint32_t t = 0; t < 9; ++t)
-      for (uint32_t co = 0; co < l.co; ++co)
-        for (uint32_t s = 0; s < cin; ++s) {
-          int r = realIn(l, s);
-          if (r >= 0) real[k + (size_t(t) * l.co + co) * rin + r] = pad[l.wOff + (size_t(t) * l.CoS + co) * cin + s];
-        }
-    k += size_t(9) * l.co * rin;
-    for (uint32_t co = 0; co < l.co; ++co) real[k + co] = pad[l.bOff + co];
-    k += l.co;
+  for (size_t i = 0; i < d->L.size(); ++i) {
+    const Layer& l = d->L[i];
+    LayerTab::Row& r = T.r[i];
+    r.CoS = l.CoS, r.CinS = l.CaS + l.CbS, r.co = l.co, r.ca = l.ca, r.CaS = l.CaS, r.cin = l.ca + l.cb;
+    r.wOff = uint32_t(l.wOff), r.bOff = uint32_t(l.bOff), r.fOff = uint32_t(l.fOff), r.rOff = uint32_t(k);
+    k += size_t(9) * l.co * (l.ca + l.cb) + l.co;
   }
+  return T;
 }
 
 static int packWeights(ash_denoiser* d) {
   if (!d->wDirty) return ASH_OK;
-  for (auto& l : d->L) {
-    uint32_t cin = l.CaS + l.CbS;
-    size_t n = size_t(9) * l.CoS * cin;
-    kPackW<<<blocks(n), 256, 0, d->stream>>>(d->theta.p + l.wOff, l.CoS, cin, d->wf.p + l.fOff, d->wb.p + l.fOff);
-  }
+  kPackW<<<blocks(d->nParams), 256, 0, d->stream>>>(layerTab(d), d->theta.p, uint32_t(d->nParams), d->wf.p, d->wb.p);
   DH(d, hipGetLastError());
   d->wDirty = false;
   return ASH_OK;
 }
 
-static uint32_t splitsFor(size_t P) { return uint32_t(std::max<size_t>(1, std::min<size_t>(256, P / 2048))); }
+// Copies a padded parameter-sized vector to the host in the real-channel order.
+static int readReal(ash_denoiser* d, const float* pad, float* host) {
+  const size_t n = realCount(d);
+  DH(d, d->real.reserve(n));
+  kRealOrder<<<blocks(n), 256, 0, d->stream>>>(layerTab(d), pad, d->real.p, uint32_t(n));
+  DH(d, hipGetLastError());
+  DH(d, hipMemcpyAsync(host, d->real.p, n * sizeof(float), hipMemcpyDeviceToHost, d->stream));
+  DH(d, hipStreamSynchronize(d->stream));
+  return ASH_OK;
+}
 
 static int allocAct(ash_denoiser* d, Act& t, uint32_t N, uint32_t H, uint32_t W, uint32_t C) {
   t.N = N, t.H = H, t.W = W, t.C = C;
   DH(d, t.a.reserve(t.count()));
-  DH(d, t.g.reserve(t.count()));
   return ASH_OK;
 }
 
@@ -1035,148 +1032,242 @@ static int ensureShape(ash_denoiser* d, uint32_t N, uint32_t H, uint32_t W) {
   }
   CK(allocAct(d, d->out, N, H, W, 32));
 #undef CK
-  size_t P = size_t(N) * H * W;
-  DH(d, d->upTmp.reserve(P * 128));
-  DH(d, d->outF.reserve(P * 32));
-  DH(d, d->lossPart.reserve(blocks(P * 32)));
   d->N = N, d->H = H, d->W = W;
   return ASH_OK;
-}
-
-static ConvArgs convArgs(ash_denoiser* d, const Layer& l, const Act& s0, bool up, const Act* s1, uint32_t N, uint32_t H,
-                         uint32_t W) {
-  ConvArgs a;
-  std::memset(&a, 0, sizeof a);
-  a.s0 = Src{s0.a.p, s0.g.p, s0.C, up ? 1u : 0u};
-  if (s1) a.s1 = Src{s1->a.p, s1->g.p, s1->C, 0};
-  a.N = N, a.H = H, a.W = W;
-  a.Cin = l.CaS + l.CbS;
-  a.Cout = l.CoS;
-  a.Wf = d->wf.p + l.fOff;
-  a.Wb = d->wb.p + l.fOff;
-  a.bias = d->theta.p + l.bOff;
-  a.relu = l.relu ? 1 : 0;
-  a.upTmp = d->upTmp.p;
-  a.dW = d->grad.p + l.wOff;
-  a.dB = d->grad.p + l.bOff;
-  return a;
 }
 
 // Layer schedule: the conv inputs of every layer in network order.
 struct Step {
   int layer;
-  const Act* s0;
+  Act* s0;
   bool up;
-  const Act* s1;
-  Act* out;  // null: the FP32 output
+  Act* s1;
+  Act* out;
+  Act* pool;  // the pooled copy of the output, or null
 };
 
 static std::vector<Step> schedule(ash_denoiser* d) {
   std::vector<Step> s;
   int li = 0;
-  const Act* h = &d->x;
+  Act* h = &d->x;
+  auto add = [&](Act* s0, bool up, Act* s1, Act* out, Act* pool) {
+    out->layer = li;
+    s.push_back({li++, s0, up, s1, out, pool});
+    h = out;
+  };
   for (int lv = 0; lv < kLevels; ++lv) {
-    if (lv) h = &d->pooled[lv];
-    s.push_back({li++, h, false, nullptr, &d->enc[lv][0]});
-    s.push_back({li++, &d->enc[lv][0], false, nullptr, &d->enc[lv][1]});
-    h = &d->enc[lv][1];
+    add(lv ? &d->pooled[lv] : h, false, nullptr, &d->enc[lv][0], nullptr);
+    add(h, false, nullptr, &d->enc[lv][1], lv + 1 < kLevels ? &d->pooled[lv + 1] : nullptr);
   }
   for (int lv = kLevels - 2; lv >= 0; --lv) {
-    s.push_back({li++, h, true, &d->enc[lv][1], &d->dec[lv][0]});
-    s.push_back({li++, &d->dec[lv][0], false, nullptr, &d->dec[lv][1]});
-    h = &d->dec[lv][1];
+    add(h, true, &d->enc[lv][1], &d->dec[lv][0], nullptr);
+    add(h, false, nullptr, &d->dec[lv][1], nullptr);
   }
-  s.push_back({li++, h, false, nullptr, nullptr});
+  add(h, false, nullptr, &d->out, nullptr);
   return s;
 }
 
-static int forwardPass(ash_denoiser* d) {
+// Which kernel runs a convolution and its pixel tiles.
+enum ConvKind { kKindSplit, kKind4, kKind8, kKind8x2 };
+struct ConvPlan {
+  ConvKind kind;
+  uint32_t tilesX, tilesY, tiles;  // tiles = N tilesX tilesY
+};
+static ConvPlan convPlan(const ash_denoiser* d, uint32_t N, uint32_t H, uint32_t W, uint32_t nCg) {
+  auto make = [&](ConvKind k, uint32_t tr, uint32_t tc) {
+    ConvPlan p{k, (W + tc - 1) / tc, (H + tr - 1) / tr, 0};
+    p.tiles = N * p.tilesX * p.tilesY;
+    return p;
+  };
+  const uint32_t cus = uint32_t(d->numCU);
+  if (nCg % 2 == 0) {
+    const ConvPlan p = make(kKind8x2, 16, 16);
+    if (uint64_t(p.tiles) * (nCg / 2) >= 2 * cus) return p;
+  }
+  const ConvPlan p8 = make(kKind8, 16, 32);
+  if (uint64_t(p8.tiles) * nCg >= 2 * cus) return p8;
+  const ConvPlan p4 = make(kKind4, 8, 32);
+  if (uint64_t(p4.tiles) * nCg >= cus) return p4;
+  return make(kKindSplit, kSplitRows, 16);
+}
+
+template <int R, int CW, int NT, ConvMode MODE>
+static void convLds(const ash_denoiser* d, const ConvArgs& a, const ConvPlan& p) {
+  const uint32_t cgb = a.nCg / CW, items = p.tiles * cgb;
+  const uint32_t cap = std::max<uint32_t>(uint32_t(d->numCU) * (R == 8 ? 2 : 3) / cgb, 1) * cgb;  // whole sets of output groups
+  kConvLds<R, CW, NT, MODE><<<std::min(items, cap), 256, ConvTile<R, CW>::lds, d->stream>>>(a, p.tilesX, p.tilesY, items);
+}
+template <ConvMode MODE>
+static void launchConv(const ash_denoiser* d, const ConvArgs& a, const ConvPlan& p) {
+  constexpr int NT = MODE == kModeLast ? 1 : 2;  // the last layer's 3 channels lie in the first of the group's two tiles
+  if (p.kind == kKindSplit) {
+    const size_t lds = size_t(a.nCh) * kSplitRows * 64 * 8 * sizeof(float);
+    kConvSplit<MODE><<<p.tiles * a.nCg, 64 * a.nCh, lds, d->stream>>>(a, p.tilesX, p.tilesY);
+  } else if (p.kind == kKind4) {
+    convLds<4, 1, NT, MODE>(d, a, p);
+  } else if (p.kind == kKind8 || MODE == kModeLast) {
+    convLds<8, 1, NT, MODE>(d, a, p);
+  } else {
+    convLds<8, 2, NT, MODE>(d, a, p);
+  }
+}
+
+// What the last layer writes (null: not wanted).
+struct Output {
+  float* pred = nullptr;    // [pixel][4], log space
+  float* rgb = nullptr;     // [pixel][3]
+  float4* film = nullptr;   // filmW x filmH RGBA
+  uint32_t filmW = 0, filmH = 0;
+};
+
+static int checkLayer(ash_denoiser* d, const Step& st) {
+  const Layer& l = d->L[st.layer];
+  const Act& o = *st.out;
+  const bool fits = st.s0->C == l.CaS && (st.s1 ? st.s1->C : 0) == l.CbS && o.C == l.CoS && l.CaS + l.CbS <= 32 * kMaxChunks &&
+                    l.CoS <= 32 * kMaxChunks && st.s0->H * (st.up ? 2 : 1) == o.H && st.s0->W * (st.up ? 2 : 1) == o.W &&
+                    (!st.s1 || (st.s1->H == o.H && st.s1->W == o.W));
+  return fits ? ASH_OK : dfail(d, ASH_E_INVALID, "layer %d: shape or channel layout mismatch", st.layer);
+}
+
+static int forwardPass(ash_denoiser* d, const Output& out) {
   int rc = packWeights(d);
   if (rc) return rc;
-  const uint32_t N = d->N;
-  auto sched = schedule(d);
-  for (const Step& st : sched) {
+  for (const Step& st : schedule(d)) {
+    if ((rc = checkLayer(d, st))) return rc;
     const Layer& l = d->L[st.layer];
-    const Act& o = st.out ? *st.out : d->out;
-    uint32_t H = o.H, W = o.W;
-    if (st.s0 != &d->x && !st.up && st.s0->H != H) return dfail(d, ASH_E_INVALID, "shape mismatch");
-    // the pooled input of an encoder level is produced just before its first conv
-    for (int lv = 1; lv < kLevels; ++lv)
-      if (st.s0 == &d->pooled[lv]) {
-        const Act& src = d->enc[lv - 1][1];
-        kPool<<<blocks(d->pooled[lv].count()), 256, 0, d->stream>>>(src.a.p, d->pooled[lv].a.p, N, src.H, src.W, src.C);
-      }
-    ConvArgs a = convArgs(d, l, *st.s0, st.up, st.s1, N, H, W);
-    if (a.Cin != a.s0.C + a.s1.C || a.Cout != o.C || a.Cin > 16 * kMaxTiles || a.Cout > 16 * kMaxTiles)
-      return dfail(d, ASH_E_INVALID, "layer %d: channel layout mismatch", st.layer);
-    if (st.out) a.Y = st.out->a.p;
-    else a.Yf = d->outF.p;
-    size_t P = size_t(N) * H * W;
-    if (!launchConvFwd(a, P, d->stream)) return dfail(d, ASH_E_INVALID, "layer %d: %u output channels", st.layer, a.Cout);
+    const Act& o = *st.out;
+    ConvArgs a;
+    std::memset(&a, 0, sizeof a);
+    a.s0 = Src{st.s0->a.p, st.s0->C, st.up ? 1u : 0u};
+    if (st.s1) a.s1 = Src{st.s1->a.p, st.s1->C, 0};
+    a.N = o.N, a.H = o.H, a.W = o.W;
+    a.nCh = (l.CaS + l.CbS) / 32, a.nCg = l.CoS / 32;
+    a.Wp = d->wf.p + l.fOff;
+    a.bias = d->theta.p + l.bOff;
+    if (l.relu) {
+      a.Y = o.a.p;
+      if (st.pool) a.pool = st.pool->a.p;
+    } else {
+      a.Yf = out.pred, a.rgb = out.rgb, a.film = out.film, a.filmW = out.filmW, a.filmH = out.filmH;
+    }
+    const ConvPlan plan = convPlan(d, a.N, a.H, a.W, a.nCg);
+    if (l.relu) launchConv<kModeAct>(d, a, plan);
+    else launchConv<kModeLast>(d, a, plan);
   }
   DH(d, hipGetLastError());
   return ASH_OK;
 }
 
-// Gradient of the loss w.r.t. all parameters into d->grad (after forwardPass
-// and the loss kernel wrote the output gradient into d->out.g).
-static int backwardPass(ash_denoiser* d) {
-  const uint32_t N = d->N;
-  DH(d, hipMemsetAsync(d->grad.p, 0, d->nParams * sizeof(float), d->stream));
-  auto zero = [&](Act& t) { return hipMemsetAsync(t.g.p, 0, t.count() * sizeof(float), d->stream); };
-  for (int lv = 0; lv < kLevels; ++lv) {
-    DH(d, zero(d->enc[lv][0]));
-    DH(d, zero(d->enc[lv][1]));
-    if (lv) DH(d, zero(d->pooled[lv]));
-    if (lv < kLevels - 1) {
-      DH(d, zero(d->dec[lv][0]));
-      DH(d, zero(d->dec[lv][1]));
+// Forward pass of a training batch: prediction kept in outF, gradient buffers made.
+static int trainForward(ash_denoiser* d) {
+  const size_t P = size_t(d->N) * d->H * d->W;
+  DH(d, d->outF.reserve(P * 4));
+  DH(d, d->lossPart.reserve(blocks(P)));
+  DH(d, d->out.g.reserve(d->out.count()));
+  for (int lv = 0; lv < kLevels; ++lv)
+    for (int k = 0; k < 2; ++k) {
+      DH(d, d->enc[lv][k].g.reserve(d->enc[lv][k].count()));
+      if (lv < kLevels - 1) DH(d, d->dec[lv][k].g.reserve(d->dec[lv][k].count()));
+      if (lv < kLevels - 1 && k) DH(d, d->enc[lv][k].skip.reserve(d->enc[lv][k].count()));
     }
-  }
-  auto sched = schedule(d);
-  // partial-sum space of the largest layer (splits x weights) and of the
-  // finest level's bias blocks; kept across calls
-  size_t wp = 0;
+  Output o;
+  o.pred = d->outF.p;
+  return forwardPass(d, o);
+}
+
+// Pixel tiles of a layer's weight gradient: 32, 16 or 8 columns by the
+// image's width, and one split per tile up to two blocks per CU.
+struct BwdWPlan {
+  uint32_t tc, tilesX, tilesY, tiles, splits;
+};
+static BwdWPlan bwdWPlan(const ash_denoiser* d, const Layer& l, uint32_t N, uint32_t H, uint32_t W) {
+  BwdWPlan p;
+  p.tc = W > 16 ? 32 : W > 8 ? 16 : 8;
+  const uint32_t tr = 256 / p.tc, pairs = (l.CoS / 32) * ((l.CaS + l.CbS) / 32);
+  p.tilesX = (W + p.tc - 1) / p.tc, p.tilesY = (H + tr - 1) / tr;
+  p.tiles = N * p.tilesX * p.tilesY;
+  p.splits = std::max<uint32_t>(1, std::min(p.tiles, 2 * uint32_t(d->numCU) / pairs));
+  return p;
+}
+
+// Loss, then the gradient of the loss w.r.t. all parameters into d->grad;
+// with `adam`, the optimiser step too.
+static int backwardPass(ash_denoiser* d, const AdamArgs* adam) {
+  const std::vector<Step> sched = schedule(d);
+  const uint32_t N = d->N;
+  const size_t P = size_t(N) * d->H * d->W;
+  // a convolution's backward-x plan, and the partial sums' places
+  auto xPlan = [&](const Step& st) { return convPlan(d, N, st.out->H, st.out->W, (d->L[st.layer].CaS + d->L[st.layer].CbS) / 32); };
+  LayerTab T = layerTab(d);
   for (const Step& st : sched) {
     const Layer& l = d->L[st.layer];
-    const Act& o = st.out ? *st.out : d->out;
-    wp = std::max(wp, size_t(9) * l.CoS * (l.CaS + l.CbS) * splitsFor(size_t(N) * o.H * o.W));
+    T.r[st.layer].splits = bwdWPlan(d, l, N, st.out->H, st.out->W).splits;
+    // the bias gradient is summed where the output's gradient is completed: by the layer that reads it
+    // (its pooled copy, where there is one), or by the loss
+    int made = -1;
+    if (st.layer > 0) {
+      const Act* src = st.s0;
+      for (int lv = 1; lv < kLevels; ++lv)
+        if (src == &d->pooled[lv]) src = &d->enc[lv - 1][1];
+      made = src->layer;
+    }
+    if (made >= 0) T.r[made].nbk = xPlan(st).tiles;
   }
-  DH(d, d->wPart.reserve(wp));
-  DH(d, d->bPart.reserve(size_t(blocks(size_t(N) * d->H * d->W, kBiasChunk)) * 128));
+  T.r[sched.back().layer].nbk = blocks(P);
+  size_t off = 0;
+  for (auto& r : T.r) {
+    r.wPart = off;
+    off += size_t(r.splits) * 9 * r.CoS * r.CinS;
+    r.bPart = off;
+    off += size_t(r.nbk) * r.CoS;
+  }
+  DH(d, d->part.reserve(off));
+  kLoss<<<blocks(P), 256, 0, d->stream>>>(reinterpret_cast<const float4*>(d->outF.p), d->target.p, uint32_t(P), d->out.g.p,
+                                          d->lossPart.p, d->part.p + T.r[sched.back().layer].bPart);
   for (int k = int(sched.size()) - 1; k >= 0; --k) {
     const Step& st = sched[k];
     const Layer& l = d->L[st.layer];
-    const Act& o = st.out ? *st.out : d->out;
-    const uint32_t H = o.H, W = o.W;
-    const size_t P = size_t(N) * H * W;
-    if (st.out && l.relu) kReluMask<<<blocks(o.count()), 256, 0, d->stream>>>(o.g.p, o.a.p, o.count());
-    ConvArgs a = convArgs(d, l, *st.s0, st.up, st.s1, N, H, W);
-    if (a.Cin != a.s0.C + a.s1.C || a.Cout != o.C) return dfail(d, ASH_E_INVALID, "layer %d: channel layout mismatch", st.layer);
-    a.dY = o.g.p;
-    a.splits = splitsFor(P);
-    a.wPart = d->wPart.p;
-    const size_t nW = size_t(9) * a.Cout * a.Cin;
-    if (nW * a.splits > d->wPart.n || a.Cout > 128)
-      return dfail(d, ASH_E_INVALID, "layer %d: gradient partial buffer too small", st.layer);
-    size_t tasks = size_t(9) * (a.Cout / 32) * (a.Cin / 32) * a.splits;
-    kConvBwdW<<<blocks(tasks, 4), 256, 0, d->stream>>>(a);
-    kReduceSplits<<<blocks(nW), 256, 0, d->stream>>>(d->wPart.p, a.splits, nW, a.dW);
-    const unsigned nb = blocks(P, kBiasChunk);
-    kBiasPart<<<nb, 128, 0, d->stream>>>(a.dY, uint32_t(P), a.Cout, d->bPart.p);
-    kBiasReduce<<<1, 128, 0, d->stream>>>(d->bPart.p, nb, a.Cout, a.dB);
+    const Act& o = *st.out;
+    const BwdWPlan wp = bwdWPlan(d, l, N, o.H, o.W);
+    BwdWArgs b;
+    std::memset(&b, 0, sizeof b);
+    b.s0 = Src{st.s0->a.p, st.s0->C, st.up ? 1u : 0u};
+    if (st.s1) b.s1 = Src{st.s1->a.p, st.s1->C, 0};
+    b.dY = o.g.p;
+    b.N = N, b.H = o.H, b.W = o.W;
+    b.nCo = l.CoS / 32, b.nCi = (l.CaS + l.CbS) / 32;
+    b.splits = wp.splits, b.tilesX = wp.tilesX, b.tilesY = wp.tilesY, b.tiles = wp.tiles;
+    b.part = d->part.p + T.r[st.layer].wPart;
+    const uint32_t grid = b.nCo * b.nCi * b.splits;
+    if (wp.tc == 32) kConvBwdW<32><<<grid, 256, 0, d->stream>>>(b);
+    else if (wp.tc == 16) kConvBwdW<16><<<grid, 256, 0, d->stream>>>(b);
+    else kConvBwdW<8><<<grid, 256, 0, d->stream>>>(b);
     if (st.s0 == &d->x) continue;  // no gradient for the input features
-    if (st.up) DH(d, hipMemsetAsync(d->upTmp.p, 0, P * st.s0->C * sizeof(float), d->stream));
-    kConvBwdX<<<blocks(P, 64), 256, 0, d->stream>>>(a);
-    if (st.up)
-      kUpBwd<<<blocks(st.s0->count()), 256, 0, d->stream>>>(d->upTmp.p, st.s0->g.p, N, H, W, st.s0->C);
+    ConvArgs a;
+    std::memset(&a, 0, sizeof a);
+    a.s0 = Src{o.g.p, o.C, 0};
+    a.N = N, a.H = o.H, a.W = o.W;
+    a.nCh = l.CoS / 32, a.nCg = (l.CaS + l.CbS) / 32;
+    a.Wp = d->wb.p + l.fOff;
+    a.cg0 = l.CaS / 32;
+    Act* dst = st.s0;
+    a.d0.kind = st.up ? kGradUp : kGradFinal;
     for (int lv = 1; lv < kLevels; ++lv)
-      if (st.s0 == &d->pooled[lv]) {
-        Act& e = d->enc[lv - 1][1];
-        kPoolBwd<<<blocks(e.count()), 256, 0, d->stream>>>(d->pooled[lv].g.p, e.g.p, N, e.H, e.W, e.C);
+      if (dst == &d->pooled[lv]) {
+        dst = &d->enc[lv - 1][1];
+        a.d0.kind = kGradPool;
+        a.d0.skip = dst->skip.p;
       }
+    a.d0.C = dst->C, a.d0.g = dst->g.p, a.d0.act = dst->a.p;
+    a.d0.bPart = d->part.p + T.r[dst->layer].bPart;
+    if (st.s1) a.d1.kind = kGradSkip, a.d1.C = st.s1->C, a.d1.skip = st.s1->skip.p;
+    launchConv<kModeGrad>(d, a, xPlan(st));
   }
+  const uint32_t nb = uint32_t(d->nParams / 32);
+  if (adam) kGradients<true><<<nb, 256, 0, d->stream>>>(T, d->part.p, d->grad.p, *adam, d->wf.p, d->wb.p);
+  else kGradients<false><<<nb, 256, 0, d->stream>>>(T, d->part.p, d->grad.p, AdamArgs{}, nullptr, nullptr);
   DH(d, hipGetLastError());
+  if (adam) ++d->step;
   return ASH_OK;
 }
 
@@ -1195,12 +1286,11 @@ static int uploadBatch(ash_denoiser* d, uint32_t n, uint32_t h, uint32_t w, cons
   return ASH_OK;
 }
 
-static int lossAndBackward(ash_denoiser* d, float* loss) {
+static int lossAndBackward(ash_denoiser* d, float* loss, const AdamArgs* adam) {
   size_t P = size_t(d->N) * d->H * d->W;
-  unsigned nb = blocks(P * 32);
-  kLoss<<<nb, 256, 0, d->stream>>>(d->outF.p, 32, d->target.p, uint32_t(P), d->out.g.p, d->lossPart.p);
+  unsigned nb = blocks(P);
   std::vector<float> part(nb);
-  int rc = backwardPass(d);
+  int rc = backwardPass(d, adam);
   if (rc) return rc;
   DH(d, hipMemcpyAsync(part.data(), d->lossPart.p, nb * sizeof(float), hipMemcpyDeviceToHost, d->stream));
   DH(d, hipStreamSynchronize(d->stream));
@@ -1223,6 +1313,8 @@ int ash_denoiser_create(int device, uint32_t seed, ash_denoiser** out) {
     delete d;
     return ASH_E_HIP;
   }
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && cus > 0) d->numCU = cus;
   buildLayers(d);
   if (d->theta.alloc(d->nParams) || d->grad.alloc(d->nParams) || d->m.alloc(d->nParams) || d->v.alloc(d->nParams) ||
       d->wf.alloc(d->nPacked) || d->wb.alloc(d->nPacked)) {
@@ -1253,10 +1345,10 @@ void ash_denoiser_destroy(ash_denoiser* d) {
   if (!d) return;
   (void)hipSetDevice(d->device);
   if (d->stream) (void)hipStreamSynchronize(d->stream);
-  for (auto* b : {&d->theta, &d->grad, &d->m, &d->v, &d->upTmp, &d->outF, &d->lossPart, &d->raw, &d->target, &d->rgb})
+  for (auto* b : {&d->theta, &d->grad, &d->m, &d->v, &d->outF, &d->lossPart, &d->raw, &d->target, &d->rgb, &d->part, &d->real})
     b->release();
   d->wf.release(), d->wb.release();
-  auto rel = [](Act& t) { t.a.release(), t.g.release(); };
+  auto rel = [](Act& t) { t.a.release(), t.g.release(), t.skip.release(); };
   rel(d->x), rel(d->out);
   for (int lv = 0; lv < kLevels; ++lv) {
     rel(d->enc[lv][0]), rel(d->enc[lv][1]), rel(d->pooled[lv]), rel(d->dec[lv][0]), rel(d->dec[lv][1]);
@@ -1275,12 +1367,8 @@ int ash_denoiser_num_params(ash_denoiser* d, uint64_t* n) {
 
 int ash_denoiser_get_params(ash_denoiser* d, float* host) {
   if (!d || !host) return ASH_E_INVALID;
-  std::vector<float> pad(d->nParams);
   DH(d, hipSetDevice(d->device));
-  DH(d, hipMemcpyAsync(pad.data(), d->theta.p, d->nParams * sizeof(float), hipMemcpyDeviceToHost, d->stream));
-  DH(d, hipStreamSynchronize(d->stream));
-  fromPadded(d, pad, host);
-  return ASH_OK;
+  return readReal(d, d->theta.p, host);
 }
 
 int ash_denoiser_set_params(ash_denoiser* d, const float* host) {
@@ -1300,12 +1388,13 @@ int ash_denoiser_set_params(ash_denoiser* d, const float* host) {
 int ash_denoiser_forward(ash_denoiser* d, uint32_t n, uint32_t h, uint32_t w, const float* input, float* out) {
   if (!d || !input || !out) return ASH_E_INVALID;
   DH(d, hipSetDevice(d->device));
-  int rc = uploadBatch(d, n, h, w, input, nullptr);
-  if (!rc) rc = forwardPass(d);
-  if (rc) return rc;
   size_t P = size_t(n) * h * w;
   if (d->rgb.n < P * 3) DH(d, d->rgb.alloc(P * 3));
-  kOutRgb<<<blocks(P * 3), 256, 0, d->stream>>>(d->outF.p, 32, uint32_t(P), d->rgb.p);
+  Output o;
+  o.rgb = d->rgb.p;
+  int rc = uploadBatch(d, n, h, w, input, nullptr);
+  if (!rc) rc = forwardPass(d, o);
+  if (rc) return rc;
   DH(d, hipMemcpyAsync(out, d->rgb.p, P * 3 * sizeof(float), hipMemcpyDeviceToHost, d->stream));
   DH(d, hipStreamSynchronize(d->stream));
   return ASH_OK;
@@ -1316,14 +1405,10 @@ int ash_denoiser_gradient(ash_denoiser* d, uint32_t n, uint32_t h, uint32_t w, c
   if (!d || !input || !target || !grad) return ASH_E_INVALID;
   DH(d, hipSetDevice(d->device));
   int rc = uploadBatch(d, n, h, w, input, target);
-  if (!rc) rc = forwardPass(d);
-  if (!rc) rc = lossAndBackward(d, loss);
+  if (!rc) rc = trainForward(d);
+  if (!rc) rc = lossAndBackward(d, loss, nullptr);
   if (rc) return rc;
-  std::vector<float> pad(d->nParams);
-  DH(d, hipMemcpyAsync(pad.data(), d->grad.p, d->nParams * sizeof(float), hipMemcpyDeviceToHost, d->stream));
-  DH(d, hipStreamSynchronize(d->stream));
-  fromPadded(d, pad, grad);
-  return ASH_OK;
+  return readReal(d, d->grad.p, grad);
 }
 
 int ash_denoiser_train_step(ash_denoiser* d, uint32_t n, uint32_t h, uint32_t w, const float* input,
@@ -1331,18 +1416,11 @@ int ash_denoiser_train_step(ash_denoiser* d, uint32_t n, uint32_t h, uint32_t w,
   if (!d || !input || !target || !(lr > 0.f)) return ASH_E_INVALID;
   DH(d, hipSetDevice(d->device));
   int rc = uploadBatch(d, n, h, w, input, target);
-  if (!rc) rc = forwardPass(d);
-  if (!rc) rc = lossAndBackward(d, loss);
+  if (!rc) rc = trainForward(d);
   if (rc) return rc;
-  ++d->step;
-  const float b1 = 0.9f, b2 = 0.999f;
-  float c1 = 1.f - std::pow(b1, float(d->step)), c2 = 1.f - std::pow(b2, float(d->step));
-  kAdam<<<blocks(d->nParams), 256, 0, d->stream>>>(d->theta.p, d->grad.p, d->m.p, d->v.p, d->nParams, lr, b1, b2,
-                                                  1e-8f, c1, c2);
-  DH(d, hipGetLastError());
-  d->wDirty = true;
-  DH(d, hipStreamSynchronize(d->stream));
-  return ASH_OK;
+  const float b1 = 0.9f, b2 = 0.999f, step = float(d->step + 1);
+  const AdamArgs adam{d->theta.p, d->m.p, d->v.p, lr, b1, b2, 1e-8f, 1.f - std::pow(b1, step), 1.f - std::pow(b2, step)};
+  return lossAndBackward(d, loss, &adam);
 }
 
 }  // extern "C"
@@ -1359,10 +1437,11 @@ int denoisePlanesAsync(ash_denoiser* d, const void* radiance, const void* albedo
   kFeaturesFilm<<<blocks(size_t(Wp) * Hp), 256, 0, d->stream>>>(
       static_cast<const float4*>(radiance), static_cast<const float4*>(albedo), static_cast<const float4*>(normal),
       static_cast<const float4*>(depth), W, H, Wp, Hp, d->x.a.p);
-  rc = forwardPass(d);
+  Output o;
+  o.film = static_cast<float4*>(out);
+  o.filmW = W, o.filmH = H;
+  rc = forwardPass(d, o);
   if (rc) return rc;
-  kFilmOut<<<blocks(size_t(W) * H), 256, 0, d->stream>>>(d->outF.p, 32, W, H, Wp, static_cast<float4*>(out));
-  DH(d, hipGetLastError());
   DH(d, hipEventRecord(done, d->stream));
   return ASH_OK;
 }

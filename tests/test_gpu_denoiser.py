@@ -234,3 +234,62 @@ def test_gradients_and_training_are_reproducible():
     np.testing.assert_array_equal(d.get_params(), d2.get_params())
     d.close()
     d2.close()
+
+
+@pytest.mark.parametrize("n,h,w", [(1, 16, 16), (3, 16, 48), (2, 48, 80), (1, 32, 336), (1, 272, 16), (5, 64, 64)])
+def test_tile_edges_match_oracle(n, h, w):
+    """Forward and gradient where tiles are cut: levels of one to a few
+    pixels, widths of 8, 16 and 32-column tiles with remainders, one image and
+    odd batches.  Bars: BF16 operands (2^-9 each) through 19 layers measure
+    0.005 in the prediction and 0.005 - 0.01 in the gradient; four times that."""
+    d = A.Denoiser(0, seed=23)
+    theta = bf16(d.get_params()).astype(np.float64)
+    rng = np.random.default_rng(n * 1000 + h + w)
+    raw = _raw(rng, n, h, w)
+    target = np.exp(rng.normal(-1.0, 1.0, size=(n, h, w, 3))).astype(np.float32)
+    x = _features64(raw)
+    ref = U.forward(theta, x)
+    got = np.log1p(d.forward(raw).astype(np.float64))
+    ferr = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    loss, g = d.gradient(raw, target)
+    rl, rg = U.loss_and_grad(theta, x, np.log1p(target.astype(np.float64)))
+    gerr = np.linalg.norm(g - rg) / np.linalg.norm(rg)
+    log(f"{n}x{h}x{w}: forward {ferr:.4f}, gradient {gerr:.4f}, loss {loss:.5f} vs {rl:.5f}")
+    assert ferr <= 0.02 and gerr <= 0.04 and abs(loss - rl) <= 0.01 * rl
+    # Biases, summed apart from the weights.  A bias gradient is a sum over its level's pixels, and a
+    # pre-activation that BF16 rounds to the other side of zero drops or adds a whole pixel of a channel:
+    # of a level's N h w co units about half are on, so four such flips are sqrt(4 / (units / 2)) of the
+    # layer's bias gradient (0.14 on the 2 x 2 pixels x 96 channels of a 16 x 16 image), on top of the
+    # 0.04 above.
+    k = 0
+    levels = [0, 0, 1, 1, 2, 2, 3, 3, 4, 4, 3, 3, 2, 2, 1, 1, 0, 0, 0]
+    for lv, (name, a, b, o, relu) in zip(levels, U.layer_shapes()):
+        k += 9 * (a + b) * o
+        e = np.linalg.norm(g[k:k + o] - rg[k:k + o]) / (np.linalg.norm(rg[k:k + o]) + 1e-12)
+        units = n * (h >> lv) * (w >> lv) * o
+        assert e <= 0.04 + np.sqrt(8.0 / units), (name, e)
+        k += o
+    d.close()
+
+
+def test_large_batch_equals_its_images():
+    """A batch large enough for the large-tile kernels (0.5 M pixels) against
+    its images one by one, which run on the small-tile ones: only the order of
+    the FP32 sums differs, then the BF16 roundings it turns over (0.0005 measured
+    by swapping orders; bar 0.01), and the batch gradient is the images' mean."""
+    n, h, w = 8, 256, 256
+    d = A.Denoiser(0, seed=29)
+    rng = np.random.default_rng(31)
+    raw = _raw(rng, n, h, w)
+    target = np.exp(rng.normal(-1.0, 1.0, size=(n, h, w, 3))).astype(np.float32)
+    out = np.log1p(d.forward(raw))
+    one = np.log1p(np.concatenate([d.forward(raw[i:i + 1]) for i in range(n)]))
+    ferr = np.linalg.norm(out - one) / np.linalg.norm(one)
+    loss, g = d.gradient(raw, target)
+    parts = [d.gradient(raw[i:i + 1], target[i:i + 1]) for i in range(n)]
+    mean = np.mean([p[1].astype(np.float64) for p in parts], 0)
+    gerr = np.linalg.norm(g - mean) / np.linalg.norm(mean)
+    log(f"batch of {n}: forward {ferr:.5f}, gradient {gerr:.5f}")
+    assert ferr <= 0.01 and gerr <= 0.01
+    assert abs(loss - np.mean([p[0] for p in parts])) <= 1e-4 * loss
+    d.close()
