@@ -54,7 +54,7 @@ struct GraphKey {
   Wavefront w;
   const ShotParams* tab;
   ShotParams one;
-  uint32_t grid, iters, n, single, lds, scheme;
+  uint32_t grid, iters, n, single, lds, scheme, walk;
 };
 
 struct GraphEntry {
@@ -117,7 +117,7 @@ struct ash_ctx {
   DBuf<uint32_t> wCtr;
   DBuf<unsigned long long> wCnt64;
   DBuf<WorkUnit> unitBuf;
-  GraphEntry graphs[4];
+  GraphEntry graphs[8];  // the render server: 4 table slots, each with either camera walk
   uint64_t graphClock = 0;
   bool graphsBroken = false;
   // two-level acceleration: BLAS arrays owned here, TLAS and tables
@@ -346,12 +346,12 @@ static int launchLoop(ash_ctx* c, const Wavefront& wf, const SceneView& sc, cons
   double* tShadow = st ? &st->shadow_ms : &scratch;
   double* tTrace = st ? &st->trace_ms : &scratch;
   int cur = 0;
-  const bool coarse = c->numTris <= kCoarseFetchTris;
+  const CameraWalk walk = cameraWalk(c->numTris, b.n, b.nAcc);
   if (!canFuseTrace(sc, scheme)) {
     for (uint32_t it = 0; it < iters; ++it) {
       launchResetCounters(wf, cur, s);
       timed(tExt, [&] {
-        if (it == 0) launchExtendCamera(sc, wf, lds, scheme, grid, count, coarse, s);
+        if (it == 0) launchExtendCamera(sc, wf, lds, scheme, grid, count, walk, s);
         else launchExtend(sc, wf, cur, lds, scheme, grid, count, s);
       });
       timed(tShade, [&] { launchShade(sc, b, wf, cur, shadeRays, s); });
@@ -360,7 +360,7 @@ static int launchLoop(ash_ctx* c, const Wavefront& wf, const SceneView& sc, cons
     }
   } else {
     launchResetCounters(wf, 0, s);
-    timed(tExt, [&] { launchExtendCamera(sc, wf, lds, scheme, grid, count, coarse, s); });
+    timed(tExt, [&] { launchExtendCamera(sc, wf, lds, scheme, grid, count, walk, s); });
     for (uint32_t it = 0; it < iters; ++it) {
       if (it > 0) launchResetShade(wf, cur, s);
       timed(tShade, [&] { launchShade(sc, b, wf, cur, shadeRays, s); });
@@ -405,6 +405,7 @@ static bool graphBounces(ash_ctx* c, const SceneView& sc, const BatchDesc& b, ui
   k.single = b.shots == 1;
   k.lds = lds;
   k.scheme = scheme;
+  k.walk = cameraWalk(c->numTris, b.n, b.nAcc);
   ++c->graphClock;
   for (auto& g : c->graphs)
     if (g.exec && std::memcmp(&g.key, &k, sizeof k) == 0) {
@@ -1478,8 +1479,7 @@ int ash_first_hit(ash_ctx* c, const GpuCamera* cam, ash_hit* out) {
   SceneView sc = viewOf(c);
   launchRaygen(b, c->wf, c->stream);
   launchResetCounters(c->wf, 0, c->stream);
-  launchExtendCamera(sc, c->wf, kStackLds, kSchemeXcdSlices, grid, false, c->numTris <= kCoarseFetchTris,
-                     c->stream);
+  launchExtendCamera(sc, c->wf, kStackLds, kSchemeXcdSlices, grid, false, cameraWalk(c->numTris, P, P), c->stream);
   launchFirstHit(sc, c->shotTab.p, c->wf, dout.p, P, c->stream);
   HIPC(c, hipGetLastError());
   HIPC(c, hipMemcpyAsync(out, dout.p, P * sizeof(ash_hit), hipMemcpyDeviceToHost, c->stream));

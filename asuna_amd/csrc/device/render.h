@@ -145,15 +145,31 @@ void launchRaygen(const BatchDesc& b, const Wavefront& w, hipStream_t s);
 // 4-wide closest-hit kernel
 void launchExtend(const SceneView& sc, const Wavefront& w, int cur, uint32_t ldsStack, uint32_t scheme,
                   uint32_t grid, bool count, hipStream_t s);
-// Closest hit of the camera rays (queue 0 after raygen): the wave-coherent
-// walk on the float 4-wide tree with XCD slices, else launchExtend.
-// coarse: a wave fetches 256 rays per atomic instead of 64 (for trees of at
-// most kCoarseFetchTris triangles, whose cheap rays would otherwise wait on
-// the fetch atomics).
+// Closest hit of the camera rays (queue 0 after raygen).  On the float 4-wide
+// tree with XCD slices, cameraWalk picks the walk:
+//  - per wave (kExtendPacket), when a wave's 64 rays lie close together: from
+//    kPacketFrames frames per pixel (8 pixels per wave), or on a tree of at
+//    most kPacketTris triangles, which every wave walks whole.  kCoarse: a wave
+//    fetches 256 rays per atomic instead of 64 (for trees of at most
+//    kCoarseFetchTris triangles, whose cheap rays would otherwise wait on the
+//    fetch atomics);
+//  - per ray (launchExtend), otherwise: with few frames a wave's rays belong to
+//    up to 64 pixels, reach different leaves, and the wave visits the union.
+// Whole render, per wave / per ray: 5.2 M triangles, 1080p: 1 frame 4.70 / 3.99
+// ms, 2: 6.32 / 5.88, 4: 9.79 / 9.61, 8: 16.85 / 16.83, 16: 30.4 / 31.2; ten
+// 256 x 256 views of a 5,450-triangle scene: 1 frame 3.21 / 2.47, 4: 3.84 /
+// 3.39; the 36-triangle box, 512 x 512: 1 frame 0.88 / 0.91, 4: 2.06 / 2.13.
+// Other schemes and trees: launchExtend.
+enum CameraWalk : uint32_t { kPerRay, kPacket, kCoarse };
+constexpr uint32_t kPacketFrames = 8, kPacketTris = 512;
 constexpr uint32_t kCoarseFetchTris = 1u << 16;
+inline CameraWalk cameraWalk(uint32_t numTris, uint64_t paths, uint64_t pixels) {
+  if (numTris > kPacketTris && paths < kPacketFrames * pixels) return kPerRay;
+  return numTris <= kCoarseFetchTris ? kCoarse : kPacket;
+}
 bool canPacketCamera(const SceneView& sc, uint32_t scheme);
 void launchExtendCamera(const SceneView& sc, const Wavefront& w, uint32_t ldsStack, uint32_t scheme, uint32_t grid,
-                        bool count, bool coarse, hipStream_t s);
+                        bool count, CameraWalk walk, hipStream_t s);
 void launchShade(const SceneView& sc, const BatchDesc& b, const Wavefront& w, int cur, uint32_t maxRays,
                  hipStream_t s);
 void launchShadow(const SceneView& sc, const Wavefront& w, uint32_t scheme, uint32_t grid, bool count,

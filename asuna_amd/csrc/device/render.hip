@@ -3562,12 +3562,12 @@ bool canPacketCamera(const SceneView& sc, uint32_t scheme) {
   return !sc.twoLevel && scheme == kSchemeXcdSlices && sc.nodes4 != nullptr && sc.nodesQ == nullptr;
 }
 void launchExtendCamera(const SceneView& sc, const Wavefront& w, uint32_t ldsStack, uint32_t scheme, uint32_t grid,
-                        bool count, bool coarse, hipStream_t s) {
-  if (!canPacketCamera(sc, scheme)) {
+                        bool count, CameraWalk walk, hipStream_t s) {
+  if (!canPacketCamera(sc, scheme) || walk == kPerRay) {
     launchExtend(sc, w, 0, ldsStack, scheme, grid, count, s);
     return;
   }
-  if (coarse) {
+  if (walk == kCoarse) {
     if (count) kExtendPacket<true, 256><<<grid, kTraceBlock, 0, s>>>(sc, w, 0);
     else kExtendPacket<false, 256><<<grid, kTraceBlock, 0, s>>>(sc, w, 0);
   } else {

@@ -177,3 +177,18 @@ def test_small_queues_are_traced_whole(renderer, box_scene, w, h, two_level):
     assert st["extension_rays"] == ref_st["extension_rays"] and st["shadow_rays"] == ref_st["shadow_rays"]
     for a, b in zip(ref, [renderer.read(i) for i in (0, 1, 8)]):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("frames", [1, 7, 8, 9])
+def test_camera_walk_does_not_change_images(renderer, spheres_small, frames):
+    """Camera rays are walked per ray below 8 frames per pixel and per wave
+    from there; both equal the queue-order scheme, also where one context
+    alternates between them (each walk has its own captured loop)."""
+    s = _load(renderer, spheres_small)
+    ref, _ = _render(renderer, s, frames, traversal=1)
+    for rep in range(2):
+        got, st = _render(renderer, s, frames)
+        assert st["graph_launches"] == st["batches"]
+        for a, b in zip(ref, got):
+            np.testing.assert_array_equal(a, b)
+        _render(renderer, s, 8 if frames < 8 else 1)  # the other walk in between
