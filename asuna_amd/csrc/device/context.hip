@@ -92,6 +92,7 @@ struct ash_ctx {
   bool hasEnv = false;
   DBuf<DevSky> sky;
   uint32_t numTris = 0, numInst = 0;
+  bool hasSide = false;  // some instance's material belongs to the second plugin group
   uint32_t maxDepth = 0;
   float4* nodes = nullptr;
   float4* nodes4 = nullptr;  // 4-wide tree when built with branching 4
@@ -229,6 +230,7 @@ static SceneView viewOf(const ash_ctx* c) {
   v.marg = c->marg.p;
   v.condX = c->condX.p;
   v.sky = c->sky.p;
+  v.hasSide = c->hasSide ? 1u : 0u;
   v.twoLevel = c->twoLevel ? 1u : 0u;
   v.tlas = c->tlas.p;
   v.tlasInst = c->tlasInst.p;
@@ -287,7 +289,7 @@ static int ensureSpill(ash_ctx* c, uint32_t grid) {
       std::max<uint32_t>(uint32_t(kSpill), c->stackNeed > uint32_t(kStackLdsMin) ? c->stackNeed - kStackLdsMin : 0);
   uint32_t threads = grid * kTraceBlock;
   Wavefront& w = c->wf;
-  if (w.spill && w.spillCap >= cap && w.spillThreads == threads) return ASH_OK;
+  if (w.spill && w.spillCap >= cap && w.spillThreads >= threads) return ASH_OK;  // spillThreads is the entries' stride
   MALLOC(c, c->wSpill, size_t(threads) * cap);
   MALLOC(c, c->wSpillT, size_t(threads) * cap);
   w.spill = c->wSpill.p;
@@ -348,27 +350,25 @@ static int launchLoop(ash_ctx* c, const Wavefront& wf, const SceneView& sc, cons
   int cur = 0;
   const CameraWalk walk = cameraWalk(c->numTris, b.n, b.nAcc);
   if (!canFuseTrace(sc, scheme)) {
+    launchResetCounters(wf, s);
     for (uint32_t it = 0; it < iters; ++it) {
-      launchResetCounters(wf, cur, s);
       timed(tExt, [&] {
         if (it == 0) launchExtendCamera(sc, wf, lds, scheme, grid, count, walk, s);
         else launchExtend(sc, wf, cur, lds, scheme, grid, count, s);
       });
       timed(tShade, [&] { launchShade(sc, b, wf, cur, shadeRays, s); });
-      timed(tShadow, [&] { launchShadow(sc, wf, scheme, grid, count, s); });
+      timed(tShadow, [&] { launchShadow(sc, wf, cur, scheme, grid, count, s); });
       cur = 1 - cur;
     }
   } else {
-    launchResetCounters(wf, 0, s);
+    launchResetCounters(wf, s);
     timed(tExt, [&] { launchExtendCamera(sc, wf, lds, scheme, grid, count, walk, s); });
     for (uint32_t it = 0; it < iters; ++it) {
-      if (it > 0) launchResetShade(wf, cur, s);
       timed(tShade, [&] { launchShade(sc, b, wf, cur, shadeRays, s); });
       if (it + 1 < iters) {
-        launchResetExtend(wf, s);
         timed(tTrace, [&] { launchTrace(sc, wf, 1 - cur, lds, grid, count, s); });
       } else {
-        timed(tShadow, [&] { launchShadow(sc, wf, scheme, grid, count, s); });
+        timed(tShadow, [&] { launchShadow(sc, wf, cur, scheme, grid, count, s); });
       }
       cur = 1 - cur;
     }
@@ -554,7 +554,9 @@ static int renderCommon(ash_ctx* c, uint32_t nShots, const ShotParams* hostShots
   }
   int rc = ensureWavefront(c, cap);
   if (rc) return rc;
-  uint32_t grid = uint32_t(std::max(1, c->numCU)) * bpc;
+  // no more blocks than give every extension and every shadow ray of the batch a lane (whole sets of XCDs)
+  const uint64_t need = (2 * ((uint64_t(cap) + kTraceBlock - 1) / kTraceBlock) + kXcds - 1) / kXcds * kXcds;
+  uint32_t grid = uint32_t(std::min<uint64_t>(uint64_t(std::max(1, c->numCU)) * bpc, need));
   rc = ensureSpill(c, grid);
   if (rc) return rc;
   std::vector<WorkUnit> flat;
@@ -1014,6 +1016,7 @@ int ash_upload_scene(ash_ctx* c, const ash_scene_desc* d) {
   std::vector<DevInstance> hinst(d->num_instances);
   std::vector<uint32_t> off(d->num_instances + 1, 0);
   uint64_t tri = 0;
+  bool side = false;
   for (uint32_t i = 0; i < d->num_instances; ++i) {
     const ash_instance_desc& id = d->instances[i];
     if (id.mesh_id >= d->num_meshes) return fail(c, ASH_E_INVALID, "instance %u: mesh id out of range", i);
@@ -1039,6 +1042,7 @@ int ash_upload_scene(ash_ctx* c, const ash_scene_desc* d) {
       const uint32_t t = d->materials[id.material_id].type;
       di.shade = id.material_id | ((t & kShadeTypeMask) << kShadeTypeShift) | (isGroup2Type(t) ? kShadeSide : 0u);
     }
+    side = side || (di.shade & kShadeSide);
     di.triBase = uint32_t(tri);
     off[i] = uint32_t(tri);
     tri += di.ntri;
@@ -1134,6 +1138,7 @@ int ash_upload_scene(ash_ctx* c, const ash_scene_desc* d) {
   HIPC(c, hipStreamSynchronize(s));
   c->numTris = uint32_t(tri);
   c->numInst = d->num_instances;
+  c->hasSide = side;
   c->hasScene = true;
   return ASH_OK;
 }
@@ -1478,7 +1483,7 @@ int ash_first_hit(ash_ctx* c, const GpuCamera* cam, ash_hit* out) {
   b.one = sp;
   SceneView sc = viewOf(c);
   launchRaygen(b, c->wf, c->stream);
-  launchResetCounters(c->wf, 0, c->stream);
+  launchResetCounters(c->wf, c->stream);
   launchExtendCamera(sc, c->wf, kStackLds, kSchemeXcdSlices, grid, false, cameraWalk(c->numTris, P, P), c->stream);
   launchFirstHit(sc, c->shotTab.p, c->wf, dout.p, P, c->stream);
   HIPC(c, hipGetLastError());

@@ -54,6 +54,7 @@ struct SceneView {
   const float2* marg;  // H entries (column 0 of the marginal table)
   const float* condX;  // W*H entries: the conditional table's inverse-CDF channel, in 8x4-texel tiles
   const DevSky* sky;   // sun & sky (inUse 0: env map / background)
+  uint32_t hasSide;    // some surface belongs to the second plugin group
   // two-level acceleration (twoLevel = 1): TLAS binary nodes over instances
   // (leaf = one instance: its index in tlasInst), per-instance BLAS slot
   uint32_t twoLevel;
@@ -82,8 +83,8 @@ struct Wavefront {
   int* side;     // second-group shading queue: slots of the current extension queue
   float4* shO;  // shadow rays: origin.xyz, tmax
   float4* shD;  // direction.xyz, path id
-  uint32_t* ctr;  // [0],[1] queue counts, [2] shadow count, [3] extend fetch,
-                  // [4] shadow fetch, [8] second-group shading queue count,
+  uint32_t* ctr;  // [0],[1] queue counts, [2],[5] shadow-ray counts of the bounce that shaded queue 0 / 1
+                  // (shadowCtr), [3] extend fetch, [4] shadow fetch, [8] second-group shading queue count,
                   // [kXcdCtr + 32 j]: fetch counters of the per-XCD queue slices
                   // (j < 8 extend, j >= 8 shadow), one 128-byte line each
   int* spill;       // traversal stack spill: spillCap entries per persistent thread
@@ -172,14 +173,13 @@ void launchExtendCamera(const SceneView& sc, const Wavefront& w, uint32_t ldsSta
                         bool count, CameraWalk walk, hipStream_t s);
 void launchShade(const SceneView& sc, const BatchDesc& b, const Wavefront& w, int cur, uint32_t maxRays,
                  hipStream_t s);
-void launchShadow(const SceneView& sc, const Wavefront& w, uint32_t scheme, uint32_t grid, bool count,
+// Shadow rays appended when queue `cur` was shaded.
+void launchShadow(const SceneView& sc, const Wavefront& w, int cur, uint32_t scheme, uint32_t grid, bool count,
                   hipStream_t s);
 void launchAccumulate(const BatchDesc& b, const Wavefront& w, hipStream_t s);
-void launchResetCounters(const Wavefront& w, int cur, hipStream_t s);
-// Resets of the fused loop: the counts shading appends to (and the shadow
-// fetch counters), and the extension fetch counters.
-void launchResetShade(const Wavefront& w, int cur, hipStream_t s);
-void launchResetExtend(const Wavefront& w, hipStream_t s);
+// Counters before the first bounce; launchShade leaves them ready for the
+// traversal that follows it and for the next bounce's appends.
+void launchResetCounters(const Wavefront& w, hipStream_t s);
 // Shadow rays of the current bounce and extension rays of queue `cur` in
 // one persistent launch (default traversal scheme on the float 4-wide tree).
 bool canFuseTrace(const SceneView& sc, uint32_t scheme);

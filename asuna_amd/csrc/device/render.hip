@@ -629,6 +629,10 @@ __global__ __launch_bounds__(256) void kRaygen(BatchDesc b, Wavefront w) {
   if (p == 0) w.ctr[0] = b.n;
 }
 
+// Count of the shadow rays appended when queue `cur` was shaded (one per
+// queue: a bounce's shading appends while nothing reads the other).
+__device__ __forceinline__ uint32_t* shadowCtr(const Wavefront& w, int cur) { return w.ctr + (cur ? 5 : 2); }
+
 // ---------------------------------------------------------------- extend
 template <bool WIDE, int NL = kStackLds>
 __device__ __forceinline__ void initStack(Stack& st, int* lds, float* ldsT, const Wavefront& w) {
@@ -1223,9 +1227,9 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(8, 
 // adds its path's pending NEE radiance.  TREE: 0 binary, 1 4-wide,
 // 2 quantized 4-wide.
 template <bool COUNT, int TREE, bool XCD>
-__device__ __forceinline__ void shadowLoop(const SceneView& sc, const Wavefront& w, Stack& st, int lane,
+__device__ __forceinline__ void shadowLoop(const SceneView& sc, const Wavefront& w, int cur, Stack& st, int lane,
                                            uint32_t& nNodes, uint32_t& nTris) {
-  const uint32_t count = w.ctr[2];
+  const uint32_t count = *shadowCtr(w, cur);
   ChunkFetch f;
   chunkInit<XCD>(f, XCD ? &w.ctr[kXcdCtr + kXcds * 32] : &w.ctr[4], count);
   uint32_t start;
@@ -1314,10 +1318,10 @@ __device__ __forceinline__ bool anyRound(const SceneView& sc, const TRay& r, flo
 // next one as soon as REFILL lanes of its wave are idle, instead of the
 // wave waiting for the slowest of its 64 rays.
 template <bool COUNT, int REFILL>
-__device__ __forceinline__ void shadowDynLoop(const SceneView& sc, const Wavefront& w, Stack& st, int lane,
+__device__ __forceinline__ void shadowDynLoop(const SceneView& sc, const Wavefront& w, int cur, Stack& st, int lane,
                                               uint32_t& nNodes, uint32_t& nTris) {
   ChunkFetch f;
-  chunkInit<true>(f, &w.ctr[kXcdCtr + kXcds * 32], w.ctr[2]);
+  chunkInit<true>(f, &w.ctr[kXcdCtr + kXcds * 32], *shadowCtr(w, cur));
   bool active = false, drained = f.surplus;
   int pid = -1;
   uint32_t slot = 0;
@@ -1587,9 +1591,9 @@ __device__ __forceinline__ int stepAny2L(const SceneView& sc, const TRay& rw, TR
 // Persistent any-hit loop over the shadow-ray queue with per-lane refill,
 // as extend2LLoop: an unoccluded ray adds its path's pending NEE radiance.
 template <bool COUNT>
-__device__ __forceinline__ void shadow2LLoop(const SceneView& sc, const Wavefront& w, Stack& st, int lane,
+__device__ __forceinline__ void shadow2LLoop(const SceneView& sc, const Wavefront& w, int cur, Stack& st, int lane,
                                              uint32_t& nNodes, uint32_t& nTris) {
-  const uint32_t count = w.ctr[2];
+  const uint32_t count = *shadowCtr(w, cur);
   ChunkFetch f;
   chunkInit<true>(f, &w.ctr[kXcdCtr + kXcds * 32], count);
   bool active = false, drained = f.surplus;
@@ -1647,13 +1651,13 @@ __global__ __launch_bounds__(kTraceBlock) void kExtend2L(SceneView sc, Wavefront
   }
 }
 template <bool COUNT>
-__global__ __launch_bounds__(kTraceBlock) void kShadow2L(SceneView sc, Wavefront w) {
+__global__ __launch_bounds__(kTraceBlock) void kShadow2L(SceneView sc, Wavefront w, int cur) {
   __shared__ int lds[kStackLds * kTraceBlock];
   __shared__ float ldsT[kStackLds * kTraceBlock];
   Stack st;
   initStack<true, kStackLds>(st, lds, ldsT, w);
   uint32_t nNodes = 0, nTris = 0;
-  shadow2LLoop<COUNT>(sc, w, st, __lane_id(), nNodes, nTris);
+  shadow2LLoop<COUNT>(sc, w, cur, st, __lane_id(), nNodes, nTris);
   if (COUNT) {
     atomicAdd(&w.cnt64[2], (unsigned long long)nNodes);
     atomicAdd(&w.cnt64[3], (unsigned long long)nTris);
@@ -1666,13 +1670,13 @@ __global__ __launch_bounds__(kTraceBlock) void kTrace2L(SceneView sc, Wavefront 
   __shared__ float ldsT[kStackLds * kTraceBlock];
   if (COUNT && blockIdx.x == 0 && threadIdx.x == 0) {
     atomicAdd(&w.cnt64[11], (unsigned long long)w.ctr[cur]);
-    atomicAdd(&w.cnt64[12], (unsigned long long)w.ctr[2]);
+    atomicAdd(&w.cnt64[12], (unsigned long long)*shadowCtr(w, 1 - cur));
   }
   Stack st;
   initStack<true, kStackLds>(st, lds, ldsT, w);
   uint32_t eN = 0, eT = 0, sN = 0, sT = 0;
   extend2LLoop<COUNT>(sc, w, cur, st, __lane_id(), eN, eT);
-  shadow2LLoop<COUNT>(sc, w, st, __lane_id(), sN, sT);
+  shadow2LLoop<COUNT>(sc, w, 1 - cur, st, __lane_id(), sN, sT);
   if (COUNT) {
     const unsigned long long v[4] = {eN, eT, sN, sT};
     for (int k = 0; k < 4; ++k) {
@@ -1683,13 +1687,13 @@ __global__ __launch_bounds__(kTraceBlock) void kTrace2L(SceneView sc, Wavefront 
 }
 
 template <bool COUNT, int TREE, bool XCD>
-__global__ __launch_bounds__(kTraceBlock) void kShadow(SceneView sc, Wavefront w) {
+__global__ __launch_bounds__(kTraceBlock) void kShadow(SceneView sc, Wavefront w, int cur) {
   __shared__ int lds[kStackLds * kTraceBlock];
   Stack st;
   initStack<false>(st, lds, nullptr, w);
   uint32_t nNodes = 0, nTris = 0;
-  if (TREE == 1 && XCD) shadowDynLoop<COUNT, kShadowRefill>(sc, w, st, __lane_id(), nNodes, nTris);
-  else shadowLoop<COUNT, TREE, XCD>(sc, w, st, __lane_id(), nNodes, nTris);
+  if (TREE == 1 && XCD) shadowDynLoop<COUNT, kShadowRefill>(sc, w, cur, st, __lane_id(), nNodes, nTris);
+  else shadowLoop<COUNT, TREE, XCD>(sc, w, cur, st, __lane_id(), nNodes, nTris);
   if (COUNT) {
     atomicAdd(&w.cnt64[2], (unsigned long long)nNodes);
     atomicAdd(&w.cnt64[3], (unsigned long long)nTris);
@@ -1713,14 +1717,14 @@ __global__ __launch_bounds__(kTraceBlock) void kTraceDyn(SceneView sc, Wavefront
   uint32_t eN = 0, eT = 0, sN = 0, sT = 0;
   if (COUNT && blockIdx.x == 0 && threadIdx.x == 0) {
     atomicAdd(&w.cnt64[11], (unsigned long long)w.ctr[cur]);
-    atomicAdd(&w.cnt64[12], (unsigned long long)w.ctr[2]);
+    atomicAdd(&w.cnt64[12], (unsigned long long)*shadowCtr(w, 1 - cur));
   }
   Stack st;
   initStack<true, NL>(st, lds, ldsT, w);
   extendDynLoop<COUNT, REFILL>(sc, w, cur, st, lane, eN, eT);
   Stack ss;
   initStack<false, NL>(ss, lds, nullptr, w);
-  shadowDynLoop<COUNT, kShadowRefill>(sc, w, ss, lane, sN, sT);
+  shadowDynLoop<COUNT, kShadowRefill>(sc, w, 1 - cur, ss, lane, sN, sT);
   if (COUNT) {
     const unsigned long long v[4] = {eN, eT, sN, sT};
     for (int k = 0; k < 4; ++k) {
@@ -1906,11 +1910,11 @@ __global__ __launch_bounds__(kTraceBlock) void kExtendWide(SceneView sc, Wavefro
 }
 
 template <bool COUNT>
-__global__ __launch_bounds__(kTraceBlock) void kShadowWide(SceneView sc, Wavefront w) {
+__global__ __launch_bounds__(kTraceBlock) void kShadowWide(SceneView sc, Wavefront w, int cur) {
   __shared__ int lds[kStackLds * kTraceBlock];
   Stack st;
   initStack<false>(st, lds, nullptr, w);
-  const uint32_t count = w.ctr[2];
+  const uint32_t count = *shadowCtr(w, cur);
   uint32_t nNodes = 0, nTris = 0;
   Trav s;
   int pid = -1;
@@ -3305,13 +3309,13 @@ __device__ __forceinline__ void shadeOne(const SceneView& sc, const BatchDesc& b
   // Appends: the NEE shadow ray (maxDist = dist - 2*EPS, rgen:117-122), the
   // continuing path, and the count of delta-lobe NEE rays (counted, not
   // traced; the extension and shadow ray counts are added per bounce by
-  // kStatRays).
+  // kAfterShade).
   int si, ni;
   if (BLOCK) {
-    blockAppend(*sApp, &w.ctr[2], c.shadow, &w.ctr[1 - cur], cont, &w.cnt64[6], c.fromDielectric, si, ni);
+    blockAppend(*sApp, shadowCtr(w, cur), c.shadow, &w.ctr[1 - cur], cont, &w.cnt64[6], c.fromDielectric, si, ni);
   } else {
     waveCount64(&w.cnt64[6], c.fromDielectric);
-    si = waveAppend(&w.ctr[2], c.shadow);
+    si = waveAppend(shadowCtr(w, cur), c.shadow);
     ni = waveAppend(&w.ctr[1 - cur], cont);
   }
   if (si >= 0) {
@@ -3391,29 +3395,27 @@ __global__ __launch_bounds__(256) void kShadeGroup2(SceneView sc, BatchDesc b, W
     shadeOne<ONE, true, kMatGlobal, false>(sc, b, w, cur, w.side[i], nullptr, nullptr);
 }
 
-// EXT: the extension fetch counters; SHADE: the counts shading appends to
-// (next queue 1 - cur, shadow rays, side queue) and the shadow fetch counters.
-template <bool EXT, bool SHADE>
-__global__ void kResetCounters(Wavefront w, int cur) {
-  if (threadIdx.x == 0) {
-    if (SHADE) {
-      w.ctr[1 - cur] = 0;
-      w.ctr[2] = 0;
-      w.ctr[4] = 0;
-      w.ctr[8] = 0;
-    }
-    if (EXT) w.ctr[3] = 0;
-  }
-  if (threadIdx.x < 2 * kXcds && (threadIdx.x < kXcds ? EXT : SHADE)) w.ctr[kXcdCtr + threadIdx.x * 32] = 0;
+// Counters before the first bounce (raygen sets the count of queue 0).
+__global__ void kResetCounters(Wavefront w) {
+  if (threadIdx.x == 0) w.ctr[1] = w.ctr[2] = w.ctr[3] = w.ctr[4] = w.ctr[5] = w.ctr[8] = 0;
+  if (threadIdx.x < 2 * kXcds) w.ctr[kXcdCtr + threadIdx.x * 32] = 0;
 }
 
-// Ray counts of the bounce: every queued path traced one extension ray,
-// every appended shadow ray is traced.
-__global__ void kStatRays(Wavefront w, int cur) {
+// After queue `cur` is shaded: adds the bounce's ray counts (every queued
+// path traced one extension ray, every appended shadow ray is traced), and
+// clears the fetch counters of the traversal that follows and the counts the
+// next bounce appends to: queue `cur`, the other shadow count, the side queue.
+// One launch in place of a count and two resets, which at 4-5 us each were a
+// fifth of a 96 x 64 render.
+__global__ void kAfterShade(Wavefront w, int cur) {
   if (threadIdx.x == 0) {
     w.cnt64[4] += w.ctr[cur];
-    w.cnt64[5] += w.ctr[2];
+    w.cnt64[5] += *shadowCtr(w, cur);
+    w.ctr[cur] = 0;
+    *shadowCtr(w, 1 - cur) = 0;
+    w.ctr[3] = w.ctr[4] = w.ctr[8] = 0;
   }
+  if (threadIdx.x < 2 * kXcds) w.ctr[kXcdCtr + threadIdx.x * 32] = 0;
 }
 
 // Ordered fold of the batch's frames into the output images
@@ -3582,43 +3584,41 @@ void launchShade(const SceneView& sc, const BatchDesc& b, const Wavefront& w, in
   if (b.shots == 1) {
     if (table) kShade<true, true><<<blocks, kShadeBlock, 0, s>>>(sc, b, w, cur);
     else kShade<true, false><<<blocks, kShadeBlock, 0, s>>>(sc, b, w, cur);
-    kShadeGroup2<true><<<512, 256, 0, s>>>(sc, b, w, cur);
+    if (sc.hasSide) kShadeGroup2<true><<<512, 256, 0, s>>>(sc, b, w, cur);
   } else {
     if (table) kShade<false, true><<<blocks, kShadeBlock, 0, s>>>(sc, b, w, cur);
     else kShade<false, false><<<blocks, kShadeBlock, 0, s>>>(sc, b, w, cur);
-    kShadeGroup2<false><<<512, 256, 0, s>>>(sc, b, w, cur);
+    if (sc.hasSide) kShadeGroup2<false><<<512, 256, 0, s>>>(sc, b, w, cur);
   }
-  kStatRays<<<1, 64, 0, s>>>(w, cur);
+  kAfterShade<<<1, 64, 0, s>>>(w, cur);
 }
 template <bool COUNT>
-static void shadowFor(const SceneView& sc, const Wavefront& w, uint32_t scheme, uint32_t grid, hipStream_t s) {
+static void shadowFor(const SceneView& sc, const Wavefront& w, int cur, uint32_t scheme, uint32_t grid, hipStream_t s) {
   const bool wide = sc.nodes4 != nullptr, quant = sc.nodesQ != nullptr, xcd = scheme == kSchemeXcdSlices;
-  if (wide && scheme == kSchemeRefill) kShadowWide<COUNT><<<grid, kTraceBlock, 0, s>>>(sc, w);
-  else if (quant && xcd) kShadow<COUNT, 2, true><<<grid, kTraceBlock, 0, s>>>(sc, w);
-  else if (quant) kShadow<COUNT, 2, false><<<grid, kTraceBlock, 0, s>>>(sc, w);
-  else if (wide && xcd) kShadow<COUNT, 1, true><<<grid, kTraceBlock, 0, s>>>(sc, w);
-  else if (wide) kShadow<COUNT, 1, false><<<grid, kTraceBlock, 0, s>>>(sc, w);
-  else if (xcd) kShadow<COUNT, 0, true><<<grid, kTraceBlock, 0, s>>>(sc, w);
-  else kShadow<COUNT, 0, false><<<grid, kTraceBlock, 0, s>>>(sc, w);
+  if (wide && scheme == kSchemeRefill) kShadowWide<COUNT><<<grid, kTraceBlock, 0, s>>>(sc, w, cur);
+  else if (quant && xcd) kShadow<COUNT, 2, true><<<grid, kTraceBlock, 0, s>>>(sc, w, cur);
+  else if (quant) kShadow<COUNT, 2, false><<<grid, kTraceBlock, 0, s>>>(sc, w, cur);
+  else if (wide && xcd) kShadow<COUNT, 1, true><<<grid, kTraceBlock, 0, s>>>(sc, w, cur);
+  else if (wide) kShadow<COUNT, 1, false><<<grid, kTraceBlock, 0, s>>>(sc, w, cur);
+  else if (xcd) kShadow<COUNT, 0, true><<<grid, kTraceBlock, 0, s>>>(sc, w, cur);
+  else kShadow<COUNT, 0, false><<<grid, kTraceBlock, 0, s>>>(sc, w, cur);
 }
-void launchShadow(const SceneView& sc, const Wavefront& w, uint32_t scheme, uint32_t grid, bool count,
+void launchShadow(const SceneView& sc, const Wavefront& w, int cur, uint32_t scheme, uint32_t grid, bool count,
                   hipStream_t s) {
   if (sc.twoLevel) {
-    if (count) kShadow2L<true><<<grid, kTraceBlock, 0, s>>>(sc, w);
-    else kShadow2L<false><<<grid, kTraceBlock, 0, s>>>(sc, w);
+    if (count) kShadow2L<true><<<grid, kTraceBlock, 0, s>>>(sc, w, cur);
+    else kShadow2L<false><<<grid, kTraceBlock, 0, s>>>(sc, w, cur);
     return;
   }
-  if (count) shadowFor<true>(sc, w, scheme, grid, s);
-  else shadowFor<false>(sc, w, scheme, grid, s);
+  if (count) shadowFor<true>(sc, w, cur, scheme, grid, s);
+  else shadowFor<false>(sc, w, cur, scheme, grid, s);
 }
 void launchAccumulate(const BatchDesc& b, const Wavefront& w, hipStream_t s) {
   kAccumulate<<<(b.nAcc + 63) / 64, 64, 0, s>>>(b, w);
 }
 void launchSkyPrepare(DevSky* sky, hipStream_t s) { kSkyPrepare<<<1, 64, 0, s>>>(sky); }
 
-void launchResetCounters(const Wavefront& w, int cur, hipStream_t s) { kResetCounters<true, true><<<1, 64, 0, s>>>(w, cur); }
-void launchResetShade(const Wavefront& w, int cur, hipStream_t s) { kResetCounters<false, true><<<1, 64, 0, s>>>(w, cur); }
-void launchResetExtend(const Wavefront& w, hipStream_t s) { kResetCounters<true, false><<<1, 64, 0, s>>>(w, 0); }
+void launchResetCounters(const Wavefront& w, hipStream_t s) { kResetCounters<<<1, 64, 0, s>>>(w); }
 bool canFuseTrace(const SceneView& sc, uint32_t scheme) {
   return sc.twoLevel || (scheme == kSchemeXcdSlices && sc.nodes4 != nullptr && sc.nodesQ == nullptr);
 }
