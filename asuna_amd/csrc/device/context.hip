@@ -554,8 +554,8 @@ static int renderCommon(ash_ctx* c, uint32_t nShots, const ShotParams* hostShots
   }
   int rc = ensureWavefront(c, cap);
   if (rc) return rc;
-  // no more blocks than give every extension and every shadow ray of the batch a lane (whole sets of XCDs)
-  const uint64_t need = (2 * ((uint64_t(cap) + kTraceBlock - 1) / kTraceBlock) + kXcds - 1) / kXcds * kXcds;
+  // no more blocks than give every 4 rays of the batch a wave (whole sets of XCDs)
+  const uint64_t need = (16 * ((uint64_t(cap) + kTraceBlock - 1) / kTraceBlock) + kXcds - 1) / kXcds * kXcds;
   uint32_t grid = uint32_t(std::min<uint64_t>(uint64_t(std::max(1, c->numCU)) * bpc, need));
   rc = ensureSpill(c, grid);
   if (rc) return rc;

@@ -653,40 +653,54 @@ __device__ __forceinline__ void initStack(Stack& st, int* lds, float* ldsT, cons
 // pixel-ordered queue instead of rays from the whole image.
 //
 // The fetch counters are device-scope atomics, resolved beyond the XCD's L2
-// one at a time, so waves that cannot get rays stay away from them: wave j
-// of an XCD takes no part when the first fetches of the waves before it
-// cover the slice (surplus).  With every wave of the 2048-block grid adding
-// to all eight counters, a launch with next to no rays lasted 124 us and a
-// fused one 156 us: a 96 x 64 render of the box at 1 spp 1530 -> 530 us;
-// launches with rays for every wave are unchanged (5.2 M triangles, 1080p,
-// 16 spp: 30.4 ms).  Reading a counter before adding to it when a wave goes
-// over to a further slice made that frame slower (33 ms): waves then help
-// other XCDs sooner and share their L2 less.
+// one at a time (about 1 us each when they do not queue).  With every wave of
+// the 2048-block grid adding to all eight, a launch with next to no rays lasted
+// 124 us and a fused one 156 us.  So
+//  - a queue of at most 4 rays per wave of the grid is handed out without them
+//    (fixed): wave j of the XCD takes entries 16 j .. (64 j .. where a wave walks
+//    a packet) of its own slice and no others, in sparse waves that diverge
+//    less;
+//  - in longer ones wave j of an XCD stays away when the first fetches of the
+//    waves before it cover the slice (surplus).
+// A 96 x 64 render of the box at 1 spp: 1530 us with neither, 500 us with the
+// second, 430 us with both; renders with rays for every wave are
+// unchanged.  Fixed fetches up to 64 rays per wave of the grid, without refill
+// and help for other slices, made renders of 2 M paths slower (256 instances, 4
+// spp: 7.04 -> 7.73 ms; up to 16: 7.11).  Reading a counter before adding to it when a wave goes over to a
+// further slice made a 5.2 M triangle frame slower (30.4 -> 33 ms): waves then
+// help other XCDs sooner and share their L2 less.
 struct ChunkFetch {
   uint32_t* ctr;  // first fetch counter (queue order) or first slice counter (XCD)
   uint32_t count;
   uint32_t slice, home, k;
   uint32_t lo, hi;
-  bool surplus;  // the XCD's earlier waves cover the slice with their first fetches
+  bool fixed;     // one fetch at `mine`, without counters
+  bool surplus;   // no rays for this wave
+  uint32_t mine;
   __device__ __forceinline__ void slicesFor(uint32_t s) {
     lo = s * slice;
     hi = lo < count ? min(count, lo + slice) : lo;
   }
 };
-// CH: queue entries of a wave's first fetch.
-template <bool XCD, uint32_t CH = 64>
+constexpr uint32_t kFixedLanes = 16, kFixedPerWave = 4;
+// LANES: entries of a fixed fetch; CH: of a wave's first fetch otherwise.
+template <bool XCD, uint32_t LANES, uint32_t CH = 64>
 __device__ __forceinline__ void chunkInit(ChunkFetch& f, uint32_t* ctr, uint32_t count) {
   f.ctr = ctr;
   f.count = count;
   f.k = 0;
-  f.surplus = false;
+  f.fixed = f.surplus = false;
+  f.mine = 0;
   if (XCD) {
     f.slice = (count + kXcds - 1) / kXcds;
     f.home = blockIdx.x % kXcds;
     f.slicesFor(f.home);
-    // slices differ in length only at the queue's end, so the rule looks at the longest; wave 0 stays while there are rays
-    const uint32_t j = (blockIdx.x / kXcds) * (kTraceBlock / 64) + (threadIdx.x >> 6);
-    f.surplus = uint64_t(j) * CH >= f.slice;
+    // the rules look at the longest slice and at the grid's whole sets of kXcds blocks, whose waves every home has
+    const uint32_t waves = gridDim.x / kXcds * (kTraceBlock / 64);
+    const uint32_t j = blockIdx.x / kXcds * (kTraceBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    f.fixed = f.slice <= waves * kFixedPerWave;
+    f.mine = f.lo + j * LANES;
+    f.surplus = f.fixed ? f.mine >= f.hi : uint64_t(j) * CH >= f.slice;
   } else {
     f.slice = count;
     f.home = 0;
@@ -699,6 +713,11 @@ __device__ __forceinline__ void chunkInit(ChunkFetch& f, uint32_t* ctr, uint32_t
 template <bool XCD, uint32_t CH = 64>
 __device__ __forceinline__ bool chunkNext(ChunkFetch& f, int lane, uint32_t& start) {
   if (f.surplus) return false;
+  if (XCD && f.fixed) {  // one packet of 64
+    start = f.mine;
+    f.surplus = true;
+    return true;
+  }
   for (;;) {
     uint32_t s = XCD ? (f.home + f.k) % kXcds : 0u;
     const uint32_t len = f.hi - f.lo;
@@ -726,7 +745,7 @@ __global__ __launch_bounds__(kTraceBlock) void kExtend(SceneView sc, Wavefront w
   int lane = __lane_id();
   uint32_t nNodes = 0, nTris = 0;
   ChunkFetch f;
-  chunkInit<XCD>(f, XCD ? &w.ctr[kXcdCtr] : &w.ctr[3], count);
+  chunkInit<XCD, 64>(f, XCD ? &w.ctr[kXcdCtr] : &w.ctr[3], count);
   uint32_t start;
   while (chunkNext<XCD>(f, lane, start)) {
     uint32_t i = start + uint32_t(lane);
@@ -832,6 +851,11 @@ __device__ __forceinline__ bool fetchIdle(ChunkFetch& f, bool idle, int lane, bo
   const uint64_t m = __ballot(idle);
   const uint32_t n = uint32_t(__popcll(m));
   if (n == 0 || drained) return false;
+  if (f.fixed) {  // the wave's one fetch: every lane is idle
+    drained = true;
+    idx = f.mine + uint32_t(lane);
+    return uint32_t(lane) < kFixedLanes && idx < f.hi;
+  }
   const uint32_t rank = uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
   for (;;) {
     const uint32_t sl = (f.home + f.k) % kXcds;
@@ -863,7 +887,7 @@ __device__ __forceinline__ void extendDynLoop(const SceneView& sc, const Wavefro
   const uint32_t count = w.ctr[cur];
   const float4 *qo = w.rayO[cur], *qd = w.rayD[cur];
   ChunkFetch f;
-  chunkInit<true>(f, &w.ctr[kXcdCtr], count);
+  chunkInit<true, kFixedLanes>(f, &w.ctr[kXcdCtr], count);
   bool active = false, drained = f.surplus;
   uint32_t slot = 0;
   TRay r;
@@ -1168,10 +1192,11 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(8, 
   const float4 *qo = w.rayO[cur], *qd = w.rayD[cur];
   uint32_t nN = 0, nT = 0;
   ChunkFetch f;
-  chunkInit<true, FETCH>(f, &w.ctr[kXcdCtr], count);
+  chunkInit<true, 64, FETCH>(f, &w.ctr[kXcdCtr], count);
+  const uint32_t fetch = f.fixed ? 64 : FETCH;
   uint32_t start;
   while (chunkNext<true, FETCH>(f, lane, start)) {
-   for (uint32_t sub = start; sub < start + FETCH && sub < f.hi; sub += 64) {
+   for (uint32_t sub = start; sub < start + fetch && sub < f.hi; sub += 64) {
     const uint32_t i = sub + uint32_t(lane);
     const bool valid = i < f.hi;  // lane 0 always holds a ray
     TRay r;
@@ -1231,7 +1256,7 @@ __device__ __forceinline__ void shadowLoop(const SceneView& sc, const Wavefront&
                                            uint32_t& nNodes, uint32_t& nTris) {
   const uint32_t count = *shadowCtr(w, cur);
   ChunkFetch f;
-  chunkInit<XCD>(f, XCD ? &w.ctr[kXcdCtr + kXcds * 32] : &w.ctr[4], count);
+  chunkInit<XCD, 64>(f, XCD ? &w.ctr[kXcdCtr + kXcds * 32] : &w.ctr[4], count);
   uint32_t start;
   while (chunkNext<XCD>(f, lane, start)) {
     uint32_t i = start + uint32_t(lane);
@@ -1321,7 +1346,7 @@ template <bool COUNT, int REFILL>
 __device__ __forceinline__ void shadowDynLoop(const SceneView& sc, const Wavefront& w, int cur, Stack& st, int lane,
                                               uint32_t& nNodes, uint32_t& nTris) {
   ChunkFetch f;
-  chunkInit<true>(f, &w.ctr[kXcdCtr + kXcds * 32], *shadowCtr(w, cur));
+  chunkInit<true, kFixedLanes>(f, &w.ctr[kXcdCtr + kXcds * 32], *shadowCtr(w, cur));
   bool active = false, drained = f.surplus;
   int pid = -1;
   uint32_t slot = 0;
@@ -1487,7 +1512,7 @@ __device__ __forceinline__ void extend2LLoop(const SceneView& sc, const Wavefron
   const uint32_t count = w.ctr[cur];
   const float4 *qo = w.rayO[cur], *qd = w.rayD[cur];
   ChunkFetch f;
-  chunkInit<true>(f, &w.ctr[kXcdCtr], count);
+  chunkInit<true, kFixedLanes>(f, &w.ctr[kXcdCtr], count);
   bool active = false, drained = f.surplus;
   uint32_t slot = 0;
   TRay rw, ro;
@@ -1595,7 +1620,7 @@ __device__ __forceinline__ void shadow2LLoop(const SceneView& sc, const Wavefron
                                              uint32_t& nNodes, uint32_t& nTris) {
   const uint32_t count = *shadowCtr(w, cur);
   ChunkFetch f;
-  chunkInit<true>(f, &w.ctr[kXcdCtr + kXcds * 32], count);
+  chunkInit<true, kFixedLanes>(f, &w.ctr[kXcdCtr + kXcds * 32], count);
   bool active = false, drained = f.surplus;
   uint32_t slot = 0;
   int pid = 0;
@@ -1665,7 +1690,7 @@ __global__ __launch_bounds__(kTraceBlock) void kShadow2L(SceneView sc, Wavefront
 }
 // COUNT: as kTraceDyn (totals and the fused launches' own counters).
 template <bool COUNT>
-__global__ __launch_bounds__(kTraceBlock) void kTrace2L(SceneView sc, Wavefront w, int cur) {
+__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(5))) void kTrace2L(SceneView sc, Wavefront w, int cur) {
   __shared__ int lds[kStackLds * kTraceBlock];
   __shared__ float ldsT[kStackLds * kTraceBlock];
   if (COUNT && blockIdx.x == 0 && threadIdx.x == 0) {
