@@ -2328,7 +2328,9 @@ struct PathCtx {
   const SceneView* sc;
   const ShotParams* sp;
   uint32_t seed;
-  f3 ro, rd, T, L;
+  f3 ro, rd, T;
+  f3 add;    // radiance this hit adds to the path's (lit)
+  bool lit;
   float bpdf;
   uint32_t bflags, depth;
   bool stop;
@@ -2422,7 +2424,8 @@ __device__ void hitLight(PathCtx& c, int lightId, f3 hitPos) {
     float lightPdf = distSquare / (light.area * fabsf(proj) + kEps);
     mis = powerHeuristic(c.bpdf, lightPdf);
   }
-  c.L = c.L + c.T * ld3(light.radiance) * mis;
+  c.add = c.T * ld3(light.radiance) * mis;
+  c.lit = true;
 }
 
 __device__ __forceinline__ void nextRay(PathCtx& c, f3 pos, f3 offN, f3 d, f3 weightOverPdf, float pdf,
@@ -3229,7 +3232,6 @@ __device__ __forceinline__ void shadeOne(const SceneView& sc, const BatchDesc& b
   c.shadow = false;
   c.fromDielectric = false;
   uint4 info = make_uint4(0u, 0u, 0u, 0u);
-  float4 rad = make_float4(0.f, 0.f, 0.f, 0.f);
   bool cont = false;
   if (active) {
     const float4 d4 = w.rayD[cur][slot];
@@ -3242,7 +3244,6 @@ __device__ __forceinline__ void shadeOne(const SceneView& sc, const BatchDesc& b
     // surface, which keeps its throughput) has throughput (1, 1, 1) and pdf
     // 0; raygen stores no record for it
     const float4 thr = (info.y & 0xffffu) == 1u ? make_float4(1.f, 1.f, 1.f, 0.f) : w.thr[cur][slot];
-    rad = w.rad[pid];
     c.sc = &sc;
     c.sp = &sp;
     c.seed = info.x;
@@ -3251,7 +3252,8 @@ __device__ __forceinline__ void shadeOne(const SceneView& sc, const BatchDesc& b
     c.rd = xyz(d4);  // the origin is read only for light hits (MIS distance)
     c.T = xyz(thr);
     c.bpdf = thr.w;
-    c.L = xyz(rad);
+    c.lit = false;
+    c.add = mk1(0.f);
     c.stop = false;
     c.shadow = false;
     c.fromDielectric = false;
@@ -3272,7 +3274,8 @@ __device__ __forceinline__ void shadeOne(const SceneView& sc, const BatchDesc& b
                         : ld3(pc.bgColor);
       float mis = 1.0f;
       if (c.depth != 1 && isNonSpecular(c.bflags)) mis = powerHeuristic(c.bpdf, envPdf);
-      c.L = c.L + c.T * env * mis;
+      c.add = c.T * env * mis;
+      c.lit = true;
     } else {
       // Surfaces draw their light sample after a fixed number of draws: one
       // (the opacity draw) for pbr, disney and kang18, none for the others.
@@ -3319,7 +3322,7 @@ __device__ __forceinline__ void shadeOne(const SceneView& sc, const BatchDesc& b
           c.stop = true;
           f3 e = ld3(m.radiance);
           if (m.radianceTextureId >= 0) e = ld3(m.radianceFactor) * xyz(tex2D(sc.textures[m.radianceTextureId], h.uvx, h.uvy));
-          if (pc.ignoreEmissive == 0) c.L = c.L + e * c.T;
+          if (pc.ignoreEmissive == 0) c.add = e * c.T, c.lit = true;
         } else if (type < MaterialTypeNum) {
           shadeSurface<GROUP2>(c, h, m, pix, aov);
         } else {
@@ -3354,7 +3357,12 @@ __device__ __forceinline__ void shadeOne(const SceneView& sc, const BatchDesc& b
     w.thr[1 - cur][ni] = f4(c.T, c.bpdf);
     w.info[1 - cur][ni] = make_uint4(c.seed, c.depth | (c.bflags << 16), info.z, info.w);
   }
-  if (active) w.rad[pid] = f4(c.L, rad.w);
+  // Radiance is read and written only where the hit adds some (misses, lights, emissive surfaces): its records lie at
+  // path ids, so after the first bounce each is a line of its own.
+  if (active && c.lit) {
+    const float4 rad = w.rad[pid];
+    w.rad[pid] = f4(xyz(rad) + c.add, rad.w);
+  }
 }
 
 // Shades the queue; paths whose surface belongs to the second plugin group
