@@ -8,9 +8,10 @@
 //   4. binary radix tree, Karras 2012 "Maximizing Parallelism in the
 //      Construction of BVHs, Octrees, and k-d Trees" (equal keys ordered by
 //      index)
-//   5. bottom-up refit with arrival counters: boxes, triangle counts and the
-//      SAH cost; a subtree with <= leafMax triangles whose leaf cost does not
-//      exceed its split cost is collapsed into one leaf
+//      or, by default, locally-ordered clustering over the sorted keys (below)
+//   5. boxes, triangle counts and the SAH cost bottom-up (level by level; the
+//      clustering makes them as it merges); a subtree with <= leafMax triangles
+//      whose leaf cost does not exceed its split cost is collapsed into one leaf
 //   6. compaction of the surviving internal nodes (prefix sum) and emission
 //      of 64-byte BVH2 nodes that hold both child boxes; triangles are
 //      reordered into leaf order.
@@ -37,6 +38,23 @@ constexpr float kCostTri = 1.0f;
       return ASH_E_HIP;                                                            \
     }                                                                              \
   } while (0)
+
+__device__ __forceinline__ uint32_t blockExclusive(uint32_t v, uint32_t* sh, uint32_t& total) {
+  // exclusive scan of one value per thread over a 256-thread block
+  const uint32_t t = threadIdx.x, lane = t & 63, w = t >> 6;
+  uint32_t x = v;
+  for (uint32_t d = 1; d < 64; d <<= 1) {
+    const uint32_t y = __shfl_up(x, d);
+    if (lane >= d) x += y;
+  }
+  if (lane == 63) sh[w] = x;
+  __syncthreads();
+  uint32_t base = 0;
+  for (uint32_t k = 0; k < w; ++k) base += sh[k];
+  total = sh[0] + sh[1] + sh[2] + sh[3];
+  __syncthreads();
+  return base + x - v;
+}
 
 __device__ __forceinline__ float3 xform(const float* m, float4 p) {
   // ((m0*x + m1*y) + m2*z) + m3 per row
@@ -94,6 +112,30 @@ __global__ void kCentroidBounds(const float4* boxLo, const float4* boxHi, uint32
   }
 }
 
+// The partial bounds of kCentroidBounds, reduced into partLo[0] / partHi[0] by
+// one block (nPart <= 2 kBlock).  When every thread of kMorton read all 512
+// partials itself, keys of 5.2 M triangles took 1.38 ms.
+__global__ __launch_bounds__(kBlock) void kBoundsOfParts(float4* partLo, float4* partHi, uint32_t nPart) {
+  __shared__ float4 sl[kBlock], sh[kBlock];
+  const uint32_t t = threadIdx.x;
+  float4 l = make_float4(FLT_MAX, FLT_MAX, FLT_MAX, 0.f), h = make_float4(-FLT_MAX, -FLT_MAX, -FLT_MAX, 0.f);
+  auto add = [&](float4 a, float4 b) {
+    l = make_float4(fminf(l.x, a.x), fminf(l.y, a.y), fminf(l.z, a.z), 0.f);
+    h = make_float4(fmaxf(h.x, b.x), fmaxf(h.y, b.y), fmaxf(h.z, b.z), 0.f);
+  };
+  for (uint32_t k = t; k < nPart; k += kBlock) add(partLo[k], partHi[k]);
+  sl[t] = l, sh[t] = h;
+  __syncthreads();
+  for (uint32_t s = kBlock / 2; s > 0; s >>= 1) {
+    if (t < s) {
+      add(sl[t + s], sh[t + s]);
+      sl[t] = l, sh[t] = h;
+    }
+    __syncthreads();
+  }
+  if (t == 0) partLo[0] = l, partHi[0] = h;
+}
+
 __device__ __forceinline__ uint64_t spread21(uint32_t v) {
   uint64_t x = v & 0x1fffffu;
   x = (x | x << 32) & 0x1f00000000ffffull;
@@ -105,15 +147,10 @@ __device__ __forceinline__ uint64_t spread21(uint32_t v) {
 }
 
 __global__ void kMorton(const float4* boxLo, const float4* boxHi, uint32_t n, const float4* partLo,
-                        const float4* partHi, uint32_t nPart, uint64_t* keys, uint32_t* ids) {
+                        const float4* partHi, uint64_t* keys, uint32_t* ids) {
   uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  float l[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, h[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-  for (uint32_t p = 0; p < nPart; ++p) {
-    float4 a = partLo[p], b = partHi[p];
-    l[0] = fminf(l[0], a.x), l[1] = fminf(l[1], a.y), l[2] = fminf(l[2], a.z);
-    h[0] = fmaxf(h[0], b.x), h[1] = fmaxf(h[1], b.y), h[2] = fmaxf(h[2], b.z);
-  }
+  const float l[3] = {partLo[0].x, partLo[0].y, partLo[0].z}, h[3] = {partHi[0].x, partHi[0].y, partHi[0].z};
   float4 a = boxLo[i], b = boxHi[i];
   float c[3] = {0.5f * (a.x + b.x), 0.5f * (a.y + b.y), 0.5f * (a.z + b.z)};
   uint64_t key = 0;
@@ -181,94 +218,238 @@ __device__ __forceinline__ float halfArea(float4 lo, float4 hi) {
 // smaller index, so the globally best pair is always mutual); mutual pairs
 // merge into a new internal node; the survivors are compacted in order.
 // Internal ids are handed out from n - 2 down, so the root is node 0.
+//
+// A cluster carries its SAH cost and triangle count in the unused lanes of its
+// box, so a merge also makes what the bottom-up refit would: the node's box,
+// cost and leaf-collapse decision (its children are complete when it is made).
+// A round is three launches and reads the cluster count from the device: the
+// host only looks at it every kPlocRounds rounds, with grids for the last
+// count it saw, and the rounds from kPlocTail clusters down run in one block.
+// A build of 1 M triangles with its first hits took 19.0 ms with one host round
+// trip and six launches per round, a level walk, one refit launch per level and
+// its temporaries allocated one by one; it takes 5.1 (2.4 in kernels).
 constexpr int kPlocRadius = 16;
+constexpr uint32_t kPlocTail = 1024;
+constexpr int kPlocRounds = 4;
+
+struct PlocTree {
+  int *left, *right, *parent, *leafParent;
+  uint32_t* nodeCnt;
+  float4 *nodeLo, *nodeHi;
+  float* cost;
+  uint8_t* collapsed;
+  uint32_t n, leafMax, quality;
+};
 
 __global__ void kPlocInit(uint32_t n, const uint32_t* sortedIds, const float4* boxLo, const float4* boxHi, int* cNode,
-                          float4* cLo, float4* cHi) {
+                          float4* cLo, float4* cHi, uint32_t* count, int* parent) {
   uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) count[0] = n, parent[0] = -1;
   if (i >= n) return;
   uint32_t t = sortedIds[i];
+  float4 lo = boxLo[t], hi = boxHi[t];
+  lo.w = kCostTri * halfArea(lo, hi);
+  hi.w = __uint_as_float(1u);
   cNode[i] = ~int(i);
-  cLo[i] = boxLo[t];
-  cHi[i] = boxHi[t];
+  cLo[i] = lo;
+  cHi[i] = hi;
 }
 
-__global__ __launch_bounds__(kBlock) void kPlocNearest(uint32_t m, const float4* cLo, const float4* cHi, int* nn) {
-  __shared__ float4 sl[kBlock + 2 * kPlocRadius], sh[kBlock + 2 * kPlocRadius];
-  const int base = int(blockIdx.x * blockDim.x) - kPlocRadius;
-  for (int k = int(threadIdx.x); k < kBlock + 2 * kPlocRadius; k += kBlock) {
-    int g = base + k;
-    if (g >= 0 && g < int(m)) {
-      sl[k] = cLo[g];
-      sh[k] = cHi[g];
-    }
-  }
-  __syncthreads();
-  const int i = int(blockIdx.x * blockDim.x + threadIdx.x);
-  if (i >= int(m)) return;
-  const int li = i - base;
-  const float4 a = sl[li], b = sh[li];
+// Merges clusters (c0, a, b) and (c1, c, d) into internal node id; returns
+// its box, cost and count in lo / hi.
+__device__ __forceinline__ void plocMerge(const PlocTree& T, int id, int c0, float4 a, float4 b, int c1, float4 c, float4 d,
+                                          float4& lo, float4& hi) {
+  const uint32_t cnt = __float_as_uint(b.w) + __float_as_uint(d.w);
+  lo = make_float4(fminf(a.x, c.x), fminf(a.y, c.y), fminf(a.z, c.z), 0.f);
+  hi = make_float4(fmaxf(b.x, d.x), fmaxf(b.y, d.y), fmaxf(b.z, d.z), 0.f);
+  const float area = halfArea(lo, hi), childCost = a.w + c.w;
+  const float splitCost = kCostNode * area + childCost, leafCost = kCostTri * area * float(cnt);
+  const bool col = T.quality > 0 && cnt <= T.leafMax && leafCost <= splitCost;
+  T.left[id] = c0;
+  T.right[id] = c1;
+  (c0 >= 0 ? T.parent[c0] : T.leafParent[~c0]) = id;
+  (c1 >= 0 ? T.parent[c1] : T.leafParent[~c1]) = id;
+  T.nodeCnt[id] = cnt;
+  T.nodeLo[id] = lo;
+  T.nodeHi[id] = hi;
+  T.cost[id] = col ? leafCost : splitCost;
+  T.collapsed[id] = col ? 1 : 0;
+  lo.w = col ? leafCost : splitCost;
+  hi.w = __uint_as_float(cnt);
+}
+
+// The best partner of cluster g among [j0, j1] (boxes at sl / sh, index j - base).
+__device__ __forceinline__ int plocNearest(const float4* sl, const float4* sh, int g, int j0, int j1, int base) {
+  const float4 a = sl[g - base], b = sh[g - base];
   float best = FLT_MAX;
   int bj = -1;
-  const int j0 = max(0, i - kPlocRadius), j1 = min(int(m) - 1, i + kPlocRadius);
   for (int j = j0; j <= j1; ++j) {
-    if (j == i) continue;
+    if (j == g) continue;
     const float4 c = sl[j - base], d = sh[j - base];
-    float4 lo = make_float4(fminf(a.x, c.x), fminf(a.y, c.y), fminf(a.z, c.z), 0.f);
-    float4 hi = make_float4(fmaxf(b.x, d.x), fmaxf(b.y, d.y), fmaxf(b.z, d.z), 0.f);
-    float cost = halfArea(lo, hi);
+    const float4 lo = make_float4(fminf(a.x, c.x), fminf(a.y, c.y), fminf(a.z, c.z), 0.f);
+    const float4 hi = make_float4(fmaxf(b.x, d.x), fmaxf(b.y, d.y), fmaxf(b.z, d.z), 0.f);
+    const float cost = halfArea(lo, hi);
     if (cost < best) best = cost, bj = j;  // ascending j: ties keep the smaller index
   }
-  nn[i] = bj;
+  return bj;
 }
 
-__global__ void kPlocMerge(uint32_t m, uint32_t n, const int* nn, const int* cNode, const float4* cLo, const float4* cHi,
-                           int* oNode, float4* oLo, float4* oHi, uint32_t* valid, int* left, int* right, int* parent,
-                           int* leafParent, uint32_t* nodeCnt, unsigned* idCounter) {
-  int i = int(blockIdx.x * blockDim.x + threadIdx.x);
-  if (i >= int(m)) return;
-  int j = nn[i];
-  bool mutual = j >= 0 && nn[j] == i;
-  if (mutual && i > j) {  // absorbed by its partner
-    valid[i] = 0;
-    return;
+// Ranks of a flag over a block of kBlock threads (exclusive) and its total.
+__device__ __forceinline__ uint32_t blockRank(bool f, uint32_t* sh, uint32_t& total) {
+  const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const uint64_t m = __ballot(f);
+  if (lane == 0) sh[w] = uint32_t(__popcll(m));
+  __syncthreads();
+  uint32_t base = 0;
+  total = 0;
+  for (uint32_t k = 0; k < blockDim.x >> 6; ++k) {
+    base += k < w ? sh[k] : 0u;
+    total += sh[k];
   }
-  valid[i] = 1;
-  if (!mutual) {
-    oNode[i] = cNode[i];
-    oLo[i] = cLo[i];
-    oHi[i] = cHi[i];
-    return;
-  }
-  int id = int(n - 2) - int(atomicAdd(idCounter, 1u));
-  int c0 = cNode[i], c1 = cNode[j];
-  left[id] = c0;
-  right[id] = c1;
-  uint32_t cnt = 0;
-  for (int c : {c0, c1}) {
-    if (c >= 0) {
-      parent[c] = id;
-      cnt += nodeCnt[c];
-    } else {
-      leafParent[~c] = id;
-      cnt += 1u;
-    }
-  }
-  nodeCnt[id] = cnt;
-  float4 a = cLo[i], b = cHi[i], c = cLo[j], d = cHi[j];
-  oNode[i] = id;
-  oLo[i] = make_float4(fminf(a.x, c.x), fminf(a.y, c.y), fminf(a.z, c.z), 0.f);
-  oHi[i] = make_float4(fmaxf(b.x, d.x), fmaxf(b.y, d.y), fmaxf(b.z, d.z), 0.f);
+  __syncthreads();
+  return base + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
 }
 
-__global__ void kPlocCompact(uint32_t m, const uint32_t* valid, const uint32_t* offs, const int* oNode,
-                             const float4* oLo, const float4* oHi, int* cNode, float4* cLo, float4* cHi) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= m || !valid[i]) return;
-  uint32_t o = offs[i];
+// One round's neighbour search and merges.  A block holds its 256 clusters
+// and two radii on either side, so it also knows its candidates' own best
+// partners; survivors per block go to tileSums for the compaction.
+__global__ __launch_bounds__(kBlock) void kPlocStep(PlocTree T, const uint32_t* count, const int* cNode, const float4* cLo,
+                                                    const float4* cHi, int* oNode, float4* oLo, float4* oHi,
+                                                    uint8_t* valid, uint32_t* tileSums, unsigned* idCounter) {
+  constexpr int kHalo = 2 * kPlocRadius, kBoxes = kBlock + 2 * kHalo, kNear = kBlock + 2 * kPlocRadius;
+  __shared__ float4 sl[kBoxes], sh[kBoxes];
+  __shared__ int sn[kNear];
+  __shared__ uint32_t sw[kBlock / 64];
+  __shared__ unsigned sId;
+  const int m = int(*count), first = int(blockIdx.x * kBlock), base = first - kHalo;
+  if (first >= m) return;
+  for (int k = int(threadIdx.x); k < kBoxes; k += kBlock) {
+    const int g = base + k;
+    if (g >= 0 && g < m) sl[k] = cLo[g], sh[k] = cHi[g];
+  }
+  __syncthreads();
+  for (int k = int(threadIdx.x); k < kNear; k += kBlock) {
+    const int g = first - kPlocRadius + k;
+    if (g >= 0 && g < m) sn[k] = plocNearest(sl, sh, g, max(0, g - kPlocRadius), min(m - 1, g + kPlocRadius), base);
+  }
+  __syncthreads();
+  const int i = first + int(threadIdx.x);
+  int j = -1;
+  bool mutual = false;
+  if (i < m) {
+    j = sn[i - first + kPlocRadius];
+    mutual = j >= 0 && sn[j - first + kPlocRadius] == i;
+  }
+  const bool merges = mutual && i < j, stays = i < m && !(mutual && i > j);  // i > j: absorbed by its partner
+  uint32_t nMerges, nStays;
+  const uint32_t rank = blockRank(merges, sw, nMerges);
+  (void)blockRank(stays, sw, nStays);
+  if (threadIdx.x == 0) {
+    tileSums[blockIdx.x] = nStays;
+    sId = nMerges ? atomicAdd(idCounter, nMerges) : 0u;
+  }
+  __syncthreads();
+  if (i >= m) return;
+  valid[i] = stays ? 1 : 0;
+  if (!stays) return;
+  float4 lo = sl[i - base], hi = sh[i - base];
+  int node = cNode[i];
+  if (merges) {
+    const int id = int(T.n - 2) - int(sId + rank);
+    plocMerge(T, id, node, lo, hi, cNode[j], sl[j - base], sh[j - base], lo, hi);
+    node = id;
+  }
+  oNode[i] = node;
+  oLo[i] = lo;
+  oHi[i] = hi;
+}
+
+// Exclusive scan of a round's tile sums by one block; the next count.
+__global__ __launch_bounds__(1024) void kPlocScan(const uint32_t* count, uint32_t* tileSums, uint32_t* next) {
+  __shared__ uint32_t sh[16];
+  const uint32_t nt = (*count + kBlock - 1) / kBlock, per = (nt + 1023) / 1024, t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const uint32_t b0 = min(nt, t * per), b1 = min(nt, b0 + per);
+  uint32_t s = 0;
+  for (uint32_t k = b0; k < b1; ++k) s += tileSums[k];
+  uint32_t x = s;
+  for (uint32_t d = 1; d < 64; d <<= 1) {
+    const uint32_t y = __shfl_up(x, d);
+    if (lane >= d) x += y;
+  }
+  if (lane == 63) sh[w] = x;
+  __syncthreads();
+  uint32_t run = x - s, total = 0;
+  for (uint32_t k = 0; k < 16; ++k) {
+    run += k < w ? sh[k] : 0u;
+    total += sh[k];
+  }
+  for (uint32_t k = b0; k < b1; ++k) {
+    const uint32_t v = tileSums[k];
+    tileSums[k] = run;
+    run += v;
+  }
+  if (t == 0) *next = total;
+}
+
+__global__ __launch_bounds__(kBlock) void kPlocCompact(const uint32_t* count, const uint8_t* valid, const uint32_t* tileOff,
+                                                       const int* oNode, const float4* oLo, const float4* oHi, int* cNode,
+                                                       float4* cLo, float4* cHi) {
+  __shared__ uint32_t sw[kBlock / 64];
+  const uint32_t m = *count, i = blockIdx.x * kBlock + threadIdx.x;
+  if (blockIdx.x * kBlock >= m) return;
+  const bool stays = i < m && valid[i];
+  uint32_t total;
+  const uint32_t o = blockRank(stays, sw, total) + tileOff[blockIdx.x];
+  if (!stays) return;
   cNode[o] = oNode[i];
   cLo[o] = oLo[i];
   cHi[o] = oHi[i];
+}
+
+// The rounds from at most kPlocTail clusters to one, in one block: a thread
+// per cluster, boxes and partners in LDS.  Ends when a round merges nothing
+// (one cluster, or boxes no cost compares below).
+__global__ __launch_bounds__(kPlocTail) void kPlocTailRounds(PlocTree T, uint32_t* count, const int* cNode, const float4* cLo,
+                                                             const float4* cHi, unsigned* idCounter) {
+  __shared__ float4 sl[kPlocTail], sh[kPlocTail];
+  __shared__ int sNode[kPlocTail], sn[kPlocTail];
+  __shared__ uint32_t sw[kPlocTail / 64];
+  const int i = int(threadIdx.x);
+  int m = int(*count);
+  if (m > int(kPlocTail)) return;  // the host launches this only for such counts
+  unsigned used = *idCounter;
+  if (i < m) sl[i] = cLo[i], sh[i] = cHi[i], sNode[i] = cNode[i];
+  __syncthreads();
+  while (m > 1) {
+    if (i < m) sn[i] = plocNearest(sl, sh, i, max(0, i - kPlocRadius), min(m - 1, i + kPlocRadius), 0);
+    __syncthreads();
+    int j = -1;
+    bool mutual = false;
+    if (i < m) {
+      j = sn[i];
+      mutual = j >= 0 && sn[j] == i;
+    }
+    const bool merges = mutual && i < j, stays = i < m && !(mutual && i > j);
+    uint32_t nMerges, nStays;
+    const uint32_t rank = blockRank(merges, sw, nMerges), at = blockRank(stays, sw, nStays);
+    float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
+    int node = 0;
+    if (stays) {
+      lo = sl[i], hi = sh[i], node = sNode[i];
+      if (merges) {
+        const int id = int(T.n - 2) - int(used + rank);
+        plocMerge(T, id, node, lo, hi, sNode[j], sl[j], sh[j], lo, hi);
+        node = id;
+      }
+    }
+    __syncthreads();
+    if (stays) sl[at] = lo, sh[at] = hi, sNode[at] = node;
+    used += nMerges;
+    m = int(nStays);
+    __syncthreads();
+    if (!nMerges) break;
+  }
+  if (i == 0) *count = uint32_t(m), *idCounter = used;
 }
 
 // Leaves in depth-first order, so each subtree covers one run of positions:
@@ -505,12 +686,20 @@ __device__ __forceinline__ float slotArea(const float* lo, const float* hi) {
   return dx * dy + dy * dz + dz * dx;
 }
 
-__global__ void kCollapse4(const float4* n2, const int2* front, uint32_t nFront, float4* n4, unsigned* n4Count,
-                           int2* next, unsigned* nextCount) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nFront) return;
-  int src = front[i].x, dst = front[i].y;
-  int ref[4];
+__global__ void kCollapseInit(int2* front, unsigned* cnts) {
+  front[0] = make_int2(0, 0);
+  cnts[0] = cnts[1] = 1;
+}
+
+__global__ __launch_bounds__(kBlock) void kCollapse4(const float4* n2, const int2* front, const unsigned* nFront, float4* n4,
+                                                     unsigned* n4Count, int2* next, unsigned* nextCount) {
+  __shared__ uint32_t sw[4];
+  __shared__ unsigned sBase[2];
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x, count = *nFront;
+  if (blockIdx.x * kBlock >= count) return;
+  const bool mine = i < count;
+  const int src = mine ? front[i].x : 0, dst = mine ? front[i].y : 0;
+  int ref[4] = {kEmptyRef, kEmptyRef, kEmptyRef, kEmptyRef};
   float lo[4][3], hi[4][3];
   auto loadChildren = [&](int node, int s0, int s1) {
     float4 a = n2[size_t(node) * 4 + 0], b = n2[size_t(node) * 4 + 1], c = n2[size_t(node) * 4 + 2],
@@ -520,9 +709,12 @@ __global__ void kCollapse4(const float4* n2, const int2* front, uint32_t nFront,
     ref[s0] = __float_as_int(d.x);
     ref[s1] = __float_as_int(d.y);
   };
-  loadChildren(src, 0, 1);
-  int cnt = 2;
-  while (cnt < 4) {
+  int cnt = 0;
+  if (mine) {
+    loadChildren(src, 0, 1);
+    cnt = 2;
+  }
+  while (mine && cnt < 4) {
     int pick = -1;
     float best = -1.f;
     for (int k = 0; k < cnt; ++k) {
@@ -536,8 +728,13 @@ __global__ void kCollapse4(const float4* n2, const int2* front, uint32_t nFront,
   }
   int internal = 0;
   for (int k = 0; k < cnt; ++k) internal += (ref[k] >= 0 && ref[k] != kEmptyRef) ? 1 : 0;
-  unsigned base = internal ? atomicAdd(n4Count, unsigned(internal)) : 0u;
-  unsigned fbase = internal ? atomicAdd(nextCount, unsigned(internal)) : 0u;
+  // ids and frontier places: one atomic per counter and block, ranks within it in thread order
+  uint32_t total;
+  const uint32_t rank = blockExclusive(uint32_t(internal), sw, total);
+  if (threadIdx.x == 0 && total) sBase[0] = atomicAdd(n4Count, total), sBase[1] = atomicAdd(nextCount, total);
+  __syncthreads();
+  if (!mine) return;
+  unsigned base = sBase[0] + rank, fbase = sBase[1] + rank;
   int out[4];
   const float far = 3.0e38f;
   for (int k = 0; k < 4; ++k) {
@@ -655,10 +852,28 @@ __global__ void kQuantize4(const float4* n4, uint32_t numNodes, float4* nq) {
   d[3] = make_float4(rf.z, rf.w, 0.f, 0.f);
 }
 
+// The build's temporaries: parts of one allocation, freed at its end (about 45
+// allocations and frees of their own took more than half of a 1 M triangle
+// build's 19 ms; hipFree waits for the device).
 template <class T> struct DevBuf {
   T* p = nullptr;
-  ~DevBuf() {
-    if (p) (void)hipFree(p);
+};
+struct Arena {
+  char* base = nullptr;
+  size_t size = 0, used = 0;
+  hipError_t status = hipSuccess;  // hipErrorOutOfMemory once a part did not fit
+  ~Arena() {
+    if (base) (void)hipFree(base);
+  }
+  static size_t bytes(size_t n) { return (n + 255) & ~size_t(255); }
+  template <class T> void take(DevBuf<T>& b, size_t count) {
+    const size_t n = bytes(std::max<size_t>(count, 1) * sizeof(T));
+    if (used + n > size) {
+      status = hipErrorOutOfMemory;
+      return;
+    }
+    b.p = reinterpret_cast<T*>(base + used);
+    used += n;
   }
 };
 
@@ -667,22 +882,6 @@ template <class T> struct DevBuf {
 // per-2048-element tile sums, one block scanning the tile sums, then each
 // tile's scan plus its offset.  Work per thread: 8 consecutive elements.
 constexpr uint32_t kScanTile = 2048;
-__device__ __forceinline__ uint32_t blockExclusive(uint32_t v, uint32_t* sh, uint32_t& total) {
-  // exclusive scan of one value per thread over a 256-thread block
-  const uint32_t t = threadIdx.x, lane = t & 63, w = t >> 6;
-  uint32_t x = v;
-  for (uint32_t d = 1; d < 64; d <<= 1) {
-    const uint32_t y = __shfl_up(x, d);
-    if (lane >= d) x += y;
-  }
-  if (lane == 63) sh[w] = x;
-  __syncthreads();
-  uint32_t base = 0;
-  for (uint32_t k = 0; k < w; ++k) base += sh[k];
-  total = sh[0] + sh[1] + sh[2] + sh[3];
-  __syncthreads();
-  return base + x - v;
-}
 __global__ __launch_bounds__(256) void kScanTileSums(const uint32_t* in, uint32_t n, uint32_t* tileSums) {
   __shared__ uint32_t sh[4];
   const uint32_t base = blockIdx.x * kScanTile + threadIdx.x * 8;
@@ -837,27 +1036,30 @@ int buildBvh(const BuildArgs& a, hipStream_t s, BuildResult& r, char* err, size_
   DevBuf<uint8_t> collapsed;
   DevBuf<uint32_t> counts, countOffs, scanScr;
   size_t nn = n ? n : 1;
-  HIPB(hipMalloc(&wtri.p, nn * 3 * sizeof(float4)));
-  HIPB(hipMalloc(&boxLo.p, nn * sizeof(float4)));
-  HIPB(hipMalloc(&boxHi.p, nn * sizeof(float4)));
-  HIPB(hipMalloc(&keys.p, nn * sizeof(uint64_t)));
-  HIPB(hipMalloc(&keys2.p, nn * sizeof(uint64_t)));
-  HIPB(hipMalloc(&ids.p, nn * sizeof(uint32_t)));
-  HIPB(hipMalloc(&ids2.p, nn * sizeof(uint32_t)));
   const uint32_t nPart = 512;
-  HIPB(hipMalloc(&partLo.p, nPart * sizeof(float4)));
-  HIPB(hipMalloc(&partHi.p, nPart * sizeof(float4)));
-  HIPB(hipMalloc(&maxDepth.p, sizeof(unsigned)));
+  const uint32_t nTiles = (n + kSortTile - 1) / kSortTile, nCounts = std::max(1u, kRadix * nTiles);
+  Arena A;
+  {
+    // triangle records, boxes, keys and ids; the tree's nodes; then clusters and leaf order, or the collapse's
+    // frontiers and reference counts, whichever is larger
+    const size_t perTri = 48 + 32 + 16 + 8, perNode = 4 * 4 + 8 + 4 + 32 + 4 + 1 + 8;
+    const size_t ploc = 2 * (4 + 32) + 1 + 4 * 4 + 1, after = 2 * 8 + 2 * 4;
+    A.size = nn * (perTri + perNode + (a.quality == 2 ? std::max(ploc, after) : after)) +
+             sizeof(uint32_t) * (2 * size_t(nCounts) + std::max(scanScratch(nCounts), scanScratch(n))) +
+             2 * nPart * sizeof(float4) + 64 * 256;  // 64 parts, each rounded up to 256 bytes
+    HIPB(hipMalloc(&A.base, A.size));
+  }
+  A.take(wtri, nn * 3), A.take(boxLo, nn), A.take(boxHi, nn), A.take(keys, nn), A.take(keys2, nn), A.take(ids, nn);
+  A.take(ids2, nn), A.take(partLo, nPart), A.take(partHi, nPart), A.take(maxDepth, 1);
+  A.take(counts, nCounts), A.take(countOffs, nCounts), A.take(scanScr, std::max(scanScratch(nCounts), scanScratch(n)));
+  HIPB(A.status);
   HIPB(hipMemsetAsync(maxDepth.p, 0, sizeof(unsigned), s));
   unsigned grid = (n + kBlock - 1) / kBlock;
   if (n) {
     kWorldTris<<<grid, kBlock, 0, s>>>(a, wtri.p, boxLo.p, boxHi.p);
     kCentroidBounds<<<nPart, kBlock, 0, s>>>(boxLo.p, boxHi.p, n, partLo.p, partHi.p);
-    kMorton<<<grid, kBlock, 0, s>>>(boxLo.p, boxHi.p, n, partLo.p, partHi.p, nPart, keys.p, ids.p);
-    const uint32_t nTiles = (n + kSortTile - 1) / kSortTile, nCounts = kRadix * nTiles;
-    HIPB(hipMalloc(&counts.p, size_t(nCounts) * sizeof(uint32_t)));
-    HIPB(hipMalloc(&countOffs.p, size_t(nCounts) * sizeof(uint32_t)));
-    HIPB(hipMalloc(&scanScr.p, std::max(scanScratch(nCounts), scanScratch(n)) * sizeof(uint32_t)));
+    kBoundsOfParts<<<1, kBlock, 0, s>>>(partLo.p, partHi.p, nPart);
+    kMorton<<<grid, kBlock, 0, s>>>(boxLo.p, boxHi.p, n, partLo.p, partHi.p, keys.p, ids.p);
     radixSortPairs(keys.p, keys2.p, ids.p, ids2.p, n, 63, counts.p, countOffs.p, scanScr.p, s);
     std::swap(keys.p, keys2.p);  // the sorted pairs live in keys2 / ids2 from here on
     std::swap(ids.p, ids2.p);
@@ -871,69 +1073,54 @@ int buildBvh(const BuildArgs& a, hipStream_t s, BuildResult& r, char* err, size_
   bool singleLeaf = n <= 1;
   if (nInternal) {
     size_t ni = nInternal;
-    HIPB(hipMalloc(&left.p, ni * sizeof(int)));
-    HIPB(hipMalloc(&right.p, ni * sizeof(int)));
-    HIPB(hipMalloc(&parent.p, ni * sizeof(int)));
-    HIPB(hipMalloc(&leafParent.p, nn * sizeof(int)));
-    HIPB(hipMalloc(&range.p, ni * sizeof(int2)));
-    HIPB(hipMalloc(&level.p, ni * sizeof(int)));
-    HIPB(hipMalloc(&maxLevel.p, sizeof(unsigned)));
-    HIPB(hipMalloc(&nodeLo.p, ni * sizeof(float4)));
-    HIPB(hipMalloc(&nodeHi.p, ni * sizeof(float4)));
-    HIPB(hipMalloc(&cost.p, ni * sizeof(float)));
-    HIPB(hipMalloc(&collapsed.p, ni));
-    HIPB(hipMalloc(&emitted.p, ni * sizeof(uint32_t)));
-    HIPB(hipMalloc(&newIdx.p, ni * sizeof(uint32_t)));
+    A.take(left, ni), A.take(right, ni), A.take(parent, ni), A.take(leafParent, nn), A.take(range, ni), A.take(level, ni);
+    A.take(maxLevel, 1), A.take(nodeLo, ni), A.take(nodeHi, ni), A.take(cost, ni), A.take(collapsed, ni), A.take(emitted, ni);
+    A.take(newIdx, ni);
+    HIPB(A.status);
     HIPB(hipMemsetAsync(maxLevel.p, 0, sizeof(unsigned), s));
     unsigned gi = (nInternal + kBlock - 1) / kBlock;
     if (a.quality == 2) {
       // PLOC hierarchy over the Morton order, then depth-first leaf order
-      DevBuf<int> cNode[2], nnb, leafParent2;
+      const size_t mark = A.used;
+      DevBuf<int> cNode[2], leafParent2;
       DevBuf<float4> cLo[2], cHi[2];
-      DevBuf<uint32_t> valid, offs, nodeCnt, posOf, sorted2;
-      DevBuf<unsigned> idCounter;
-      for (int b2 = 0; b2 < 2; ++b2) {
-        HIPB(hipMalloc(&cNode[b2].p, nn * sizeof(int)));
-        HIPB(hipMalloc(&cLo[b2].p, nn * sizeof(float4)));
-        HIPB(hipMalloc(&cHi[b2].p, nn * sizeof(float4)));
-      }
-      HIPB(hipMalloc(&nnb.p, nn * sizeof(int)));
-      HIPB(hipMalloc(&valid.p, nn * sizeof(uint32_t)));
-      HIPB(hipMalloc(&offs.p, nn * sizeof(uint32_t)));
-      HIPB(hipMalloc(&nodeCnt.p, ni * sizeof(uint32_t)));
-      HIPB(hipMalloc(&posOf.p, nn * sizeof(uint32_t)));
-      HIPB(hipMalloc(&sorted2.p, nn * sizeof(uint32_t)));
-      HIPB(hipMalloc(&leafParent2.p, nn * sizeof(int)));
-      HIPB(hipMalloc(&idCounter.p, sizeof(unsigned)));
-      HIPB(hipMemsetAsync(idCounter.p, 0, sizeof(unsigned), s));
-      int rootParent = -1;
-      HIPB(hipMemcpyAsync(parent.p, &rootParent, sizeof(int), hipMemcpyHostToDevice, s));
-      kPlocInit<<<grid, kBlock, 0, s>>>(n, ids2.p, boxLo.p, boxHi.p, cNode[0].p, cLo[0].p, cHi[0].p);
-      uint32_t m = n, iters = 0;
+      DevBuf<uint32_t> nodeCnt, posOf, sorted2, tileSums, cnt;
+      DevBuf<uint8_t> valid;
+      for (int b2 = 0; b2 < 2; ++b2) A.take(cNode[b2], nn), A.take(cLo[b2], nn), A.take(cHi[b2], nn);
+      A.take(valid, nn), A.take(nodeCnt, ni), A.take(posOf, nn), A.take(sorted2, nn), A.take(leafParent2, nn);
+      A.take(tileSums, grid), A.take(cnt, 3);  // cnt: the cluster counts of this and the next round, the nodes made
+      HIPB(A.status);
+      HIPB(hipMemsetAsync(cnt.p, 0, 3 * sizeof(uint32_t), s));
+      const PlocTree T{left.p, right.p, parent.p, leafParent.p, nodeCnt.p, nodeLo.p, nodeHi.p, cost.p, collapsed.p,
+                       n, a.leafMax, a.quality};
+      kPlocInit<<<grid, kBlock, 0, s>>>(n, ids2.p, boxLo.p, boxHi.p, cNode[0].p, cLo[0].p, cHi[0].p, cnt.p, parent.p);
+      uint32_t m = n, state[3] = {n, 0, 0};
+      static_assert(kPlocRounds % 2 == 0, "a batch of rounds ends on the first count");
       while (m > 1) {
-        unsigned gm = (m + kBlock - 1) / kBlock;
-        kPlocNearest<<<gm, kBlock, 0, s>>>(m, cLo[0].p, cHi[0].p, nnb.p);
-        kPlocMerge<<<gm, kBlock, 0, s>>>(m, n, nnb.p, cNode[0].p, cLo[0].p, cHi[0].p, cNode[1].p, cLo[1].p, cHi[1].p,
-                                          valid.p, left.p, right.p, parent.p, leafParent.p, nodeCnt.p, idCounter.p);
-        exclusiveScan(valid.p, offs.p, m, scanScr.p, s);
-        kPlocCompact<<<gm, kBlock, 0, s>>>(m, valid.p, offs.p, cNode[1].p, cLo[1].p, cHi[1].p, cNode[0].p, cLo[0].p,
-                                            cHi[0].p);
-        uint32_t lastOff = 0, lastValid = 0;
-        HIPB(hipMemcpyAsync(&lastOff, offs.p + m - 1, 4, hipMemcpyDeviceToHost, s));
-        HIPB(hipMemcpyAsync(&lastValid, valid.p + m - 1, 4, hipMemcpyDeviceToHost, s));
+        const unsigned gm = (m + kBlock - 1) / kBlock;
+        if (m <= kPlocTail) {
+          kPlocTailRounds<<<1, kPlocTail, 0, s>>>(T, cnt.p, cNode[0].p, cLo[0].p, cHi[0].p, cnt.p + 2);
+        } else {
+          for (int r = 0; r < kPlocRounds; ++r) {
+            uint32_t *now = cnt.p + r % 2, *next = cnt.p + 1 - r % 2;
+            kPlocStep<<<gm, kBlock, 0, s>>>(T, now, cNode[0].p, cLo[0].p, cHi[0].p, cNode[1].p, cLo[1].p, cHi[1].p, valid.p,
+                                            tileSums.p, cnt.p + 2);
+            kPlocScan<<<1, 1024, 0, s>>>(now, tileSums.p, next);
+            kPlocCompact<<<gm, kBlock, 0, s>>>(now, valid.p, tileSums.p, cNode[1].p, cLo[1].p, cHi[1].p, cNode[0].p, cLo[0].p,
+                                               cHi[0].p);
+          }
+        }
+        HIPB(hipMemcpyAsync(state, cnt.p, sizeof state, hipMemcpyDeviceToHost, s));
         HIPB(hipStreamSynchronize(s));
-        uint32_t next = lastOff + lastValid;
-        if (next >= m || ++iters > 100000) {
+        // every round of comparable boxes merges at least the best pair, and the tail ends with one cluster
+        if (state[0] >= m || (m <= kPlocTail && state[0] != 1)) {
           std::snprintf(err, errLen, "bvh: clustering made no progress (%u clusters)", m);
           return ASH_E_INVALID;
         }
-        m = next;
+        m = state[0];
       }
-      unsigned used = 0;
-      HIPB(hipMemcpyAsync(&used, idCounter.p, sizeof used, hipMemcpyDeviceToHost, s));
-      HIPB(hipStreamSynchronize(s));
-      if (used != nInternal) {
-        std::snprintf(err, errLen, "bvh: clustering produced %u of %u internal nodes", used, nInternal);
+      if (state[2] != nInternal) {
+        std::snprintf(err, errLen, "bvh: clustering produced %u of %u internal nodes", state[2], nInternal);
         return ASH_E_INVALID;
       }
       kPlocLeafOrder<<<grid, kBlock, 0, s>>>(n, left.p, right.p, parent.p, leafParent.p, nodeCnt.p, ids2.p, posOf.p,
@@ -943,20 +1130,21 @@ int buildBvh(const BuildArgs& a, hipStream_t s, BuildResult& r, char* err, size_
       HIPB(hipMemcpyAsync(ids2.p, sorted2.p, nn * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
       HIPB(hipMemcpyAsync(leafParent.p, leafParent2.p, nn * sizeof(int), hipMemcpyDeviceToDevice, s));
       HIPB(hipGetLastError());
+      A.used = mark;  // later takers are ordered after these kernels on the stream
     } else {
       kKarras<<<gi, kBlock, 0, s>>>(keys2.p, int(n), left.p, right.p, parent.p, leafParent.p, range.p);
+      kNodeLevel<<<gi, kBlock, 0, s>>>(int(nInternal), parent.p, level.p, maxLevel.p);
+      unsigned deepest = 0;
+      HIPB(hipMemcpyAsync(&deepest, maxLevel.p, sizeof deepest, hipMemcpyDeviceToHost, s));
+      HIPB(hipStreamSynchronize(s));
+      if (deepest >= nInternal) {
+        std::snprintf(err, errLen, "bvh: tree deeper (%u) than its node count", deepest);
+        return ASH_E_INVALID;
+      }
+      for (int lv = int(deepest); lv >= 0; --lv)
+        kRefitLevel<<<gi, kBlock, 0, s>>>(int(nInternal), lv, level.p, sorted, boxLo.p, boxHi.p, left.p, right.p,
+                                          range.p, nodeLo.p, nodeHi.p, cost.p, collapsed.p, a.leafMax, a.quality);
     }
-    kNodeLevel<<<gi, kBlock, 0, s>>>(int(nInternal), parent.p, level.p, maxLevel.p);
-    unsigned deepest = 0;
-    HIPB(hipMemcpyAsync(&deepest, maxLevel.p, sizeof deepest, hipMemcpyDeviceToHost, s));
-    HIPB(hipStreamSynchronize(s));
-    if (deepest >= nInternal) {
-      std::snprintf(err, errLen, "bvh: tree deeper (%u) than its node count", deepest);
-      return ASH_E_INVALID;
-    }
-    for (int lv = int(deepest); lv >= 0; --lv)
-      kRefitLevel<<<gi, kBlock, 0, s>>>(int(nInternal), lv, level.p, sorted, boxLo.p, boxHi.p, left.p, right.p,
-                                        range.p, nodeLo.p, nodeHi.p, cost.p, collapsed.p, a.leafMax, a.quality);
     kEmitFlags<<<gi, kBlock, 0, s>>>(int(nInternal), parent.p, collapsed.p, emitted.p, maxDepth.p);
     exclusiveScan(emitted.p, newIdx.p, nInternal, scanScr.p, s);
     uint32_t lastIdx = 0, lastEm = 0;
@@ -995,8 +1183,8 @@ int buildBvh(const BuildArgs& a, hipStream_t s, BuildResult& r, char* err, size_
   HIPB(hipGetLastError());
   {
     DevBuf<unsigned> refcnt, bad;
-    HIPB(hipMalloc(&refcnt.p, size_t(numNodes) * sizeof(unsigned)));
-    HIPB(hipMalloc(&bad.p, sizeof(unsigned)));
+    A.take(refcnt, numNodes), A.take(bad, 1);
+    HIPB(A.status);
     HIPB(hipMemsetAsync(refcnt.p, 0, size_t(numNodes) * sizeof(unsigned), s));
     HIPB(hipMemsetAsync(bad.p, 0, sizeof(unsigned), s));
     unsigned gv = (numNodes + kBlock - 1) / kBlock;
@@ -1011,37 +1199,46 @@ int buildBvh(const BuildArgs& a, hipStream_t s, BuildResult& r, char* err, size_
     }
   }
   if (a.branching == 4) {
-    DevBuf<int2> f0, f1;
-    DevBuf<unsigned> cnts;  // [0] 4-wide nodes allocated, [1] next frontier size
+    // one launch per level of the 4-wide tree; the host looks at the frontier sizes every kCollapseLevels levels,
+    // with grids for four times the last one
+    constexpr uint32_t kCollapseLevels = 4, kMaxLevels = 200;
+    DevBuf<int2> f[2];
+    DevBuf<unsigned> cnts;  // [0] 4-wide nodes allocated, [1 + l] frontier size of level l
     HIPB(hipMalloc(&r.nodes4, size_t(numNodes) * 8 * sizeof(float4)));
-    HIPB(hipMalloc(&f0.p, size_t(numNodes) * sizeof(int2)));
-    HIPB(hipMalloc(&f1.p, size_t(numNodes) * sizeof(int2)));
-    HIPB(hipMalloc(&cnts.p, 2 * sizeof(unsigned)));
-    int2 root = make_int2(0, 0);
-    unsigned init[2] = {1u, 0u};
-    HIPB(hipMemcpyAsync(f0.p, &root, sizeof root, hipMemcpyHostToDevice, s));
-    HIPB(hipMemcpyAsync(cnts.p, init, sizeof init, hipMemcpyHostToDevice, s));
-    uint32_t nFront = 1, levels = 0;
-    while (nFront) {
-      kCollapse4<<<(nFront + kBlock - 1) / kBlock, kBlock, 0, s>>>(r.nodes, f0.p, nFront, r.nodes4, cnts.p, f1.p,
-                                                                    cnts.p + 1);
-      unsigned c[2];
-      HIPB(hipMemcpyAsync(c, cnts.p, sizeof c, hipMemcpyDeviceToHost, s));
-      HIPB(hipMemsetAsync(cnts.p + 1, 0, sizeof(unsigned), s));
+    A.take(f[0], numNodes), A.take(f[1], numNodes), A.take(cnts, kMaxLevels + kCollapseLevels + 2);
+    HIPB(A.status);
+    HIPB(hipMemsetAsync(cnts.p, 0, (kMaxLevels + kCollapseLevels + 2) * sizeof(unsigned), s));
+    kCollapseInit<<<1, 1, 0, s>>>(f[0].p, cnts.p);
+    uint32_t bound = 1, levels = 0;
+    for (;;) {
+      for (uint32_t k = 0; k < kCollapseLevels; ++k, ++levels) {
+        kCollapse4<<<(bound + kBlock - 1) / kBlock, kBlock, 0, s>>>(r.nodes, f[levels & 1].p, cnts.p + 1 + levels, r.nodes4,
+                                                                    cnts.p, f[1 - (levels & 1)].p, cnts.p + 2 + levels);
+        bound = uint32_t(std::min<uint64_t>(4ull * bound, numNodes));
+      }
+      unsigned c[kCollapseLevels + 1], made = 0;  // sizes of the levels just done and of the next
+      HIPB(hipMemcpyAsync(c, cnts.p + 1 + levels - kCollapseLevels, sizeof c, hipMemcpyDeviceToHost, s));
+      HIPB(hipMemcpyAsync(&made, cnts.p, sizeof made, hipMemcpyDeviceToHost, s));
       HIPB(hipStreamSynchronize(s));
-      std::swap(f0.p, f1.p);
-      nFront = c[1];
-      r.numNodes4 = c[0];
-      ++levels;
-      if (levels > 200 || r.numNodes4 > numNodes) {
+      r.numNodes4 = made;
+      bool done = false;
+      for (uint32_t k = 1; k <= kCollapseLevels && !done; ++k)
+        if (!c[k]) levels = levels - kCollapseLevels + k, done = true;  // level k - 1 was the last
+      if (done) break;
+      bound = c[kCollapseLevels];
+      if (levels > kMaxLevels || r.numNodes4 > numNodes) {
         std::snprintf(err, errLen, "bvh: 4-wide collapse did not terminate");
         return ASH_E_INVALID;
       }
     }
+    if (levels > kMaxLevels || r.numNodes4 > numNodes) {
+      std::snprintf(err, errLen, "bvh: 4-wide collapse did not terminate");
+      return ASH_E_INVALID;
+    }
     r.depth4 = levels;
     DevBuf<unsigned> refcnt, bad;
-    HIPB(hipMalloc(&refcnt.p, size_t(r.numNodes4) * sizeof(unsigned)));
-    HIPB(hipMalloc(&bad.p, sizeof(unsigned)));
+    A.take(refcnt, r.numNodes4), A.take(bad, 1);
+    HIPB(A.status);
     HIPB(hipMemsetAsync(refcnt.p, 0, size_t(r.numNodes4) * sizeof(unsigned), s));
     HIPB(hipMemsetAsync(bad.p, 0, sizeof(unsigned), s));
     unsigned gv = (r.numNodes4 + kBlock - 1) / kBlock;

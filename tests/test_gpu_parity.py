@@ -479,3 +479,36 @@ def test_error_paths_do_not_exit(renderer):
         r = A.Renderer(0)
         cam = A.camera_lookat(8, 8, 45, (0, 0, 1), (0, 0, 0))
         r.render(cam, A.GpuPushConstantRaytrace(), 0, 1)  # render before upload
+
+
+@pytest.mark.parametrize("tris", [1, 2, 3, 33, 255, 257, 1023, 1025, 2600, 5000])
+def test_clustered_build_of_any_size_matches_lbvh(renderer, tris, tmp_path):
+    """The clustering rounds at block, halo and one-block-tail edges: the tree
+    of `tris` triangles holds them all (the build validates it) and renders
+    as the LBVH of the same triangles does, bit for bit."""
+    rng = np.random.default_rng(tris)
+    c = rng.uniform(-1, 1, (tris, 1, 3))
+    v = (c + rng.uniform(-0.1, 0.1, (tris, 3, 3))).reshape(-1, 3)
+    obj = "".join(f"v {a:.6f} {b:.6f} {z:.6f}\n" for a, b, z in v)
+    obj += "".join(f"f {3 * i + 1} {3 * i + 2} {3 * i + 3}\n" for i in range(tris))
+    (tmp_path / "soup.obj").write_text(obj)
+    (tmp_path / "scene.json").write_text(
+        '{"state": {"path_tracing": {"spp": 2, "max_path_depth": 4, "multi_channel": ["normal"]}, "output_hdr": true},'
+        ' "camera": {"type": "perspective", "film": {"resolution": [96, 64]}, "fov": 50.0},'
+        ' "materials": [{"name": "m", "type": "brdf_lambertian", "diffuse_reflectance": [0.7, 0.6, 0.5]}],'
+        ' "lights": [{"type": "rect", "radiance": [9, 9, 9], "position": [-1, 2, -1], "v1": [1, 2, -1], "v2": [-1, 2, 1]}],'
+        ' "meshes": [{"name": "soup", "path": "soup.obj"}], "instances": [{"mesh": "soup", "material": "m"}],'
+        ' "shots": [{"type": "lookat", "eye": [0, 0, 4], "lookat": [0, 0, 0], "up": [0, 1, 0]}]}')
+    s = A.HostScene(str(tmp_path / "scene.json"))
+    cam, pc = s.shot(0)
+    out = []
+    for q in (2, 0):
+        renderer.upload(s)
+        info = renderer.build(quality=q)
+        assert info["num_triangles"] == s.state.num_triangles
+        renderer.set_film(96, 64)
+        renderer.render(cam, pc, 0, 2)
+        out.append([renderer.read(0), renderer.first_hit(cam)])
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    for k in ("t", "prim_id", "normal"):
+        np.testing.assert_array_equal(out[0][1][k], out[1][1][k])
