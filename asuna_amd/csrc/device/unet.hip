@@ -498,16 +498,25 @@ __global__ __launch_bounds__(64 * kMaxChunks) void kConvSplit(ConvArgs a, uint32
 // x 16 channels), at any pixel offset, so the nine taps read the one staged
 // tile.  Each wave takes 2 of the tile's 8 steps of 32 pixels and keeps all 36
 // output tiles in registers: 20 fragments read for 36 MFMAs.  The waves' sums
-// are added in wave order through LDS.  (One wave per tap, 32 x 32 block and
-// split, gathering 2-byte values from memory, took 319 us per layer of a
-// batch of 8 x 128 x 128 on average; this takes 12.)
-struct BwdWArgs {
+// are added in wave order through LDS.
+//
+// One launch does every layer once all output gradients are there: alone, a
+// small level's layer cannot fill the chip and lasts as long as a large one.
+// A batch of 8 x 128 x 128: 319 us per layer with one wave per tap, 32 x 32
+// block and split gathering 2-byte values from memory, 12 us per layer as 19
+// launches of this kernel (230 us), 74 us for all layers in one.
+struct BwdWLayer {
   Src s0, s1;
   const bf16* dY;  // [N][H][W][32 nCo], masked
-  uint32_t N, H, W, nCo, nCi, splits;
-  uint32_t tilesX, tilesY, tiles;
   float* part;     // [splits][9][32 nCo][32 nCi]
+  uint32_t H, W, tilesX, tilesY, tiles;
+  uint16_t nCo, nCi, splits, tc;
+  uint32_t block0;  // first block of the layer
 };
+struct BwdWArgs {
+  BwdWLayer l[kNumLayers];
+};
+static_assert(sizeof(BwdWArgs) <= 4096, "kernel argument limit");
 template <int TC> struct BwdWTile {
   static constexpr uint32_t TR = 256 / TC, P = (TR + 2) * (TC + 2);
   static constexpr uint32_t LX = (P * 4 + 255) / 256;
@@ -521,15 +530,14 @@ __device__ __forceinline__ bf16x8 readTr(const bf16* p0, const bf16* p1) {
   return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 template <int TC>
-__global__ __launch_bounds__(256, 2) void kConvBwdW(BwdWArgs a) {
+__device__ __forceinline__ void bwdW(const BwdWLayer& a, uint32_t block, bf16* lds) {
   using T = BwdWTile<TC>;
   static_assert(T::lds >= 4 * 9 * 1024, "the reduction reuses the staging space");
-  __shared__ __align__(16) bf16 lds[T::lds / 2];
   bf16* xs = lds;              // [T::P][4 slots][8]
   bf16* ys = lds + T::P * 32;  // [256][4 slots][8]
   const uint32_t tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const uint32_t pairs = a.nCo * a.nCi, split = blockIdx.x / pairs;
-  const uint32_t cob = (blockIdx.x % pairs) / a.nCi, cib = (blockIdx.x % pairs) % a.nCi;
+  const uint32_t pairs = a.nCo * a.nCi, split = block / pairs;
+  const uint32_t cob = (block % pairs) / a.nCi, cib = (block % pairs) % a.nCi;
   u32x4 px[T::LX], py[4];
   auto fresh = [&]() {  // as in kConvLds
     uint32_t i = tid;
@@ -640,6 +648,17 @@ __global__ __launch_bounds__(256, 2) void kConvBwdW(BwdWArgs a) {
       for (uint32_t r = 0; r < 4; ++r) out[(size_t(tap) * Co + co + r) * Ci + ci] = s[r];
     }
   }
+}
+
+__global__ __launch_bounds__(256, 2) void kConvBwdW(BwdWArgs a) {
+  __shared__ __align__(16) bf16 lds[std::max({BwdWTile<32>::lds, BwdWTile<16>::lds, BwdWTile<8>::lds}) / 2];
+  int k = 0;
+  while (k + 1 < kNumLayers && blockIdx.x >= a.l[k + 1].block0) ++k;
+  const BwdWLayer& l = a.l[k];
+  const uint32_t block = blockIdx.x - l.block0;
+  if (l.tc == 32) bwdW<32>(l, block, lds);
+  else if (l.tc == 16) bwdW<16>(l, block, lds);
+  else bwdW<8>(l, block, lds);
 }
 
 // ------------------------------------------------- parameters (all layers)
@@ -1176,18 +1195,17 @@ static int trainForward(ash_denoiser* d) {
 }
 
 // Pixel tiles of a layer's weight gradient: 32, 16 or 8 columns by the
-// image's width, and one split per tile up to two blocks per CU.
-struct BwdWPlan {
-  uint32_t tc, tilesX, tilesY, tiles, splits;
-};
-static BwdWPlan bwdWPlan(const ash_denoiser* d, const Layer& l, uint32_t N, uint32_t H, uint32_t W) {
-  BwdWPlan p;
-  p.tc = W > 16 ? 32 : W > 8 ? 16 : 8;
-  const uint32_t tr = 256 / p.tc, pairs = (l.CoS / 32) * ((l.CaS + l.CbS) / 32);
+// image's width, kBwdWTiles of them per block (fewer partial sums to write and
+// add than with a block per tile, more blocks than with one per CU).
+constexpr uint32_t kBwdWTiles = 4;
+static void bwdWPlan(const Layer& l, uint32_t N, uint32_t H, uint32_t W, BwdWLayer& p) {
+  p.tc = uint16_t(W > 16 ? 32 : W > 8 ? 16 : 8);
+  const uint32_t tr = 256 / p.tc;
+  p.H = H, p.W = W;
+  p.nCo = uint16_t(l.CoS / 32), p.nCi = uint16_t((l.CaS + l.CbS) / 32);
   p.tilesX = (W + p.tc - 1) / p.tc, p.tilesY = (H + tr - 1) / tr;
   p.tiles = N * p.tilesX * p.tilesY;
-  p.splits = std::max<uint32_t>(1, std::min(p.tiles, 2 * uint32_t(d->numCU) / pairs));
-  return p;
+  p.splits = uint16_t(std::min<uint32_t>((p.tiles + kBwdWTiles - 1) / kBwdWTiles, 512));
 }
 
 // Loss, then the gradient of the loss w.r.t. all parameters into d->grad;
@@ -1199,9 +1217,16 @@ static int backwardPass(ash_denoiser* d, const AdamArgs* adam) {
   // a convolution's backward-x plan, and the partial sums' places
   auto xPlan = [&](const Step& st) { return convPlan(d, N, st.out->H, st.out->W, (d->L[st.layer].CaS + d->L[st.layer].CbS) / 32); };
   LayerTab T = layerTab(d);
+  BwdWArgs w;
+  std::memset(&w, 0, sizeof w);
+  uint32_t wBlocks = 0;
   for (const Step& st : sched) {
     const Layer& l = d->L[st.layer];
-    T.r[st.layer].splits = bwdWPlan(d, l, N, st.out->H, st.out->W).splits;
+    BwdWLayer& wl = w.l[st.layer];
+    bwdWPlan(l, N, st.out->H, st.out->W, wl);
+    T.r[st.layer].splits = wl.splits;
+    wl.block0 = wBlocks;
+    wBlocks += uint32_t(wl.splits) * wl.nCo * wl.nCi;
     // the bias gradient is summed where the output's gradient is completed: by the layer that reads it
     // (its pooled copy, where there is one), or by the loss
     int made = -1;
@@ -1228,20 +1253,11 @@ static int backwardPass(ash_denoiser* d, const AdamArgs* adam) {
     const Step& st = sched[k];
     const Layer& l = d->L[st.layer];
     const Act& o = *st.out;
-    const BwdWPlan wp = bwdWPlan(d, l, N, o.H, o.W);
-    BwdWArgs b;
-    std::memset(&b, 0, sizeof b);
-    b.s0 = Src{st.s0->a.p, st.s0->C, st.up ? 1u : 0u};
-    if (st.s1) b.s1 = Src{st.s1->a.p, st.s1->C, 0};
-    b.dY = o.g.p;
-    b.N = N, b.H = o.H, b.W = o.W;
-    b.nCo = l.CoS / 32, b.nCi = (l.CaS + l.CbS) / 32;
-    b.splits = wp.splits, b.tilesX = wp.tilesX, b.tilesY = wp.tilesY, b.tiles = wp.tiles;
-    b.part = d->part.p + T.r[st.layer].wPart;
-    const uint32_t grid = b.nCo * b.nCi * b.splits;
-    if (wp.tc == 32) kConvBwdW<32><<<grid, 256, 0, d->stream>>>(b);
-    else if (wp.tc == 16) kConvBwdW<16><<<grid, 256, 0, d->stream>>>(b);
-    else kConvBwdW<8><<<grid, 256, 0, d->stream>>>(b);
+    BwdWLayer& wl = w.l[st.layer];
+    wl.s0 = Src{st.s0->a.p, st.s0->C, st.up ? 1u : 0u};
+    if (st.s1) wl.s1 = Src{st.s1->a.p, st.s1->C, 0};
+    wl.dY = o.g.p;
+    wl.part = d->part.p + T.r[st.layer].wPart;
     if (st.s0 == &d->x) continue;  // no gradient for the input features
     ConvArgs a;
     std::memset(&a, 0, sizeof a);
@@ -1263,6 +1279,7 @@ static int backwardPass(ash_denoiser* d, const AdamArgs* adam) {
     if (st.s1) a.d1.kind = kGradSkip, a.d1.C = st.s1->C, a.d1.skip = st.s1->skip.p;
     launchConv<kModeGrad>(d, a, xPlan(st));
   }
+  kConvBwdW<<<wBlocks, 256, 0, d->stream>>>(w);
   const uint32_t nb = uint32_t(d->nParams / 32);
   if (adam) kGradients<true><<<nb, 256, 0, d->stream>>>(T, d->part.p, d->grad.p, *adam, d->wf.p, d->wb.p);
   else kGradients<false><<<nb, 256, 0, d->stream>>>(T, d->part.p, d->grad.p, AdamArgs{}, nullptr, nullptr);
