@@ -55,7 +55,7 @@ struct SceneView {
   const float* condX;  // W*H entries: the conditional table's inverse-CDF channel, in 8x4-texel tiles
   const DevSky* sky;   // sun & sky (inUse 0: env map / background)
   uint32_t hasSide;    // some surface belongs to the second plugin group
-  // two-level acceleration (twoLevel = 1): TLAS binary nodes over instances
+  // two-level acceleration (twoLevel = 1): TLAS 4-wide nodes over instances
   // (leaf = one instance: its index in tlasInst), per-instance BLAS slot
   uint32_t twoLevel;
   const float4* tlas;

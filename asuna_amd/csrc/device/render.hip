@@ -484,7 +484,7 @@ __device__ __forceinline__ int popClosest(Stack& st, int best, float bt) {
 }
 
 // ------------------------------------------------ two-level traversal
-// The TLAS is a binary tree over the instances' world boxes, walked with
+// The TLAS is a tree over the instances' world boxes, walked with
 // the world ray.  At an instance leaf the ray enters the instance's BLAS in
 // object space (origin and direction through the world-to-object
 // transform; the direction is not normalised, so t is the same parameter
@@ -509,29 +509,6 @@ __device__ __forceinline__ float4 toWorld(const DevInstance& in, float4 p) {
   const float* m = in.o2w;
   return make_float4(m[0] * p.x + m[1] * p.y + m[2] * p.z + m[3], m[4] * p.x + m[5] * p.y + m[6] * p.z + m[7],
                      m[8] * p.x + m[9] * p.y + m[10] * p.z + m[11], 0.f);
-}
-
-// One TLAS node step: pushes the farther of two entered children; returns
-// the next node, or kDoneRef when neither child is entered.
-__device__ __forceinline__ int tlasStep(const SceneView& sc, const TRay& rw, int node, float tmin, float lim,
-                                        Stack& st) {
-  const float4* np = sc.tlas + size_t(node) * 4;
-  const float4 n0 = np[0], n1 = np[1], n2 = np[2], n3 = np[3];
-  float t0, t1;
-  const bool h0 = slab(n0.x, n0.y, n0.z, n0.w, n2.x, n2.y, rw, tmin, lim, t0);
-  const bool h1 = slab(n1.x, n1.y, n1.z, n1.w, n2.z, n2.w, rw, tmin, lim, t1);
-  int c0 = __float_as_int(n3.x), c1 = __float_as_int(n3.y);
-  if (h0 && h1) {
-    if (t1 < t0) {
-      const int c = c0;
-      c0 = c1, c1 = c;
-      const float t = t0;
-      t0 = t1, t1 = t;
-    }
-    st.push(c1, t1);
-    return c0;
-  }
-  return h0 ? c0 : (h1 ? c1 : kDoneRef);
 }
 
 
@@ -1393,10 +1370,15 @@ __device__ __forceinline__ void shadowDynLoop(const SceneView& sc, const Wavefro
 // TLAS node, the entry into a BLAS with the ray taken to object space, a
 // BLAS node or a BLAS leaf, then the pop when the step does not descend).
 // It leaves a BLAS when the stack falls back to the depth it had on entry.
+// Both levels have 4-wide nodes and the walk keeps the ray of the level it is in
+// (ro, the world ray again on leaving a BLAS), so lanes in the TLAS and lanes in
+// a BLAS share the node test; with binary TLAS nodes tested apart and median
+// splits, 256 instances of four meshes at 4 spp took 7.04 ms, now 5.54.
 // Visit order, culling and tie rule (equal t: smaller global id) are those
 // of the flat walk, so the closest hit does not depend on how a lane's steps
 // are grouped into rounds.
 struct Walk2L {
+  const float4* nodes;  // of the level the walk is in
   int node, cur, base, best, bestGid, bInst;
   float bt, bu, bv;
   uint32_t triBase, blas;
@@ -1409,33 +1391,11 @@ template <bool COUNT>
 __device__ __forceinline__ bool step2L(const SceneView& sc, const TRay& rw, TRay& ro, Walk2L& s, Stack& st,
                                        uint32_t& nN, uint32_t& nT) {
   const float tmin = kMinimum, tmax = kInf;
-  if (s.node == kDoneRef) {
-    // falls through to the pop below
-  } else if (s.cur < 0) {
-    if (s.node >= 0) {
-      if (s.node != kEmptyRef) {
-        if (COUNT) ++nN;
-        s.node = tlasStep(sc, rw, s.node, tmin, s.best >= 0 ? s.bt : tmax, st);
-        if (s.node != kDoneRef) return false;
-      }
-    } else {
-      uint32_t first, cnt;
-      decodeLeaf(s.node, first, cnt);
-      const uint32_t i = sc.tlasInst[first];
-      const DevInstance& in = sc.inst[i];
-      toObject(in, rw, ro);
-      s.blas = sc.instBlas[i];
-      s.cur = int(i);
-      s.triBase = in.triBase;
-      s.base = st.sp;
-      s.node = 0;
-      return false;
-    }
-  } else if (s.node >= 0) {
+  if (s.node >= 0) {
     if (s.node != kEmptyRef) {
       if (COUNT) ++nN;
       Kids k;
-      testNode4(sc.blas[s.blas].nodes4 + size_t(s.node) * 8, ro, tmin, s.best >= 0 ? s.bt : tmax, k);
+      testNode4(s.nodes + size_t(s.node) * 8, ro, tmin, s.best >= 0 ? s.bt : tmax, k);
       if (k.n > 0) {
         if (k.n > 3) st.push(k.c[3], k.t[3]);
         if (k.n > 2) st.push(k.c[2], k.t[2]);
@@ -1444,6 +1404,19 @@ __device__ __forceinline__ bool step2L(const SceneView& sc, const TRay& rw, TRay
         return false;
       }
     }
+  } else if (s.cur < 0) {
+    uint32_t first, cnt;
+    decodeLeaf(s.node, first, cnt);
+    const uint32_t i = sc.tlasInst[first];
+    const DevInstance& in = sc.inst[i];
+    toObject(in, rw, ro);
+    s.blas = sc.instBlas[i];
+    s.nodes = sc.blas[s.blas].nodes4;
+    s.cur = int(i);
+    s.triBase = in.triBase;
+    s.base = st.sp;
+    s.node = 0;
+    return false;
   } else {
     uint32_t first, cnt;
     decodeLeaf(s.node, first, cnt);
@@ -1465,7 +1438,11 @@ __device__ __forceinline__ bool step2L(const SceneView& sc, const TRay& rw, TRay
     }
   }
   for (;;) {
-    if (s.cur >= 0 && st.sp == s.base) s.cur = -1;  // this instance's BLAS is done
+    if (s.cur >= 0 && st.sp == s.base) {  // this instance's BLAS is done
+      s.cur = -1;
+      s.nodes = sc.tlas;
+      ro = rw;
+    }
     if (st.sp == 0) {
       s.node = kDoneRef;
       return true;
@@ -1524,6 +1501,8 @@ __device__ __forceinline__ void extend2LLoop(const SceneView& sc, const Wavefron
       if (fetchIdle(f, !active, lane, drained, i)) {
         slot = i;
         setupRay(rw, xyz(qo[i]), xyz(qd[i]));
+        ro = rw;
+        s.nodes = sc.tlas;
         s.node = 0;
         s.cur = -1;
         s.base = 0;
@@ -1555,6 +1534,7 @@ __device__ __forceinline__ void extend2LLoop(const SceneView& sc, const Wavefron
 // The any-hit walk in the same resumable form; step result 0: walking,
 // 1: finished without a hit, 2: occluded.
 struct Any2L {
+  const float4* nodes;
   int node, cur, base;
   uint32_t blas;
 };
@@ -1562,31 +1542,11 @@ template <bool COUNT>
 __device__ __forceinline__ int stepAny2L(const SceneView& sc, const TRay& rw, TRay& ro, float tmax, Any2L& s,
                                          Stack& st, uint32_t& nN, uint32_t& nT) {
   const float tmin = 0.0f;
-  if (s.node == kDoneRef) {
-    // falls through to the pop below
-  } else if (s.cur < 0) {
-    if (s.node >= 0) {
-      if (s.node != kEmptyRef) {
-        if (COUNT) ++nN;
-        s.node = tlasStep(sc, rw, s.node, tmin, tmax, st);
-        if (s.node != kDoneRef) return 0;
-      }
-    } else {
-      uint32_t first, cnt;
-      decodeLeaf(s.node, first, cnt);
-      const uint32_t i = sc.tlasInst[first];
-      toObject(sc.inst[i], rw, ro);
-      s.blas = sc.instBlas[i];
-      s.cur = int(i);
-      s.base = st.sp;
-      s.node = 0;
-      return 0;
-    }
-  } else if (s.node >= 0) {
+  if (s.node >= 0) {
     if (s.node != kEmptyRef) {
       if (COUNT) ++nN;
       Kids k;
-      testNode4(sc.blas[s.blas].nodes4 + size_t(s.node) * 8, ro, tmin, tmax, k);
+      testNode4(s.nodes + size_t(s.node) * 8, ro, tmin, tmax, k);
       if (k.n > 0) {
         if (k.n > 3) st.push(k.c[3], k.t[3]);
         if (k.n > 2) st.push(k.c[2], k.t[2]);
@@ -1595,6 +1555,17 @@ __device__ __forceinline__ int stepAny2L(const SceneView& sc, const TRay& rw, TR
         return 0;
       }
     }
+  } else if (s.cur < 0) {
+    uint32_t first, cnt;
+    decodeLeaf(s.node, first, cnt);
+    const uint32_t i = sc.tlasInst[first];
+    toObject(sc.inst[i], rw, ro);
+    s.blas = sc.instBlas[i];
+    s.nodes = sc.blas[s.blas].nodes4;
+    s.cur = int(i);
+    s.base = st.sp;
+    s.node = 0;
+    return 0;
   } else {
     uint32_t first, cnt;
     decodeLeaf(s.node, first, cnt);
@@ -1606,7 +1577,11 @@ __device__ __forceinline__ int stepAny2L(const SceneView& sc, const TRay& rw, TR
       if (hitTri(ro, tp[0], tp[1], tp[2], tmin, tmax, t, u, v)) return 2;
     }
   }
-  if (s.cur >= 0 && st.sp == s.base) s.cur = -1;  // this instance's BLAS is done
+  if (s.cur >= 0 && st.sp == s.base) {  // this instance's BLAS is done
+    s.cur = -1;
+    s.nodes = sc.tlas;
+    ro = rw;
+  }
   if (st.sp == 0) return 1;
   float tn;
   s.node = st.pop(tn);
@@ -1635,6 +1610,8 @@ __device__ __forceinline__ void shadow2LLoop(const SceneView& sc, const Wavefron
         slot = i;
         const float4 so = w.shO[i], sd = w.shD[i];
         setupRay(rw, xyz(so), xyz(sd));
+        ro = rw;
+        s.nodes = sc.tlas;
         tmax = so.w;
         pid = __float_as_int(sd.w);
         s.node = 0;
@@ -1663,7 +1640,7 @@ __device__ __forceinline__ void shadow2LLoop(const SceneView& sc, const Wavefron
   }
 }
 template <bool COUNT>
-__global__ __launch_bounds__(kTraceBlock) void kExtend2L(SceneView sc, Wavefront w, int cur) {
+__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(5))) void kExtend2L(SceneView sc, Wavefront w, int cur) {
   __shared__ int lds[kStackLds * kTraceBlock];
   __shared__ float ldsT[kStackLds * kTraceBlock];
   Stack st;
