@@ -1365,15 +1365,16 @@ __device__ __forceinline__ void shadowDynLoop(const SceneView& sc, const Wavefro
 // slices, as the flat walks take them), as separate kernels and fused like
 // kTraceDyn (a wave that runs out of closest-hit rays takes shadow rays).
 //
-// The closest-hit walk is resumable, for per-lane refill: its state stays in
-// registers between rounds, and each step is one iteration of the walk (a
-// TLAS node, the entry into a BLAS with the ray taken to object space, a
-// BLAS node or a BLAS leaf, then the pop when the step does not descend).
-// It leaves a BLAS when the stack falls back to the depth it had on entry.
+// The walk is resumable, for per-lane refill: its state stays in registers
+// between rounds.  It enters a BLAS at an instance leaf, with the ray taken to
+// object space, and leaves it when the stack falls back to the depth it had on
+// entry.
 // Both levels have 4-wide nodes and the walk keeps the ray of the level it is in
 // (ro, the world ray again on leaving a BLAS), so lanes in the TLAS and lanes in
-// a BLAS share the node test; with binary TLAS nodes tested apart and median
-// splits, 256 instances of four meshes at 4 spp took 7.04 ms, now 5.54.
+// a BLAS share the node test: 256 instances of four meshes at 4 spp 7.04 ms with
+// binary TLAS nodes tested apart and median splits, 5.50 with both; in rounds
+// that descend together and then turn to the leaves, instead of 8 mixed steps of
+// node, entry or leaf per lane, 4.77.
 // Visit order, culling and tie rule (equal t: smaller global id) are those
 // of the flat walk, so the closest hit does not depend on how a lane's steps
 // are grouped into rounds.
@@ -1383,15 +1384,40 @@ struct Walk2L {
   float bt, bu, bv;
   uint32_t triBase, blas;
 };
-constexpr int kSteps2L = 8;    // steps per round between refills
+constexpr int kBreak2L = 8;    // lanes at inner nodes below which a round turns to the leaves
 constexpr int kRefill2L = 48;  // idle lanes of a wave that trigger a refill
 
-// One step; true when the walk has finished.
+// Next node after the current one is done: leaves a BLAS whose entries are
+// all popped, drops entries beyond the closest hit; kDoneRef at the end.
+__device__ __forceinline__ void pop2L(const SceneView& sc, const TRay& rw, TRay& ro, Walk2L& s, Stack& st) {
+  for (;;) {
+    if (s.cur >= 0 && st.sp == s.base) {  // this instance's BLAS is done
+      s.cur = -1;
+      s.nodes = sc.tlas;
+      ro = rw;
+    }
+    if (st.sp == 0) {
+      s.node = kDoneRef;
+      return;
+    }
+    float tn;
+    const int c = st.pop(tn);
+    if (s.best < 0 || tn <= s.bt * 1.0000004f) {
+      s.node = c;
+      return;
+    }
+  }
+}
+
+// One round: the lanes descend until fewer than kBreak2L of them are at inner
+// nodes (of either level), then those at a leaf enter its instance or test its
+// triangles.  True when the walk has finished.
 template <bool COUNT>
-__device__ __forceinline__ bool step2L(const SceneView& sc, const TRay& rw, TRay& ro, Walk2L& s, Stack& st,
-                                       uint32_t& nN, uint32_t& nT) {
+__device__ __forceinline__ bool round2L(const SceneView& sc, const TRay& rw, TRay& ro, Walk2L& s, Stack& st,
+                                        uint32_t& nN, uint32_t& nT) {
   const float tmin = kMinimum, tmax = kInf;
-  if (s.node >= 0) {
+  while (s.node >= 0) {
+    bool in = false;
     if (s.node != kEmptyRef) {
       if (COUNT) ++nN;
       Kids k;
@@ -1401,12 +1427,16 @@ __device__ __forceinline__ bool step2L(const SceneView& sc, const TRay& rw, TRay
         if (k.n > 2) st.push(k.c[2], k.t[2]);
         if (k.n > 1) st.push(k.c[1], k.t[1]);
         s.node = k.c[0];
-        return false;
+        in = true;
       }
     }
-  } else if (s.cur < 0) {
-    uint32_t first, cnt;
-    decodeLeaf(s.node, first, cnt);
+    if (!in) pop2L(sc, rw, ro, s, st);
+    if (__popcll(__ballot(s.node >= 0)) < kBreak2L) break;
+  }
+  if (s.node >= 0 || s.node == kDoneRef) return s.node == kDoneRef;
+  uint32_t first, cnt;
+  decodeLeaf(s.node, first, cnt);
+  if (s.cur < 0) {
     const uint32_t i = sc.tlasInst[first];
     const DevInstance& in = sc.inst[i];
     toObject(in, rw, ro);
@@ -1417,43 +1447,25 @@ __device__ __forceinline__ bool step2L(const SceneView& sc, const TRay& rw, TRay
     s.base = st.sp;
     s.node = 0;
     return false;
-  } else {
-    uint32_t first, cnt;
-    decodeLeaf(s.node, first, cnt);
-    const float4* tris = sc.blas[s.blas].tris;
-    for (uint32_t k = first; k < first + cnt; ++k) {
-      const float4* tp = tris + size_t(k) * 3;
-      const float4 p0 = tp[0], p1 = tp[1], p2 = tp[2];
-      if (COUNT) ++nT;
-      float t, u, v;
-      if (hitTri(ro, p0, p1, p2, tmin, s.best >= 0 ? s.bt : tmax, t, u, v)) {
-        const int gid = int(s.triBase) + __float_as_int(p2.w);
-        if (s.best < 0 || t < s.bt || (t == s.bt && gid < s.bestGid)) {
-          s.bt = t, s.bu = u, s.bv = v;
-          s.best = int(k);
-          s.bestGid = gid;
-          s.bInst = s.cur;
-        }
+  }
+  const float4* tris = sc.blas[s.blas].tris;
+  for (uint32_t k = first; k < first + cnt; ++k) {
+    const float4* tp = tris + size_t(k) * 3;
+    const float4 p0 = tp[0], p1 = tp[1], p2 = tp[2];
+    if (COUNT) ++nT;
+    float t, u, v;
+    if (hitTri(ro, p0, p1, p2, tmin, s.best >= 0 ? s.bt : tmax, t, u, v)) {
+      const int gid = int(s.triBase) + __float_as_int(p2.w);
+      if (s.best < 0 || t < s.bt || (t == s.bt && gid < s.bestGid)) {
+        s.bt = t, s.bu = u, s.bv = v;
+        s.best = int(k);
+        s.bestGid = gid;
+        s.bInst = s.cur;
       }
     }
   }
-  for (;;) {
-    if (s.cur >= 0 && st.sp == s.base) {  // this instance's BLAS is done
-      s.cur = -1;
-      s.nodes = sc.tlas;
-      ro = rw;
-    }
-    if (st.sp == 0) {
-      s.node = kDoneRef;
-      return true;
-    }
-    float tn;
-    const int c = st.pop(tn);
-    if (s.best < 0 || tn <= s.bt * 1.0000004f) {
-      s.node = c;
-      return false;
-    }
-  }
+  pop2L(sc, rw, ro, s, st);
+  return s.node == kDoneRef;
 }
 
 // Records the closest hit of queue slot i.  t and barycentrics of the hit
@@ -1481,8 +1493,7 @@ __device__ __forceinline__ void write2LHit(const SceneView& sc, const Wavefront&
 
 // Persistent closest-hit loop over queue `cur` with per-lane refill (idle
 // lanes take new rays from the XCD slices once kRefill2L of them are idle),
-// as the flat walk's extendDynLoop; each active lane runs up to kSteps2L
-// steps per round.
+// as the flat walk's extendDynLoop, in rounds.
 template <bool COUNT>
 __device__ __forceinline__ void extend2LLoop(const SceneView& sc, const Wavefront& w, int cur, Stack& st, int lane,
                                              uint32_t& nNodes, uint32_t& nTris) {
@@ -1522,27 +1533,35 @@ __device__ __forceinline__ void extend2LLoop(const SceneView& sc, const Wavefron
       continue;
     }
     if (active) {
-      bool done = false;
-      for (int k = 0; k < kSteps2L && !done; ++k) done = step2L<COUNT>(sc, rw, ro, s, st, nNodes, nTris);
-      if (done) {
+      if (round2L<COUNT>(sc, rw, ro, s, st, nNodes, nTris)) {
         active = false;
         write2LHit(sc, w, slot, rw, s.bInst, s.best, s.bt, s.bu, s.bv);
       }
     }
   }
 }
-// The any-hit walk in the same resumable form; step result 0: walking,
-// 1: finished without a hit, 2: occluded.
+// The any-hit walk in the same rounds; result 0: walking, 1: finished without
+// a hit, 2: occluded.
 struct Any2L {
   const float4* nodes;
   int node, cur, base;
   uint32_t blas;
 };
+__device__ __forceinline__ void popAny2L(const SceneView& sc, const TRay& rw, TRay& ro, Any2L& s, Stack& st) {
+  if (s.cur >= 0 && st.sp == s.base) {  // this instance's BLAS is done
+    s.cur = -1;
+    s.nodes = sc.tlas;
+    ro = rw;
+  }
+  float tn;
+  s.node = st.sp == 0 ? kDoneRef : st.pop(tn);
+}
 template <bool COUNT>
-__device__ __forceinline__ int stepAny2L(const SceneView& sc, const TRay& rw, TRay& ro, float tmax, Any2L& s,
-                                         Stack& st, uint32_t& nN, uint32_t& nT) {
+__device__ __forceinline__ int roundAny2L(const SceneView& sc, const TRay& rw, TRay& ro, float tmax, Any2L& s,
+                                          Stack& st, uint32_t& nN, uint32_t& nT) {
   const float tmin = 0.0f;
-  if (s.node >= 0) {
+  while (s.node >= 0) {
+    bool in = false;
     if (s.node != kEmptyRef) {
       if (COUNT) ++nN;
       Kids k;
@@ -1552,12 +1571,17 @@ __device__ __forceinline__ int stepAny2L(const SceneView& sc, const TRay& rw, TR
         if (k.n > 2) st.push(k.c[2], k.t[2]);
         if (k.n > 1) st.push(k.c[1], k.t[1]);
         s.node = k.c[0];
-        return 0;
+        in = true;
       }
     }
-  } else if (s.cur < 0) {
-    uint32_t first, cnt;
-    decodeLeaf(s.node, first, cnt);
+    if (!in) popAny2L(sc, rw, ro, s, st);
+    if (__popcll(__ballot(s.node >= 0)) < kBreak2L) break;
+  }
+  if (s.node >= 0) return 0;
+  if (s.node == kDoneRef) return 1;
+  uint32_t first, cnt;
+  decodeLeaf(s.node, first, cnt);
+  if (s.cur < 0) {
     const uint32_t i = sc.tlasInst[first];
     toObject(sc.inst[i], rw, ro);
     s.blas = sc.instBlas[i];
@@ -1566,26 +1590,16 @@ __device__ __forceinline__ int stepAny2L(const SceneView& sc, const TRay& rw, TR
     s.base = st.sp;
     s.node = 0;
     return 0;
-  } else {
-    uint32_t first, cnt;
-    decodeLeaf(s.node, first, cnt);
-    const float4* tris = sc.blas[s.blas].tris;
-    for (uint32_t k = first; k < first + cnt; ++k) {
-      const float4* tp = tris + size_t(k) * 3;
-      float t, u, v;
-      if (COUNT) ++nT;
-      if (hitTri(ro, tp[0], tp[1], tp[2], tmin, tmax, t, u, v)) return 2;
-    }
   }
-  if (s.cur >= 0 && st.sp == s.base) {  // this instance's BLAS is done
-    s.cur = -1;
-    s.nodes = sc.tlas;
-    ro = rw;
+  const float4* tris = sc.blas[s.blas].tris;
+  for (uint32_t k = first; k < first + cnt; ++k) {
+    const float4* tp = tris + size_t(k) * 3;
+    float t, u, v;
+    if (COUNT) ++nT;
+    if (hitTri(ro, tp[0], tp[1], tp[2], tmin, tmax, t, u, v)) return 2;
   }
-  if (st.sp == 0) return 1;
-  float tn;
-  s.node = st.pop(tn);
-  return 0;
+  popAny2L(sc, rw, ro, s, st);
+  return s.node == kDoneRef ? 1 : 0;
 }
 
 // Persistent any-hit loop over the shadow-ray queue with per-lane refill,
@@ -1627,8 +1641,7 @@ __device__ __forceinline__ void shadow2LLoop(const SceneView& sc, const Wavefron
       continue;
     }
     if (active) {
-      int r = 0;
-      for (int k = 0; k < kSteps2L && r == 0; ++k) r = stepAny2L<COUNT>(sc, rw, ro, tmax, s, st, nNodes, nTris);
+      const int r = roundAny2L<COUNT>(sc, rw, ro, tmax, s, st, nNodes, nTris);
       if (r != 0) {
         active = false;
         if (r == 1) {
