@@ -192,3 +192,24 @@ def test_camera_walk_does_not_change_images(renderer, spheres_small, frames):
         for a, b in zip(ref, got):
             np.testing.assert_array_equal(a, b)
         _render(renderer, s, 8 if frames < 8 else 1)  # the other walk in between
+
+
+@pytest.mark.parametrize("shots", [3, 400, 1500])
+def test_shot_tables_of_any_size(renderer, box_scene, shots):
+    """Small unit and shot tables go through the context's pinned buffer,
+    large ones are copied from ordinary memory: a shot's image is that of the
+    shot rendered alone, right after calls of the other kind too."""
+    s = A.HostScene(box_scene)
+    renderer.upload(s)
+    renderer.build()
+    _, pc = s.shot(0)
+    cams = [A.camera_lookat(8, 8, 60.0, (0.1 * k, 0.0, 2.5), (0.0, 0.0, 0.0)) for k in range(3)]
+    ref = []
+    for cam in cams:
+        renderer.set_film(8, 8)
+        renderer.render(cam, pc, 0, 2)
+        ref.append(renderer.read(0))
+    st = renderer.render_shots([cams[i % 3] for i in range(shots)], [pc] * shots, 2)
+    assert st["paths"] == shots * 64 * 2
+    for i in (0, 1, 2, shots // 2, shots - 1):
+        np.testing.assert_array_equal(renderer.read_shot(i, 0), ref[i % 3])
