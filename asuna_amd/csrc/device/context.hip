@@ -114,9 +114,10 @@ struct ash_ctx {
   uint32_t shotCount = 0, shotW = 0, shotH = 0;
   // wavefront
   Wavefront wf{};
-  DBuf<float4> wRayO0, wRayO1, wRayD0, wRayD1, wThr0, wThr1, wRad, wLd, wHitF, wShO, wShD;
+  DBuf<float4> wRayO0, wRayO1, wRayD0, wRayD1, wThr0, wThr1, wRad, wLd, wShO, wShD;
   DBuf<uint4> wInfo0, wInfo1;
-  DBuf<int4> wHitI;
+  DBuf<int4> wHit;
+  DBuf<float> wHitT;
   DBuf<int> wSide, wSpill;
   DBuf<float> wSpillT;
   DBuf<uint32_t> wCtr;
@@ -156,10 +157,10 @@ struct ash_ctx {
     if (shadeTris) (void)hipFree(shadeTris);
     for (auto& t : texData) t.release();
     for (auto* b : {&verts, &env, &images, &shotImages, &wRayO0, &wRayO1, &wRayD0, &wRayD1, &wThr0, &wThr1, &wRad, &wLd,
-                    &wHitF, &wShO, &wShD})
+                    &wShO, &wShD})
       b->release();
     inst.release(), idx.release(), instTriOffset.release(), mats.release(), lights.release(), texTab.release();
-    marg.release(), condX.release(), shotTab.release(), wInfo0.release(), wInfo1.release(), wHitI.release();
+    marg.release(), condX.release(), shotTab.release(), wInfo0.release(), wInfo1.release(), wHit.release(), wHitT.release();
     wSide.release(), wSpill.release(), wSpillT.release(), wCtr.release(), wCnt64.release();
     unitBuf.release(), sky.release();
     for (auto& g : graphs) releaseGraph(g);
@@ -261,12 +262,12 @@ static int ensureWavefront(ash_ctx* c, uint32_t cap) {
   MALLOC(c, c->wThr1, cap);
   MALLOC(c, c->wRad, cap);
   MALLOC(c, c->wLd, cap);
-  MALLOC(c, c->wHitF, cap);
   MALLOC(c, c->wShO, cap);
   MALLOC(c, c->wShD, cap);
   MALLOC(c, c->wInfo0, cap);
   MALLOC(c, c->wInfo1, cap);
-  MALLOC(c, c->wHitI, cap);
+  MALLOC(c, c->wHit, cap);
+  MALLOC(c, c->wHitT, cap);
   MALLOC(c, c->wSide, cap);
   MALLOC(c, c->wCtr, kNumCtr);
   MALLOC(c, c->wCnt64, kNumCnt64);
@@ -282,8 +283,8 @@ static int ensureWavefront(ash_ctx* c, uint32_t cap) {
   w.ld = c->wLd.p;
   w.info[0] = c->wInfo0.p;
   w.info[1] = c->wInfo1.p;
-  w.hitF = c->wHitF.p;
-  w.hitI = c->wHitI.p;
+  w.hit = c->wHit.p;
+  w.hitT = c->wHitT.p;
   w.side = c->wSide.p;
   w.shO = c->wShO.p;
   w.shD = c->wShD.p;
@@ -1064,11 +1065,11 @@ static size_t noAllocLayout(unsigned char* base, uint32_t threads, uint32_t cap,
   for (int q = 0; q < 2; ++q) w.thr[q] = reinterpret_cast<float4*>(take(n * sizeof(float4)));
   w.rad = reinterpret_cast<float4*>(take(n * sizeof(float4)));
   w.ld = reinterpret_cast<float4*>(take(n * sizeof(float4)));
-  w.hitF = reinterpret_cast<float4*>(take(n * sizeof(float4)));
   w.shO = reinterpret_cast<float4*>(take(n * sizeof(float4)));
   w.shD = reinterpret_cast<float4*>(take(n * sizeof(float4)));
   for (int q = 0; q < 2; ++q) w.info[q] = reinterpret_cast<uint4*>(take(n * sizeof(uint4)));
-  w.hitI = reinterpret_cast<int4*>(take(n * sizeof(int4)));
+  w.hit = reinterpret_cast<int4*>(take(n * sizeof(int4)));
+  w.hitT = reinterpret_cast<float*>(take(n * sizeof(float)));
   w.side = reinterpret_cast<int*>(take(n * sizeof(int)));
   w.ctr = reinterpret_cast<uint32_t*>(take(kNumCtr * sizeof(uint32_t)));
   w.cnt64 = reinterpret_cast<unsigned long long*>(take(kNumCnt64 * sizeof(unsigned long long)));

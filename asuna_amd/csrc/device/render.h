@@ -78,8 +78,8 @@ struct Wavefront {
   uint4* info[2];   // x seed, y depth | bsdfFlags << 16, z pixel, w shot | (frame == 0) << 16
   float4* rad;   // by path id: radiance.xyz, w = Gaussian filter weight
   float4* ld;    // pending NEE radiance of the current bounce, per shadow-ray slot
-  float4* hitF;  // per slot of the queue being traced: t, u, v
-  int4* hitI;    // instance (-1 miss), shade word, global triangle id, leaf position
+  int4* hit;     // per slot of the queue being traced: instance (-1 miss), leaf position, u, v
+  float* hitT;   // its distance, which only the depth channel and the first-hit query read
   int* side;     // second-group shading queue: slots of the current extension queue
   float4* shO;  // shadow rays: origin.xyz, tmax
   float4* shD;  // direction.xyz, path id

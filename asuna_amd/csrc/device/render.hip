@@ -552,6 +552,13 @@ __device__ __forceinline__ uint32_t findUnit(const WorkUnit* u, uint32_t n, uint
   return lo;
 }
 
+// The closest hit of a queue slot.
+__device__ __forceinline__ void writeHit(const Wavefront& w, uint32_t i, int inst, int leaf, float t, float u, float v) {
+  w.hit[i] = make_int4(inst, leaf, __float_as_int(u), __float_as_int(v));
+  w.hitT[i] = t;
+}
+__device__ __forceinline__ void writeMiss(const Wavefront& w, uint32_t i) { w.hit[i] = make_int4(-1, -1, 0, 0); }
+
 // Pixel of position k of a film's pixel order: 8x8 tiles in row-major
 // order over the largest multiple-of-8 rectangle, then the right strip and
 // the bottom strip row by row.  Work units are runs of this order, so a
@@ -733,11 +740,9 @@ __global__ __launch_bounds__(kTraceBlock) void kExtend(SceneView sc, Wavefront w
       int pos = TREE ? traceClosest4<COUNT, TREE == 2>(sc, r, kMinimum, kInf, st, t, u, v, nNodes, nTris)
                      : traceClosest<COUNT>(sc, r, kMinimum, kInf, st, t, u, v, nNodes, nTris);
       if (pos >= 0) {
-        const float4* tp = sc.tris + size_t(pos) * 3;
-        w.hitF[i] = make_float4(t, u, v, 0.f);
-        w.hitI[i] = make_int4(__float_as_int(tp[0].w), __float_as_int(tp[1].w), __float_as_int(tp[2].w), pos);
+        writeHit(w, i, __float_as_int(sc.tris[size_t(pos) * 3].w), pos, t, u, v);
       } else {
-        w.hitI[i] = make_int4(-1, -1, -1, -1);
+        writeMiss(w, i);
       }
     }
   }
@@ -893,11 +898,9 @@ __device__ __forceinline__ void extendDynLoop(const SceneView& sc, const Wavefro
     if (active && dynRound<COUNT>(sc, r, s, st, nNodes, nTris)) {
       active = false;
       if (s.best >= 0) {
-        const float4* tp = sc.tris + size_t(s.best) * 3;
-        w.hitF[slot] = make_float4(s.bt, s.bu, s.bv, 0.f);
-        w.hitI[slot] = make_int4(__float_as_int(tp[0].w), __float_as_int(tp[1].w), __float_as_int(tp[2].w), s.best);
+        writeHit(w, slot, __float_as_int(sc.tris[size_t(s.best) * 3].w), s.best, s.bt, s.bu, s.bv);
       } else {
-        w.hitI[slot] = make_int4(-1, -1, -1, -1);
+        writeMiss(w, slot);
       }
     }
   }
@@ -1209,11 +1212,9 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(8, 
       packetWalk<COUNT, false>(sc, w, r, q, valid, lane, gt, cap, sRef[wv], sT[wv], best, bt, bu, bv, nN, nT);
     if (valid) {
       if (best >= 0) {
-        const float4* tp = sc.tris + size_t(best) * 3;
-        w.hitF[i] = make_float4(bt, bu, bv, 0.f);
-        w.hitI[i] = make_int4(__float_as_int(tp[0].w), __float_as_int(tp[1].w), __float_as_int(tp[2].w), best);
+        writeHit(w, i, __float_as_int(sc.tris[size_t(best) * 3].w), best, bt, bu, bv);
       } else {
-        w.hitI[i] = make_int4(-1, -1, -1, -1);
+        writeMiss(w, i);
       }
     }
    }
@@ -1477,18 +1478,16 @@ __device__ __forceinline__ bool round2L(const SceneView& sc, const TRay& rw, TRa
 __device__ __forceinline__ void write2LHit(const SceneView& sc, const Wavefront& w, uint32_t i, const TRay& rw, int inst,
                                            int pos, float t, float u, float v) {
   if (pos < 0) {
-    w.hitI[i] = make_int4(-1, -1, -1, -1);
+    writeMiss(w, i);
     return;
   }
   const DevBlas& bl = sc.blas[sc.instBlas[inst]];
   const DevInstance& in = sc.inst[inst];
   const float4* tp = bl.tris + size_t(pos) * 3;
-  const int prim = __float_as_int(tp[2].w);
   float t2, u2, v2;
   if (hitTri(rw, toWorld(in, tp[0]), toWorld(in, tp[1]), toWorld(in, tp[2]), kMinimum, kInf, t2, u2, v2))
     t = t2, u = u2, v = v2;
-  w.hitF[i] = make_float4(t, u, v, 0.f);
-  w.hitI[i] = make_int4(inst, int(in.shade), int(in.triBase) + prim, int(bl.shadeBase) + pos);
+  writeHit(w, i, inst, int(bl.shadeBase) + pos, t, u, v);
 }
 
 // Persistent closest-hit loop over queue `cur` with per-lane refill (idle
@@ -1910,11 +1909,9 @@ __global__ __launch_bounds__(kTraceBlock) void kExtendWide(SceneView sc, Wavefro
     if (active && stepClosest4<COUNT>(sc, s, st, nNodes, nTris)) {
       active = false;
       if (s.best >= 0) {
-        const float4* tp = sc.tris + size_t(s.best) * 3;
-        w.hitF[slot] = make_float4(s.bt, s.bu, s.bv, 0.f);
-        w.hitI[slot] = make_int4(__float_as_int(tp[0].w), __float_as_int(tp[1].w), __float_as_int(tp[2].w), s.best);
+        writeHit(w, slot, __float_as_int(sc.tris[size_t(s.best) * 3].w), s.best, s.bt, s.bu, s.bv);
       } else {
-        w.hitI[slot] = make_int4(-1, -1, -1, -1);
+        writeMiss(w, slot);
       }
     }
   }
@@ -1978,8 +1975,7 @@ struct Hit {
 // getHitState + configureShadingFrame, rchit_layouts.glsl:61-95.
 // `leaf`: the triangle's position in leaf order, whose shading record holds
 // the same vertex data as the mesh's index triple and vertices.
-// `shade`: the instance's shade word (emitter or material id), carried by
-// the hit so that the material can be fetched without the instance record.
+// `shade`: the instance's shade word (emitter or material id).
 __device__ __forceinline__ void hitState(const SceneView& sc, int inst, uint32_t shade, int leaf, float bu, float bv,
                                          f3 rayDir, uint32_t useFaceNormal, Hit& h) {
   const DevInstance& in = sc.inst[inst];
@@ -3249,7 +3245,7 @@ __device__ __forceinline__ void shadeOne(const SceneView& sc, const BatchDesc& b
     c.fromDielectric = false;
     c.preEnv = false;
     c.Ld = mk1(0.f);
-    int4 hi = w.hitI[slot];
+    const int4 hi = w.hit[slot];
     uint32_t pix = info.z;
     bool frame0 = (info.w >> 16) & 1u;
     if (hi.x < 0) {
@@ -3272,7 +3268,7 @@ __device__ __forceinline__ void shadeOne(const SceneView& sc, const BatchDesc& b
       // With an env map, the env branch of that sample depends on nothing
       // but those draws, so it is taken here; sampleLights uses it only if
       // its selection draw starts from the same seed.
-      const uint32_t sw = uint32_t(hi.y);
+      const uint32_t sw = sc.inst[hi.x].shade;
       if (!(sw & kShadeLight) && sc.hasEnv && pc.hasEnvMap == 1 && sc.sky->inUse != 1) {
         const uint32_t t = (sw >> kShadeTypeShift) & kShadeTypeMask;
         uint32_t s = c.seed;
@@ -3286,11 +3282,10 @@ __device__ __forceinline__ void shadeOne(const SceneView& sc, const BatchDesc& b
           c.preEnv = true;
         }
       }
-      float4 hf = w.hitF[slot];
       Hit h;
-      hitState(sc, hi.x, uint32_t(hi.y), hi.w, hf.y, hf.z, c.rd, pc.useFaceNormal, h);
+      hitState(sc, hi.x, sw, hi.y, __int_as_float(hi.z), __int_as_float(hi.w), c.rd, pc.useFaceNormal, h);
       bool aov = frame0 && c.depth == 1;
-      if (aov && sp.depthChannel >= 0) writeAov(c, sp.depthChannel, mk1(hf.x), pix);
+      if (aov && sp.depthChannel >= 0) writeAov(c, sp.depthChannel, mk1(w.hitT[slot]), pix);
       if (h.lightId >= 0) {
         c.ro = xyz(w.rayO[cur][slot]);
         hitLight(c, h.lightId, h.pos);
@@ -3380,10 +3375,10 @@ __global__ __launch_bounds__(kShadeBlock) void kShade(SceneView sc, BatchDesc b,
   bool side = false;
   uint32_t key = kShadeKeys - 1;
   if (valid) {
-    int2 hi = *reinterpret_cast<const int2*>(&w.hitI[i]);  // the hit carries its instance's shade word
-    const uint32_t sw = uint32_t(hi.y);
-    side = hi.x >= 0 && (sw & kShadeSide);
-    key = hi.x < 0 ? 0u : (sw & kShadeLight) ? 1u : 2u + ((sw >> kShadeTypeShift) & kShadeTypeMask);
+    const int inst = w.hit[i].x;
+    const uint32_t sw = inst < 0 ? 0u : sc.inst[inst].shade;
+    side = sw & kShadeSide;
+    key = inst < 0 ? 0u : (sw & kShadeLight) ? 1u : 2u + ((sw >> kShadeTypeShift) & kShadeTypeMask);
     if (side || key >= uint32_t(kShadeKeys - 1)) key = kShadeKeys - 1;
   }
   int si = waveAppend(&w.ctr[8], side);
@@ -3509,7 +3504,7 @@ __global__ __launch_bounds__(256) void kFirstHitState(SceneView sc, const ShotPa
                                                       uint32_t P) {
   uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= P) return;
-  int4 hi = w.hitI[p];  // slot p of queue 0 after raygen is path p
+  const int4 hi = w.hit[p];  // slot p of queue 0 after raygen is path p
   ash_hit o;
   if (hi.x < 0) {
     o.t = kInf;
@@ -3518,14 +3513,19 @@ __global__ __launch_bounds__(256) void kFirstHitState(SceneView sc, const ShotPa
     o.prim_id = -1;
     for (int k = 0; k < 3; ++k) o.normal[k] = 0.f, o.pos[k] = 0.f;
   } else {
-    float4 hf = w.hitF[p];
+    const float u = __int_as_float(hi.z), v = __int_as_float(hi.w);
     Hit h;
-    hitState(sc, hi.x, uint32_t(hi.y), hi.w, hf.y, hf.z, xyz(w.rayD[0][p]), 0u, h);
-    o.t = hf.x;
-    o.u = hf.y;
-    o.v = hf.z;
+    hitState(sc, hi.x, sc.inst[hi.x].shade, hi.y, u, v, xyz(w.rayD[0][p]), 0u, h);
+    o.t = w.hitT[p];
+    o.u = u;
+    o.v = v;
     o.inst_id = hi.x;
-    o.prim_id = hi.z - int(sc.inst[hi.x].triBase);  // global id minus the instance's first triangle
+    if (sc.twoLevel) {
+      const DevBlas& bl = sc.blas[sc.instBlas[hi.x]];  // its triangles carry the mesh's own numbers
+      o.prim_id = __float_as_int(bl.tris[(size_t(hi.y) - bl.shadeBase) * 3 + 2].w);
+    } else {  // global id minus the instance's first triangle
+      o.prim_id = __float_as_int(sc.tris[size_t(hi.y) * 3 + 2].w) - int(sc.inst[hi.x].triBase);
+    }
     o.normal[0] = h.N.x, o.normal[1] = h.N.y, o.normal[2] = h.N.z;
     o.pos[0] = h.pos.x, o.pos[1] = h.pos.y, o.pos[2] = h.pos.z;
   }
