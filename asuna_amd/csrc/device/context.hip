@@ -114,8 +114,10 @@ struct ash_ctx {
   uint32_t shotCount = 0, shotW = 0, shotH = 0;
   // wavefront
   Wavefront wf{};
-  DBuf<float4> wRayO0, wRayO1, wRayD0, wRayD1, wThr0, wThr1, wRad, wLd, wShO, wShD;
-  DBuf<uint4> wInfo0, wInfo1;
+  DBuf<float4> wRayD0, wRayD1, wThr0, wThr1, wRad, wShO, wShD;
+  DBuf<f3> wRayO0, wRayO1, wLd;
+  DBuf<uint2> wRng0, wRng1, wOrigin;
+  DBuf<uint32_t> wShot0, wShot1;
   DBuf<int4> wHit;
   DBuf<float> wHitT;
   DBuf<int> wSide, wSpill;
@@ -156,11 +158,12 @@ struct ash_ctx {
     if (tris) (void)hipFree(tris);
     if (shadeTris) (void)hipFree(shadeTris);
     for (auto& t : texData) t.release();
-    for (auto* b : {&verts, &env, &images, &shotImages, &wRayO0, &wRayO1, &wRayD0, &wRayD1, &wThr0, &wThr1, &wRad, &wLd,
+    for (auto* b : {&verts, &env, &images, &shotImages, &wRayD0, &wRayD1, &wThr0, &wThr1, &wRad,
                     &wShO, &wShD})
       b->release();
     inst.release(), idx.release(), instTriOffset.release(), mats.release(), lights.release(), texTab.release();
-    marg.release(), condX.release(), shotTab.release(), wInfo0.release(), wInfo1.release(), wHit.release(), wHitT.release();
+    marg.release(), condX.release(), shotTab.release(), wRng0.release(), wRng1.release(), wOrigin.release(),
+        wShot0.release(), wShot1.release(), wRayO0.release(), wRayO1.release(), wLd.release(), wHit.release(), wHitT.release();
     wSide.release(), wSpill.release(), wSpillT.release(), wCtr.release(), wCnt64.release();
     unitBuf.release(), sky.release();
     for (auto& g : graphs) releaseGraph(g);
@@ -264,8 +267,11 @@ static int ensureWavefront(ash_ctx* c, uint32_t cap) {
   MALLOC(c, c->wLd, cap);
   MALLOC(c, c->wShO, cap);
   MALLOC(c, c->wShD, cap);
-  MALLOC(c, c->wInfo0, cap);
-  MALLOC(c, c->wInfo1, cap);
+  MALLOC(c, c->wRng0, cap);
+  MALLOC(c, c->wRng1, cap);
+  MALLOC(c, c->wOrigin, cap);
+  MALLOC(c, c->wShot0, cap);
+  MALLOC(c, c->wShot1, cap);
   MALLOC(c, c->wHit, cap);
   MALLOC(c, c->wHitT, cap);
   MALLOC(c, c->wSide, cap);
@@ -281,8 +287,11 @@ static int ensureWavefront(ash_ctx* c, uint32_t cap) {
   w.thr[1] = c->wThr1.p;
   w.rad = c->wRad.p;
   w.ld = c->wLd.p;
-  w.info[0] = c->wInfo0.p;
-  w.info[1] = c->wInfo1.p;
+  w.rng[0] = c->wRng0.p;
+  w.rng[1] = c->wRng1.p;
+  w.origin = c->wOrigin.p;
+  w.shot[0] = c->wShot0.p;
+  w.shot[1] = c->wShot1.p;
   w.hit = c->wHit.p;
   w.hitT = c->wHitT.p;
   w.side = c->wSide.p;
@@ -1059,15 +1068,19 @@ static size_t noAllocLayout(unsigned char* base, uint32_t threads, uint32_t cap,
   std::memset(&w, 0, sizeof w);
   w.capacity = kNoAllocPaths;
   for (int q = 0; q < 2; ++q) {
-    w.rayO[q] = reinterpret_cast<float4*>(take(n * sizeof(float4)));
+    w.rayO[q] = reinterpret_cast<f3*>(take(n * sizeof(f3)));
     w.rayD[q] = reinterpret_cast<float4*>(take(n * sizeof(float4)));
   }
   for (int q = 0; q < 2; ++q) w.thr[q] = reinterpret_cast<float4*>(take(n * sizeof(float4)));
   w.rad = reinterpret_cast<float4*>(take(n * sizeof(float4)));
-  w.ld = reinterpret_cast<float4*>(take(n * sizeof(float4)));
+  w.ld = reinterpret_cast<f3*>(take(n * sizeof(f3)));
   w.shO = reinterpret_cast<float4*>(take(n * sizeof(float4)));
   w.shD = reinterpret_cast<float4*>(take(n * sizeof(float4)));
-  for (int q = 0; q < 2; ++q) w.info[q] = reinterpret_cast<uint4*>(take(n * sizeof(uint4)));
+  for (int q = 0; q < 2; ++q) {
+    w.rng[q] = reinterpret_cast<uint2*>(take(n * sizeof(uint2)));
+    w.shot[q] = reinterpret_cast<uint32_t*>(take(n * sizeof(uint32_t)));
+  }
+  w.origin = reinterpret_cast<uint2*>(take(n * sizeof(uint2)));
   w.hit = reinterpret_cast<int4*>(take(n * sizeof(int4)));
   w.hitT = reinterpret_cast<float*>(take(n * sizeof(float)));
   w.side = reinterpret_cast<int*>(take(n * sizeof(int)));

@@ -69,15 +69,20 @@ struct SceneView {
 // there); its ray, throughput and RNG / pixel record, and the hit of its
 // ray, live in the slot order of the extension queue that holds it, so that
 // traversal and shading read and write them in runs (the queue after
-// raygen is the identity: slot = path id).
+// raygen is the identity: slot = path id).  What stays the same along a path
+// is kept by path id, and read at first hits only: a continuing path writes 52
+// bytes (56 in batches of several shots) in place of 64, a shadow ray 44 in
+// place of 48 (512 x 512 box, 64 spp: 11.97 -> 11.86 ms).
 struct Wavefront {
   uint32_t capacity;
-  float4* rayO[2];  // extension queues (alternating): ray origin.xyz per slot
+  f3* rayO[2];      // extension queues (alternating): ray origin per slot
   float4* rayD[2];  // ray direction.xyz, w = path id
   float4* thr[2];   // throughput.xyz, w = pdf of the last BSDF sample (read only at depth > 1)
-  uint4* info[2];   // x seed, y depth | bsdfFlags << 16, z pixel, w shot | (frame == 0) << 16
+  uint2* rng[2];       // x seed, y depth | bsdfFlags << 16
+  uint32_t* shot[2];   // batches of several shots: the path's shot (written from the first bounce on)
+  uint2* origin;       // by path id: x pixel, y shot | (frame == 0) << 16
   float4* rad;   // by path id: radiance.xyz, w = Gaussian filter weight
-  float4* ld;    // pending NEE radiance of the current bounce, per shadow-ray slot
+  f3* ld;        // pending NEE radiance of the current bounce, per shadow-ray slot
   int4* hit;     // per slot of the queue being traced: instance (-1 miss), leaf position, u, v
   float* hitT;   // its distance, which only the depth channel and the first-hit query read
   int* side;     // second-group shading queue: slots of the current extension queue
