@@ -1300,6 +1300,12 @@ struct ConvPlan {
   ConvKind kind;
   uint32_t tilesX, tilesY, tiles;  // tiles = N tilesX tilesY
 };
+// The larger a block's tile, the less it reads per product, so the largest that gives every CU a block is taken: waiting
+// for two blocks a CU costs 1024 -> 984 us at 1920 x 1080, 403 -> 367 at 960 x 540 and 265 -> 239 at 640 x 360 (two
+// blocks -> one).  16 x 16 pixels by two output groups before 16 x 32 by one: without it 984 -> 1086 us.  8 rows are for
+// images the 16-row tiles leave CUs idle at: taken for the finest level of 1920 x 1080 instead they cost 1033 -> 1180 us.
+// Below one such block a CU the input channels are split over a block's waves: with 8-row tiles from half a block a CU on,
+// 1920 x 1080 goes 984 -> 997 us and 480 x 270 166 -> 183.  (Whole passes, before the first and last pairs were fused.)
 static ConvPlan convPlan(const ash_denoiser* d, uint32_t N, uint32_t H, uint32_t W, uint32_t nCg) {
   auto make = [&](ConvKind k, uint32_t tr, uint32_t tc) {
     ConvPlan p{k, (W + tc - 1) / tc, (H + tr - 1) / tr, 0};
@@ -1332,9 +1338,9 @@ static void launchConv(const ash_denoiser* d, const ConvArgs& a, const ConvPlan&
     kConvSplit<MODE><<<p.tiles * a.nCg, 64 * a.nCh, lds, d->stream>>>(a, p.tilesX, p.tilesY);
   } else if (p.kind == kKind4) {
     convLds<4, 1, NT, MODE>(d, a, p);
-  } else if (p.kind == kKind8 || MODE == kModeLast) {
+  } else if (p.kind == kKind8) {
     convLds<8, 1, NT, MODE>(d, a, p);
-  } else {
+  } else if constexpr (MODE != kModeLast) {  // that layer has one output group
     convLds<8, 2, NT, MODE>(d, a, p);
   }
 }
@@ -1440,7 +1446,9 @@ static int trainForward(ash_denoiser* d) {
 
 // Pixel tiles of a layer's weight gradient: 32, 16 or 8 columns by the
 // image's width, kBwdWTiles of them per block (fewer partial sums to write and
-// add than with a block per tile, more blocks than with one per CU).
+// add than with a block per tile, more blocks than with one per CU).  2, 4 and
+// 8 a block: 3.62, 3.45 and 3.42 ms for 4 steps on 8 crops of 128 x 128, 680,
+// 684 and 707 us for a gradient of 2 images of 80 x 48.
 constexpr uint32_t kBwdWTiles = 4;
 static void bwdWPlan(const Layer& l, uint32_t N, uint32_t H, uint32_t W, BwdWLayer& p) {
   p.tc = uint16_t(W > 16 ? 32 : W > 8 ? 16 : 8);
