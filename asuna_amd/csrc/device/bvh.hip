@@ -80,7 +80,7 @@ __global__ void kWorldTris(BuildArgs a, float4* wtri, float4* boxLo, float4* box
     p[k] = xform(in.o2w, a.vertices[2 * size_t(vi)]);
   }
   wtri[3 * size_t(g) + 0] = make_float4(p[0].x, p[0].y, p[0].z, __int_as_float(int(lo)));
-  wtri[3 * size_t(g) + 1] = make_float4(p[1].x, p[1].y, p[1].z, __uint_as_float(in.shade));
+  wtri[3 * size_t(g) + 1] = make_float4(p[1].x, p[1].y, p[1].z, 0.f);
   wtri[3 * size_t(g) + 2] = make_float4(p[2].x, p[2].y, p[2].z, __int_as_float(int(g)));
   boxLo[g] = make_float4(fminf(p[0].x, fminf(p[1].x, p[2].x)), fminf(p[0].y, fminf(p[1].y, p[2].y)),
                          fminf(p[0].z, fminf(p[1].z, p[2].z)), 0.f);

@@ -7,7 +7,7 @@
 //                                           node: lo.x[4] hi.x[4] lo.y[4] hi.y[4] lo.z[4] hi.z[4]
 //                                           child refs[4], unused[4]
 //   tris       float4[3*numTris]           world-space v0,v1,v2 in leaf order (48 B/tri);
-//                                           .w of v0/v1/v2 = instance, shade word, global id
+//                                           .w of v0/v1/v2 = instance, unused, global id
 //   materials  GpuMaterial[], lights GpuLight[], textures (RGBA32F), env + tables
 #pragma once
 
@@ -27,7 +27,7 @@ struct DevInstance {
   int32_t light;      // light id, -1 if not an emitter
   uint32_t triBase;   // global id of the instance's first triangle
   uint32_t ntri;
-  uint32_t shade;     // shade word, carried by each triangle record into the hit buffer
+  uint32_t shade;     // shade word: material or emitter id, material type, group
   uint32_t pad;
 };
 // Shade word of an instance: bit 31 = surface of the second shading group,
@@ -67,7 +67,7 @@ __host__ __device__ inline void decodeLeaf(int32_t ref, uint32_t& first, uint32_
 constexpr int32_t kEmptyRef = int32_t(0x7fffffff);
 
 // Two-level acceleration (instancing without duplication): one object-space
-// BVH (BLAS) per distinct mesh, shared by all its instances, under a binary
+// BVH (BLAS) per distinct mesh, shared by all its instances, under a
 // tree over the instances' world boxes (TLAS).  A BLAS triangle record keeps
 // the mesh-local primitive in v2.w; the instance, its shade word and its
 // global triangle ids come from the instance walked.

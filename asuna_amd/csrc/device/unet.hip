@@ -1305,7 +1305,7 @@ struct ConvPlan {
 // blocks -> one).  16 x 16 pixels by two output groups before 16 x 32 by one: without it 984 -> 1086 us.  8 rows are for
 // images the 16-row tiles leave CUs idle at: taken for the finest level of 1920 x 1080 instead they cost 1033 -> 1180 us.
 // Below one such block a CU the input channels are split over a block's waves: with 8-row tiles from half a block a CU on,
-// 1920 x 1080 goes 984 -> 997 us and 480 x 270 166 -> 183.  (Whole passes, before the first and last pairs were fused.)
+// 1920 x 1080 goes 984 -> 997 us and 317 x 179 166 -> 183.  (Whole passes, before the first and last pairs were fused.)
 static ConvPlan convPlan(const ash_denoiser* d, uint32_t N, uint32_t H, uint32_t W, uint32_t nCg) {
   auto make = [&](ConvKind k, uint32_t tr, uint32_t tc) {
     ConvPlan p{k, (W + tc - 1) / tc, (H + tr - 1) / tr, 0};

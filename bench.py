@@ -25,8 +25,8 @@ Prints one JSON line:
                VALU issue and lane utilisation of the same dispatches.  The
                algorithmic bytes per launch (node visits x node bytes: 64 B for
                the quantized 4-wide node, 112 B for the float 4-wide node, 64 B
-               binary; + triangle tests x 48 B + ray I/O, 68 B per extension
-               ray, 48 B per shadow ray; counted in a calibration render of the
+               binary; + triangle tests x 48 B + ray I/O, 48 B per extension
+               ray, 44 B per shadow ray; counted in a calibration render of the
                same batches) are reported as algorithmic_bytes: the L2 and the
                MALL serve most of them, so over the launch time they exceed the
                HBM peak
@@ -50,10 +50,12 @@ HBM_PEAK_GBS = 8000.0
 # bytes a node visit reads: binary node 64 B; float 4-wide node 7 x 16 B (6
 # box planes + child refs) of its 128 B line; quantized 4-wide node 64 B
 NODE_BYTES = {(2, 64): 64, (4, 128): 112, (4, 64): 64}
-TRI_BYTES, RAY_IO_BYTES = 48, 68
+TRI_BYTES = 48
+# extension ray I/O: origin, direction+path id; the hit's record and distance
+RAY_IO_BYTES = 48
 L2_BYTES = 4 << 20  # L2 of one XCD
 # shadow ray I/O: origin+tmax, direction+path id, and the pending NEE radiance
-SHADOW_IO_BYTES = 48
+SHADOW_IO_BYTES = 44
 # counters of the in-run pass: L2-to-memory (EA) read and write requests by
 # size, VALU issue and lane activity, GPU cycles (within one pass's limits:
 # 4 TCC, 4 SQ, 1 GRBM)
