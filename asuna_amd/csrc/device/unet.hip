@@ -42,6 +42,7 @@
 
 #include "../../../include/asuna_denoise.h"
 #include "ctx_internal.h"
+#include "log1p.h"
 
 namespace {
 
@@ -462,37 +463,12 @@ struct PairArgs {
 constexpr uint32_t kPairRows = 14, kPairCols = 30, kPairPitch = 34, kPairPix = 18 * kPairPitch;
 constexpr size_t kPairLds = size_t(kPairPix) * 64 + 2 * 18 * 1024;
 
-// log(1 + x) for x >= 0 (or infinity), to 2 units in the last place: the
-// rounding error of u = 1 + x is carried as c / u, u = 2^k m with m around 1, and
-// log m = 2 atanh(s), s = (m - 1) / (m + 1), by the series to s^11 (|s| <= 0.1716:
-// the rest is below 4e-11).  30 instructions; the library's 120 were a third of
-// the first pair's time.  After the features' BF16 rounding 1 in 100,000 differs
-// from the rounded exact value, and their RMS error against 64 bits (1.66e-3) is
-// the library's to 9 digits, for x from 1e-13 to 1e34.
-__device__ __forceinline__ float log1pPos(float x) {
-  const float u = 1.0f + x, c = x - (u - 1.0f);
-  uint32_t bits = __float_as_uint(u);
-  int k = int(bits >> 23) - 127;
-  float m = __uint_as_float((bits & 0x7fffffu) | 0x3f800000u);
-  const bool high = m > 1.41421356f;
-  m = high ? 0.5f * m : m;
-  const float kf = float(high ? k + 1 : k);
-  const float f = m - 1.0f, d = m + 1.0f;
-  const float r = __builtin_amdgcn_rcpf(d), s0 = f * r, s = fmaf(fmaf(-s0, d, f), r, s0);
-  const float z = s * s;
-  const float p = z * fmaf(z, fmaf(z, fmaf(z, fmaf(z, 1.0f / 11, 1.0f / 9), 1.0f / 7), 1.0f / 5), 1.0f / 3);
-  const float lo = fmaf(kf, -1.90465421e-09f, c * __builtin_amdgcn_rcpf(u));  // k (ln 2 - its 24-bit value) + c / u
-  const float s2 = 2.0f * s;
-  const float l = fmaf(kf, 0.693147182f, s2 + fmaf(s2, p, lo));
-  return x > 3.0e38f ? x : l;
-}
-
 // The network's ten input features of a pixel.
 __device__ __forceinline__ void featuresOf(const float (&v)[10], bf16x8& lo, bf16x8& hi) {
   lo = hi = zero8();
 #pragma unroll
   for (int c = 0; c < 10; ++c) {
-    const float f = c < 3 || c == 9 ? log1pPos(fmaxf(v[c], 0.f)) : v[c];
+    const float f = c < 3 || c == 9 ? ashd::log1pPos(fmaxf(v[c], 0.f), [](float d) { return __builtin_amdgcn_rcpf(d); }) : v[c];
     if (c < 8) lo[c] = bf16(f);
     else hi[c - 8] = bf16(f);
   }

@@ -7,6 +7,7 @@ similarity >= 0.98 and relative L2 error <= 0.15 (BF16 activations and
 operands); the film path equals the host path bit for bit; after training
 on renders, the denoised 4-spp image has lower relMSE against a 1024-spp
 render than the 4-spp input on held-out views."""
+import ctypes as C
 import os
 
 import numpy as np
@@ -292,4 +293,45 @@ def test_large_batch_equals_its_images():
     log(f"batch of {n}: forward {ferr:.5f}, gradient {gerr:.5f}")
     assert ferr <= 0.01 and gerr <= 0.01
     assert abs(loss - np.mean([p[0] for p in parts])) <= 1e-4 * loss
+    d.close()
+
+
+def test_features_of_any_magnitude_reach_the_network():
+    """Weights that hand the radiance features through every full-resolution
+    layer unchanged: the output is expm1 of the BF16 rounding of log(1 + x), for x
+    from 1e-36 to the largest finite number, in both feature kernels.  log(1 + x) is
+    within 0.54 units of its last place, which rounds to the other BF16 neighbour
+    for at most 2 x 0.54 / 2^16 of the values; bar 3 times that."""
+    theta = np.zeros(U.num_params(), np.float32)
+    k = 0
+    for name, a, b, o, relu in U.layer_shapes():
+        n = 9 * (a + b) * o
+        if name in ("enc0a", "enc0b", "dec0a", "dec0b", "out"):
+            W = theta[k:k + n].reshape(9, o, a + b)
+            for c in range(3):
+                W[4, c, (a if name == "dec0a" else 0) + c] = 1.0  # dec0a: from the skip tensor
+        k += n + o
+    d = A.Denoiser(0)
+    d.set_params(theta)
+    h = w = 256
+    x = np.zeros((1, h, w, 10), np.float32)
+    x[..., :3] = np.geomspace(1e-36, np.finfo(np.float32).max, 3 * h * w).astype(np.float32).reshape(1, h, w, 3)
+    x[0, 0, 0, :3] = (0.0, 3.0e38, np.finfo(np.float32).max)
+    out = d.forward(x)
+    got = bf16(np.log1p(out.astype(np.float64)).astype(np.float32))[0]
+    want = bf16(np.log1p(x[0, ..., :3].astype(np.float64)).astype(np.float32))
+    assert np.isfinite(out).all()
+    differ = got != want
+    log(f"features: {int(differ.sum())} of {differ.size} round to the other BF16 neighbour")
+    assert differ.mean() <= 3 * 2 * 0.54 / 2 ** 16
+    np.testing.assert_allclose(got, want, rtol=2.0 ** -7)
+    # and from a film's planes
+    r = A.Renderer(0)
+    r.set_film(w, h)
+    rad = np.concatenate([x[0, ..., :3], np.ones((h, w, 1), np.float32)], -1)
+    src, dst = r.output_device_ptr(0), r.output_device_ptr(7)
+    assert C.CDLL("libamdhip64.so").hipMemcpy(C.c_void_p(src), C.c_void_p(rad.ctypes.data), C.c_size_t(rad.nbytes), 1) == 0
+    d._check(A.lib().ash_denoise_planes(d._d, src, None, None, None, w, h, dst, C.byref(C.c_double())), "denoise_planes")
+    np.testing.assert_array_equal(r.read(7)[..., :3], out[0])
+    r.close()
     d.close()
