@@ -228,9 +228,19 @@ __device__ __forceinline__ float halfArea(float4 lo, float4 hi) {
 // A build of 1 M triangles with its first hits took 19.0 ms with one host round
 // trip and six launches per round, a level walk, one refit launch per level and
 // its temporaries allocated one by one; it takes 5.1 (2.4 in kernels).
+//
+// Rounds are bounded.  Among clusters of equal cost (coincident or zero-extent
+// triangles) every one prefers the smallest index, so a round merges one pair of
+// them and the tree below is a chain; from round kPlocPair on, equal costs prefer
+// the neighbour g ^ 1, which is mutual and halves such a run.  Clusters that still
+// take more than kPlocMaxRounds (boxes nested in one another, each nearest to the
+// next smaller one) get the radix tree of their keys instead.  A tree of so many
+// rounds has no more levels, which the 4-wide collapse takes in any shape.
 constexpr int kPlocRadius = 16;
 constexpr uint32_t kPlocTail = 1024;
 constexpr int kPlocRounds = 4;
+constexpr uint32_t kMaxLevels4 = 200;  // of the 4-wide tree
+constexpr uint32_t kPlocPair = 96, kPlocMaxRounds = kMaxLevels4;
 
 struct PlocTree {
   int *left, *right, *parent, *leafParent;
@@ -279,7 +289,8 @@ __device__ __forceinline__ void plocMerge(const PlocTree& T, int id, int c0, flo
 }
 
 // The best partner of cluster g among [j0, j1] (boxes at sl / sh, index j - base).
-__device__ __forceinline__ int plocNearest(const float4* sl, const float4* sh, int g, int j0, int j1, int base) {
+// Equal costs: the smallest index, or (pairs) g ^ 1 where it is one of them.
+__device__ __forceinline__ int plocNearest(const float4* sl, const float4* sh, int g, int j0, int j1, int base, bool pairs) {
   const float4 a = sl[g - base], b = sh[g - base];
   float best = FLT_MAX;
   int bj = -1;
@@ -289,7 +300,7 @@ __device__ __forceinline__ int plocNearest(const float4* sl, const float4* sh, i
     const float4 lo = make_float4(fminf(a.x, c.x), fminf(a.y, c.y), fminf(a.z, c.z), 0.f);
     const float4 hi = make_float4(fmaxf(b.x, d.x), fmaxf(b.y, d.y), fmaxf(b.z, d.z), 0.f);
     const float cost = halfArea(lo, hi);
-    if (cost < best) best = cost, bj = j;  // ascending j: ties keep the smaller index
+    if (cost < best || (pairs && cost == best && j == (g ^ 1))) best = cost, bj = j;  // ascending j
   }
   return bj;
 }
@@ -315,7 +326,7 @@ __device__ __forceinline__ uint32_t blockRank(bool f, uint32_t* sh, uint32_t& to
 // partners; survivors per block go to tileSums for the compaction.
 __global__ __launch_bounds__(kBlock) void kPlocStep(PlocTree T, const uint32_t* count, const int* cNode, const float4* cLo,
                                                     const float4* cHi, int* oNode, float4* oLo, float4* oHi,
-                                                    uint8_t* valid, uint32_t* tileSums, unsigned* idCounter) {
+                                                    uint8_t* valid, uint32_t* tileSums, unsigned* idCounter, bool pairs) {
   constexpr int kHalo = 2 * kPlocRadius, kBoxes = kBlock + 2 * kHalo, kNear = kBlock + 2 * kPlocRadius;
   __shared__ float4 sl[kBoxes], sh[kBoxes];
   __shared__ int sn[kNear];
@@ -330,7 +341,7 @@ __global__ __launch_bounds__(kBlock) void kPlocStep(PlocTree T, const uint32_t* 
   __syncthreads();
   for (int k = int(threadIdx.x); k < kNear; k += kBlock) {
     const int g = first - kPlocRadius + k;
-    if (g >= 0 && g < m) sn[k] = plocNearest(sl, sh, g, max(0, g - kPlocRadius), min(m - 1, g + kPlocRadius), base);
+    if (g >= 0 && g < m) sn[k] = plocNearest(sl, sh, g, max(0, g - kPlocRadius), min(m - 1, g + kPlocRadius), base, pairs);
   }
   __syncthreads();
   const int i = first + int(threadIdx.x);
@@ -408,9 +419,11 @@ __global__ __launch_bounds__(kBlock) void kPlocCompact(const uint32_t* count, co
 
 // The rounds from at most kPlocTail clusters to one, in one block: a thread
 // per cluster, boxes and partners in LDS.  Ends when a round merges nothing
-// (one cluster, or boxes no cost compares below).
+// (one cluster, or boxes no cost compares below: *stalled) and after round
+// kPlocMaxRounds; `round` have been done before.
 __global__ __launch_bounds__(kPlocTail) void kPlocTailRounds(PlocTree T, uint32_t* count, const int* cNode, const float4* cLo,
-                                                             const float4* cHi, unsigned* idCounter) {
+                                                             const float4* cHi, unsigned* idCounter, uint32_t round,
+                                                             uint32_t* stalled) {
   __shared__ float4 sl[kPlocTail], sh[kPlocTail];
   __shared__ int sNode[kPlocTail], sn[kPlocTail];
   __shared__ uint32_t sw[kPlocTail / 64];
@@ -420,8 +433,8 @@ __global__ __launch_bounds__(kPlocTail) void kPlocTailRounds(PlocTree T, uint32_
   unsigned used = *idCounter;
   if (i < m) sl[i] = cLo[i], sh[i] = cHi[i], sNode[i] = cNode[i];
   __syncthreads();
-  while (m > 1) {
-    if (i < m) sn[i] = plocNearest(sl, sh, i, max(0, i - kPlocRadius), min(m - 1, i + kPlocRadius), 0);
+  for (; m > 1 && round < kPlocMaxRounds; ++round) {
+    if (i < m) sn[i] = plocNearest(sl, sh, i, max(0, i - kPlocRadius), min(m - 1, i + kPlocRadius), 0, round >= kPlocPair);
     __syncthreads();
     int j = -1;
     bool mutual = false;
@@ -447,7 +460,10 @@ __global__ __launch_bounds__(kPlocTail) void kPlocTailRounds(PlocTree T, uint32_
     used += nMerges;
     m = int(nStays);
     __syncthreads();
-    if (!nMerges) break;
+    if (!nMerges) {
+      if (i == 0) *stalled = 1;
+      break;
+    }
   }
   if (i == 0) *count = uint32_t(m), *idCounter = used;
 }
@@ -1079,7 +1095,8 @@ int buildBvh(const BuildArgs& a, hipStream_t s, BuildResult& r, char* err, size_
     HIPB(A.status);
     HIPB(hipMemsetAsync(maxLevel.p, 0, sizeof(unsigned), s));
     unsigned gi = (nInternal + kBlock - 1) / kBlock;
-    if (a.quality == 2) {
+    bool radix = a.quality != 2;
+    if (!radix) {
       // PLOC hierarchy over the Morton order, then depth-first leaf order
       const size_t mark = A.used;
       DevBuf<int> cNode[2], leafParent2;
@@ -1088,23 +1105,24 @@ int buildBvh(const BuildArgs& a, hipStream_t s, BuildResult& r, char* err, size_
       DevBuf<uint8_t> valid;
       for (int b2 = 0; b2 < 2; ++b2) A.take(cNode[b2], nn), A.take(cLo[b2], nn), A.take(cHi[b2], nn);
       A.take(valid, nn), A.take(nodeCnt, ni), A.take(posOf, nn), A.take(sorted2, nn), A.take(leafParent2, nn);
-      A.take(tileSums, grid), A.take(cnt, 3);  // cnt: the cluster counts of this and the next round, the nodes made
+      A.take(tileSums, grid), A.take(cnt, 4);  // cnt: the cluster counts of this and the next round, the nodes made, the tail's stall
       HIPB(A.status);
-      HIPB(hipMemsetAsync(cnt.p, 0, 3 * sizeof(uint32_t), s));
+      HIPB(hipMemsetAsync(cnt.p, 0, 4 * sizeof(uint32_t), s));
       const PlocTree T{left.p, right.p, parent.p, leafParent.p, nodeCnt.p, nodeLo.p, nodeHi.p, cost.p, collapsed.p,
                        n, a.leafMax, a.quality};
       kPlocInit<<<grid, kBlock, 0, s>>>(n, ids2.p, boxLo.p, boxHi.p, cNode[0].p, cLo[0].p, cHi[0].p, cnt.p, parent.p);
-      uint32_t m = n, state[3] = {n, 0, 0};
-      static_assert(kPlocRounds % 2 == 0, "a batch of rounds ends on the first count");
-      while (m > 1) {
+      uint32_t m = n, rounds = 0, state[4] = {n, 0, 0, 0};
+      static_assert(kPlocRounds % 2 == 0 && kPlocMaxRounds % kPlocRounds == 0, "a batch of rounds ends on the first count");
+      while (m > 1 && !radix) {
         const unsigned gm = (m + kBlock - 1) / kBlock;
-        if (m <= kPlocTail) {
-          kPlocTailRounds<<<1, kPlocTail, 0, s>>>(T, cnt.p, cNode[0].p, cLo[0].p, cHi[0].p, cnt.p + 2);
+        const bool tail = m <= kPlocTail;
+        if (tail) {
+          kPlocTailRounds<<<1, kPlocTail, 0, s>>>(T, cnt.p, cNode[0].p, cLo[0].p, cHi[0].p, cnt.p + 2, rounds, cnt.p + 3);
         } else {
-          for (int r = 0; r < kPlocRounds; ++r) {
+          for (int r = 0; r < kPlocRounds; ++r, ++rounds) {
             uint32_t *now = cnt.p + r % 2, *next = cnt.p + 1 - r % 2;
             kPlocStep<<<gm, kBlock, 0, s>>>(T, now, cNode[0].p, cLo[0].p, cHi[0].p, cNode[1].p, cLo[1].p, cHi[1].p, valid.p,
-                                            tileSums.p, cnt.p + 2);
+                                            tileSums.p, cnt.p + 2, rounds >= kPlocPair);
             kPlocScan<<<1, 1024, 0, s>>>(now, tileSums.p, next);
             kPlocCompact<<<gm, kBlock, 0, s>>>(now, valid.p, tileSums.p, cNode[1].p, cLo[1].p, cHi[1].p, cNode[0].p, cLo[0].p,
                                                cHi[0].p);
@@ -1112,26 +1130,30 @@ int buildBvh(const BuildArgs& a, hipStream_t s, BuildResult& r, char* err, size_
         }
         HIPB(hipMemcpyAsync(state, cnt.p, sizeof state, hipMemcpyDeviceToHost, s));
         HIPB(hipStreamSynchronize(s));
-        // every round of comparable boxes merges at least the best pair, and the tail ends with one cluster
-        if (state[0] >= m || (m <= kPlocTail && state[0] != 1)) {
+        // every round of comparable boxes merges at least the best pair
+        if ((!tail && state[0] >= m) || state[3]) {
           std::snprintf(err, errLen, "bvh: clustering made no progress (%u clusters)", m);
           return ASH_E_INVALID;
         }
         m = state[0];
+        radix = m > 1 && (tail || rounds >= kPlocMaxRounds);
       }
-      if (state[2] != nInternal) {
-        std::snprintf(err, errLen, "bvh: clustering produced %u of %u internal nodes", state[2], nInternal);
-        return ASH_E_INVALID;
+      if (!radix) {
+        if (state[2] != nInternal) {
+          std::snprintf(err, errLen, "bvh: clustering produced %u of %u internal nodes", state[2], nInternal);
+          return ASH_E_INVALID;
+        }
+        kPlocLeafOrder<<<grid, kBlock, 0, s>>>(n, left.p, right.p, parent.p, leafParent.p, nodeCnt.p, ids2.p, posOf.p,
+                                               sorted2.p, leafParent2.p);
+        kPlocRanges<<<gi, kBlock, 0, s>>>(nInternal, left.p, posOf.p, nodeCnt.p, range.p);
+        kPlocRelabel<<<gi, kBlock, 0, s>>>(nInternal, left.p, right.p, posOf.p);
+        HIPB(hipMemcpyAsync(ids2.p, sorted2.p, nn * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
+        HIPB(hipMemcpyAsync(leafParent.p, leafParent2.p, nn * sizeof(int), hipMemcpyDeviceToDevice, s));
+        HIPB(hipGetLastError());
       }
-      kPlocLeafOrder<<<grid, kBlock, 0, s>>>(n, left.p, right.p, parent.p, leafParent.p, nodeCnt.p, ids2.p, posOf.p,
-                                             sorted2.p, leafParent2.p);
-      kPlocRanges<<<gi, kBlock, 0, s>>>(nInternal, left.p, posOf.p, nodeCnt.p, range.p);
-      kPlocRelabel<<<gi, kBlock, 0, s>>>(nInternal, left.p, right.p, posOf.p);
-      HIPB(hipMemcpyAsync(ids2.p, sorted2.p, nn * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
-      HIPB(hipMemcpyAsync(leafParent.p, leafParent2.p, nn * sizeof(int), hipMemcpyDeviceToDevice, s));
-      HIPB(hipGetLastError());
       A.used = mark;  // later takers are ordered after these kernels on the stream
-    } else {
+    }
+    if (radix) {
       kKarras<<<gi, kBlock, 0, s>>>(keys2.p, int(n), left.p, right.p, parent.p, leafParent.p, range.p);
       kNodeLevel<<<gi, kBlock, 0, s>>>(int(nInternal), parent.p, level.p, maxLevel.p);
       unsigned deepest = 0;
@@ -1201,13 +1223,13 @@ int buildBvh(const BuildArgs& a, hipStream_t s, BuildResult& r, char* err, size_
   if (a.branching == 4) {
     // one launch per level of the 4-wide tree; the host looks at the frontier sizes every kCollapseLevels levels,
     // with grids for four times the last one
-    constexpr uint32_t kCollapseLevels = 4, kMaxLevels = 200;
+    constexpr uint32_t kCollapseLevels = 4;
     DevBuf<int2> f[2];
     DevBuf<unsigned> cnts;  // [0] 4-wide nodes allocated, [1 + l] frontier size of level l
     HIPB(hipMalloc(&r.nodes4, size_t(numNodes) * 8 * sizeof(float4)));
-    A.take(f[0], numNodes), A.take(f[1], numNodes), A.take(cnts, kMaxLevels + kCollapseLevels + 2);
+    A.take(f[0], numNodes), A.take(f[1], numNodes), A.take(cnts, kMaxLevels4 + kCollapseLevels + 2);
     HIPB(A.status);
-    HIPB(hipMemsetAsync(cnts.p, 0, (kMaxLevels + kCollapseLevels + 2) * sizeof(unsigned), s));
+    HIPB(hipMemsetAsync(cnts.p, 0, (kMaxLevels4 + kCollapseLevels + 2) * sizeof(unsigned), s));
     kCollapseInit<<<1, 1, 0, s>>>(f[0].p, cnts.p);
     uint32_t bound = 1, levels = 0;
     for (;;) {
@@ -1226,12 +1248,12 @@ int buildBvh(const BuildArgs& a, hipStream_t s, BuildResult& r, char* err, size_
         if (!c[k]) levels = levels - kCollapseLevels + k, done = true;  // level k - 1 was the last
       if (done) break;
       bound = c[kCollapseLevels];
-      if (levels > kMaxLevels || r.numNodes4 > numNodes) {
+      if (levels > kMaxLevels4 || r.numNodes4 > numNodes) {
         std::snprintf(err, errLen, "bvh: 4-wide collapse did not terminate");
         return ASH_E_INVALID;
       }
     }
-    if (levels > kMaxLevels || r.numNodes4 > numNodes) {
+    if (levels > kMaxLevels4 || r.numNodes4 > numNodes) {
       std::snprintf(err, errLen, "bvh: 4-wide collapse did not terminate");
       return ASH_E_INVALID;
     }

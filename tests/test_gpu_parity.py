@@ -10,6 +10,7 @@ Bars (stated per test):
   AOV / weights frame-0 channels equal to 1e-5; weight image 1e-6 relative
 """
 import os
+import time
 
 import numpy as np
 import pytest
@@ -506,6 +507,62 @@ def test_clustered_build_of_any_size_matches_lbvh(renderer, tris, tmp_path):
         renderer.upload(s)
         info = renderer.build(quality=q)
         assert info["num_triangles"] == s.state.num_triangles
+        renderer.set_film(96, 64)
+        renderer.render(cam, pc, 0, 2)
+        out.append([renderer.read(0), renderer.first_hit(cam)])
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    for k in ("t", "prim_id", "normal"):
+        np.testing.assert_array_equal(out[0][1][k], out[1][1][k])
+
+
+def _degenerate(kind, n):
+    """n triangles that cluster badly, and (mixed) 3,000 ordinary ones around them."""
+    rng = np.random.default_rng(n)
+    if kind == "nested":  # each box nearest to the next smaller one's, which is nearer to its own
+        s = 0.001 * 1.02 ** np.arange(n)
+        v = np.array([[-1, -1, 0], [1, -1, 0], [0, 1, 0]]) * s[:, None, None]
+        v[..., 2] = -1e-7 * np.arange(n)[:, None]
+        return v
+    one = np.array([[0.0, 0, 0], [0.8, 0, 0.1], [0, 0.8, 0.2]])
+    if kind == "points":
+        one = np.full((3, 3), 0.25)
+    v = np.tile(one, (n, 1, 1))
+    if kind == "mixed":
+        c = rng.uniform(-1, 1, (3000, 1, 3))
+        v = np.concatenate([v, c + rng.uniform(-0.1, 0.1, (3000, 3, 3))])
+    return v
+
+
+@pytest.mark.parametrize("branching", [4, 2])
+@pytest.mark.parametrize("kind,n", [("same", 90), ("same", 700), ("same", 5000), ("points", 2000), ("mixed", 1500),
+                                    ("nested", 150), ("nested", 300), ("nested", 400)])
+def test_clustered_build_of_degenerate_meshes(renderer, kind, n, branching, tmp_path):
+    """Coincident, zero-extent and nested triangles, which cluster one pair a
+    round: the build ends in a bounded number of rounds with a tree no deeper
+    than those, and renders as the LBVH of the same triangles does, bit for bit."""
+    v = _degenerate(kind, n)
+    tris = len(v)
+    obj = "".join(f"v {a:.9f} {b:.9f} {z:.9f}\n" for a, b, z in v.reshape(-1, 3))
+    obj += "".join(f"f {3 * i + 1} {3 * i + 2} {3 * i + 3}\n" for i in range(tris))
+    (tmp_path / "soup.obj").write_text(obj)
+    (tmp_path / "scene.json").write_text(
+        '{"state": {"path_tracing": {"spp": 2, "max_path_depth": 4, "multi_channel": ["normal"]}, "output_hdr": true},'
+        ' "camera": {"type": "perspective", "film": {"resolution": [96, 64]}, "fov": 50.0},'
+        ' "materials": [{"name": "m", "type": "brdf_lambertian", "diffuse_reflectance": [0.7, 0.6, 0.5]}],'
+        ' "lights": [{"type": "rect", "radiance": [9, 9, 9], "position": [-1, 2, -1], "v1": [1, 2, -1], "v2": [-1, 2, 1]}],'
+        ' "meshes": [{"name": "soup", "path": "soup.obj"}], "instances": [{"mesh": "soup", "material": "m"}],'
+        ' "shots": [{"type": "lookat", "eye": [0, 0, 4], "lookat": [0, 0, 0], "up": [0, 1, 0]}]}')
+    s = A.HostScene(str(tmp_path / "scene.json"))
+    cam, pc = s.shot(0)
+    out = []
+    for q in (2, 0):
+        renderer.upload(s)
+        t0 = time.perf_counter()
+        info = renderer.build(quality=q, branching=branching)
+        log(f"{kind} {n}, branching {branching}, quality {q}: {(time.perf_counter() - t0) * 1e3:.1f} ms, "
+            f"depth {info['max_depth']}, {info['wide_depth']} wide levels")
+        assert info["num_triangles"] == s.state.num_triangles
+        assert info["max_depth"] <= 201  # rounds, and the leaf
         renderer.set_film(96, 64)
         renderer.render(cam, pc, 0, 2)
         out.append([renderer.read(0), renderer.first_hit(cam)])
