@@ -12,6 +12,7 @@
 
 #include "../host/scene.h"
 #include "ctx_internal.h"
+#include "tlas.h"
 
 using namespace ashd;
 
@@ -658,187 +659,6 @@ static int renderCommon(ash_ctx* c, uint32_t nShots, const ShotParams* hostShots
 }
 
 // ------------------------------------------------- two-level acceleration
-// TLAS over the instances' world boxes: a binary tree built on the host (the
-// instance count is small beside the triangle count) in the BVH2 node layout
-// (child boxes in the parent, leaf = one instance), then opened to 4-wide nodes.
-// Splits are the best of 31 planes per axis by the surface area heuristic, so
-// that a box much larger than its neighbours (a ground plane under a field of
-// instances) leaves near the root: with median splits of the box centres it sat
-// in a deep leaf, and every ancestor of it covered the scene.  256 instances of
-// four meshes on a ground quad, 4 spp: 7.04 -> 6.37 ms.  Where no plane parts the
-// centres, or the better split would make the tree deeper than `levels` more
-// levels allow, the median along the widest axis is taken.
-struct HostBox {
-  double lo[3], hi[3];
-};
-static float refBits(int32_t r) {
-  float f;
-  std::memcpy(&f, &r, 4);
-  return f;
-}
-static int32_t bitsRef(float f) {
-  int32_t r;
-  std::memcpy(&r, &f, 4);
-  return r;
-}
-static void tlasNode(std::vector<float4>& nodes, size_t at, const HostBox& L, int32_t rl, const HostBox& R, int32_t rr) {
-  auto f = [](double v, bool up) {
-    float x = float(v);
-    if (up ? double(x) < v : double(x) > v) x = std::nextafter(x, up ? INFINITY : -INFINITY);
-    return x;
-  };
-  nodes[at + 0] = make_float4(f(L.lo[0], false), f(L.hi[0], true), f(L.lo[1], false), f(L.hi[1], true));
-  nodes[at + 1] = make_float4(f(R.lo[0], false), f(R.hi[0], true), f(R.lo[1], false), f(R.hi[1], true));
-  nodes[at + 2] = make_float4(f(L.lo[2], false), f(L.hi[2], true), f(R.lo[2], false), f(R.hi[2], true));
-  nodes[at + 3] = make_float4(refBits(rl), refBits(rr), 0.f, 0.f);
-}
-// Splits items [b, e) at the plane of least cost (box area x count on either
-// side) among 31 per axis between the centres' bounds; returns the first item
-// of the second part, or b when there is none whose parts fit in trees of
-// levels - 1 levels.
-static size_t tlasSplit(const std::vector<HostBox>& box, std::vector<uint32_t>& items, size_t b, size_t e,
-                        const double* clo, const double* chi, uint32_t levels) {
-  constexpr int kBins = 32;
-  const double most = levels > 60 ? 1e18 : double(uint64_t(1) << (levels ? levels - 1 : 0));
-  auto bin = [&](uint32_t i, int ax) {
-    const double c = 0.5 * (box[i].lo[ax] + box[i].hi[ax]);
-    const double t = (c - clo[ax]) / (chi[ax] - clo[ax]) * kBins;
-    return t > 0.0 ? std::min(kBins - 1, int(t)) : 0;
-  };
-  auto area = [](const HostBox& h) {
-    const double x = h.hi[0] - h.lo[0], y = h.hi[1] - h.lo[1], z = h.hi[2] - h.lo[2];
-    return x * y + y * z + z * x;
-  };
-  auto grow = [](HostBox& h, const HostBox& k) {
-    for (int a = 0; a < 3; ++a) h.lo[a] = std::min(h.lo[a], k.lo[a]), h.hi[a] = std::max(h.hi[a], k.hi[a]);
-  };
-  const HostBox none{{INFINITY, INFINITY, INFINITY}, {-INFINITY, -INFINITY, -INFINITY}};
-  double best = INFINITY;
-  int bestAx = -1, bestBin = 0;
-  for (int ax = 0; ax < 3; ++ax) {
-    if (!(chi[ax] - clo[ax] > 0.0) || !std::isfinite(chi[ax] - clo[ax])) continue;
-    HostBox hb[kBins];
-    size_t cnt[kBins] = {};
-    for (HostBox& h : hb) h = none;
-    for (size_t k = b; k < e; ++k) {
-      const int i = bin(items[k], ax);
-      grow(hb[i], box[items[k]]);
-      ++cnt[i];
-    }
-    double right[kBins];
-    size_t nRight[kBins];
-    HostBox acc = none;
-    size_t n = 0;
-    for (int i = kBins - 1; i > 0; --i) {
-      grow(acc, hb[i]);
-      n += cnt[i];
-      right[i] = n ? area(acc) : 0.0;
-      nRight[i] = n;
-    }
-    acc = none;
-    n = 0;
-    for (int i = 1; i < kBins; ++i) {
-      grow(acc, hb[i - 1]);
-      n += cnt[i - 1];
-      if (!n || !nRight[i] || double(std::max(n, nRight[i])) > most) continue;
-      const double cost = area(acc) * double(n) + right[i] * double(nRight[i]);
-      if (cost < best) best = cost, bestAx = ax, bestBin = i;
-    }
-  }
-  if (bestAx < 0) return b;
-  auto mid = std::stable_partition(items.begin() + b, items.begin() + e, [&](uint32_t i) { return bin(i, bestAx) < bestBin; });
-  return size_t(mid - items.begin());
-}
-static int32_t tlasBuild(std::vector<float4>& nodes, std::vector<uint32_t>& order, const std::vector<HostBox>& box,
-                         std::vector<uint32_t>& items, size_t b, size_t e, HostBox& out, uint32_t depth,
-                         uint32_t levels, uint32_t& maxDepth) {
-  maxDepth = std::max(maxDepth, depth);
-  if (e - b == 1) {
-    out = box[items[b]];
-    order.push_back(items[b]);
-    return encodeLeaf(uint32_t(order.size() - 1), 1);
-  }
-  const size_t at = nodes.size();
-  nodes.resize(at + 4);
-  double clo[3] = {INFINITY, INFINITY, INFINITY}, chi[3] = {-INFINITY, -INFINITY, -INFINITY};
-  for (size_t k = b; k < e; ++k)
-    for (int a = 0; a < 3; ++a) {
-      const double cc = 0.5 * (box[items[k]].lo[a] + box[items[k]].hi[a]);
-      clo[a] = std::min(clo[a], cc), chi[a] = std::max(chi[a], cc);
-    }
-  size_t m = tlasSplit(box, items, b, e, clo, chi, levels);
-  if (m == b) {
-    int ax = 0;
-    for (int a = 1; a < 3; ++a)
-      if (chi[a] - clo[a] > chi[ax] - clo[ax]) ax = a;
-    m = b + (e - b) / 2;
-    std::nth_element(items.begin() + b, items.begin() + m, items.begin() + e, [&](uint32_t x, uint32_t y) {
-      const double cx = box[x].lo[ax] + box[x].hi[ax], cy = box[y].lo[ax] + box[y].hi[ax];
-      return cx < cy || (cx == cy && x < y);
-    });
-  }
-  HostBox L, R;
-  const int32_t rl = tlasBuild(nodes, order, box, items, b, m, L, depth + 1, levels - 1, maxDepth);
-  const int32_t rr = tlasBuild(nodes, order, box, items, m, e, R, depth + 1, levels - 1, maxDepth);
-  tlasNode(nodes, at, L, rl, R, rr);
-  for (int a = 0; a < 3; ++a) out.lo[a] = std::min(L.lo[a], R.lo[a]), out.hi[a] = std::max(L.hi[a], R.hi[a]);
-  return int32_t(at / 4);
-}
-
-// The binary TLAS as nodes of up to `width` children in the BLAS's 4-wide
-// layout, so that one step of the walk serves both levels: a node opens its
-// largest internal child until it is full.  Returns the traversal stack entries
-// that the part below node `bin` can need (one less than the children per
-// node on a path).
-static uint32_t tlasWide(const std::vector<float4>& bin, int32_t node, uint32_t width, std::vector<float4>& out) {
-  struct Kid {
-    float lo[3], hi[3];
-    int32_t ref;
-  } kid[4];
-  auto load = [&](int32_t n, Kid& a, Kid& b) {
-    const float4 *p = &bin[size_t(n) * 4], x = p[0], y = p[1], z = p[2];
-    a = Kid{{x.x, x.z, z.x}, {x.y, x.w, z.y}, bitsRef(p[3].x)};
-    b = Kid{{y.x, y.z, z.z}, {y.y, y.w, z.w}, bitsRef(p[3].y)};
-  };
-  auto internal = [](const Kid& k) { return k.ref >= 0 && k.ref != kEmptyRef; };
-  auto area = [](const Kid& k) {
-    const double x = double(k.hi[0]) - k.lo[0], y = double(k.hi[1]) - k.lo[1], z = double(k.hi[2]) - k.lo[2];
-    return x * y + y * z + z * x;
-  };
-  load(node, kid[0], kid[1]);
-  uint32_t n = 2;
-  while (n < width) {
-    int pick = -1;
-    for (uint32_t k = 0; k < n; ++k)
-      if (internal(kid[k]) && (pick < 0 || area(kid[k]) > area(kid[pick]))) pick = int(k);
-    if (pick < 0) break;
-    load(kid[pick].ref, kid[pick], kid[n]);
-    ++n;
-  }
-  const size_t at = out.size();
-  out.resize(at + 8);
-  uint32_t below = 0;
-  int32_t ref[4];
-  for (uint32_t k = 0; k < 4; ++k) {
-    if (k >= n) {
-      for (int a = 0; a < 3; ++a) kid[k].lo[a] = kid[k].hi[a] = 3.0e38f;
-      ref[k] = kEmptyRef;
-    } else if (internal(kid[k])) {
-      ref[k] = int32_t(out.size() / 8);
-      below = std::max(below, tlasWide(bin, kid[k].ref, width, out));
-    } else {
-      ref[k] = kid[k].ref;
-    }
-  }
-  for (int a = 0; a < 3; ++a) {
-    out[at + 2 * a] = make_float4(kid[0].lo[a], kid[1].lo[a], kid[2].lo[a], kid[3].lo[a]);
-    out[at + 2 * a + 1] = make_float4(kid[0].hi[a], kid[1].hi[a], kid[2].hi[a], kid[3].hi[a]);
-  }
-  out[at + 6] = make_float4(refBits(ref[0]), refBits(ref[1]), refBits(ref[2]), refBits(ref[3]));
-  out[at + 7] = make_float4(0.f, 0.f, 0.f, 0.f);
-  return n - 1 + below;
-}
-
 // One object-space BLAS per distinct mesh (instances share a mesh when
 // they share its vertex and index ranges), each built by buildBvh over a
 // single identity instance, then the TLAS.
@@ -946,36 +766,10 @@ static int buildTwoLevel(ash_ctx* c, const BuildArgs& tmpl, ash_build_info* info
     ibox[i] = w;
     items.push_back(i);
   }
-  std::vector<float4> tnodes;
-  std::vector<uint32_t> order;
-  uint32_t tdepth = 1;
-  const HostBox far{{3.0e38, 3.0e38, 3.0e38}, {3.0e38, 3.0e38, 3.0e38}};
-  if (items.size() <= 1) {
-    tnodes.resize(4);
-    if (items.empty()) {
-      tlasNode(tnodes, 0, far, kEmptyRef, far, kEmptyRef);
-    } else {
-      order.push_back(items[0]);
-      tlasNode(tnodes, 0, ibox[items[0]], encodeLeaf(0, 1), far, kEmptyRef);
-    }
-  } else {
-    // levels of the balanced tree, and as many more as fit in the smallest traversal stacks (kStackLdsMin + kSpill
-    // entries): a tree that fitted there still does, and renders with fixed scratch are refused for no other trees
-    uint32_t levels = 0;
-    while ((size_t(1) << levels) < items.size()) ++levels;
-    const uint32_t need = levels + 1 + 3 * depth4, room = uint32_t(kStackLdsMin + kSpill);
-    if (need < room) levels += std::min<uint32_t>(room - need, 16);
-    HostBox all;
-    tdepth = 0;
-    (void)tlasBuild(tnodes, order, ibox, items, 0, items.size(), all, 0, levels, tdepth);
-  }
-  // 4-wide unless that needs larger traversal stacks than the smallest ones and than the binary tree
-  std::vector<float4> wide;
-  uint32_t tlasNeed = tlasWide(tnodes, 0, 4, wide);
-  if (tlasNeed + 3 * depth4 > std::max(uint32_t(kStackLdsMin + kSpill), tdepth + 1 + 3 * depth4)) {
-    wide.clear();
-    tlasNeed = tlasWide(tnodes, 0, 2, wide);
-  }
+  // three stack entries per 4-wide BLAS level
+  const Tlas t = buildTlas(ibox, items, 3 * depth4, uint32_t(kStackLdsMin + kSpill));
+  const std::vector<float4>& wide = t.nodes;
+  const std::vector<uint32_t>& order = t.order;
   MALLOC(c, c->tlas, wide.size());
   MALLOC(c, c->tlasInst, std::max<size_t>(order.size(), 1));
   MALLOC(c, c->instBlas, std::max<size_t>(instBlas.size(), 1));
@@ -986,8 +780,8 @@ static int buildTwoLevel(ash_ctx* c, const BuildArgs& tmpl, ash_build_info* info
   if (!tab.empty()) HIPC(c, hipMemcpy(c->blasTab.p, tab.data(), tab.size() * sizeof(DevBlas), hipMemcpyHostToDevice));
   c->twoLevel = true;
   c->nodeCount = nodes4;
-  c->maxDepth = tdepth + depth4;
-  c->stackNeed = tlasNeed + 3 * depth4;  // three entries per 4-wide BLAS level
+  c->maxDepth = t.depth + depth4;
+  c->stackNeed = t.need + 3 * depth4;
   if (info) {
     std::memset(info, 0, sizeof *info);
     info->num_triangles = c->numTris;
