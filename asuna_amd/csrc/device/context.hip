@@ -335,6 +335,11 @@ static int checkPc(ash_ctx* c, const GpuPushConstantRaytrace* pc) {
   return ASH_OK;
 }
 
+// The walk of a batch's camera rays, one value where the tree or the scheme leaves no choice.
+static CameraWalk batchWalk(const ash_ctx* c, const SceneView& sc, uint32_t scheme, const BatchDesc& b) {
+  return canPacketCamera(sc, scheme) ? cameraWalk(c->numTris, b.n, b.nAcc) : kPerRay;
+}
+
 // The bounce loop of a batch.  On the default traversal scheme the shadow
 // rays of each bounce are traced in the same persistent launch as the
 // extension rays of the next one (extend, then per bounce: shade, fused
@@ -371,7 +376,7 @@ static int launchLoop(ash_ctx* c, const Wavefront& wf, const SceneView& sc, cons
   double* tShadow = st ? &st->shadow_ms : &scratch;
   double* tTrace = st ? &st->trace_ms : &scratch;
   int cur = 0;
-  const CameraWalk walk = cameraWalk(c->numTris, b.n, b.nAcc);
+  const CameraWalk walk = batchWalk(c, sc, scheme, b);
   if (!canFuseTrace(sc, scheme)) {
     launchResetCounters(wf, s);
     for (uint32_t it = 0; it < iters; ++it) {
@@ -428,7 +433,7 @@ static bool graphBounces(ash_ctx* c, const SceneView& sc, const BatchDesc& b, ui
   k.single = b.shots == 1;
   k.lds = lds;
   k.scheme = scheme;
-  k.walk = cameraWalk(c->numTris, b.n, b.nAcc);
+  k.walk = batchWalk(c, sc, scheme, b);
   ++c->graphClock;
   for (auto& g : c->graphs)
     if (g.exec && std::memcmp(&g.key, &k, sizeof k) == 0) {
@@ -577,9 +582,7 @@ static int renderCommon(ash_ctx* c, uint32_t nShots, const ShotParams* hostShots
   }
   int rc = ensureWavefront(c, cap);
   if (rc) return rc;
-  // no more blocks than give every 4 rays of the batch a wave (whole sets of XCDs)
-  const uint64_t need = (16 * ((uint64_t(cap) + kTraceBlock - 1) / kTraceBlock) + kXcds - 1) / kXcds * kXcds;
-  uint32_t grid = uint32_t(std::min<uint64_t>(uint64_t(std::max(1, c->numCU)) * bpc, need));
+  uint32_t grid = uint32_t(std::max(1, c->numCU)) * bpc;
   rc = ensureSpill(c, grid);
   if (rc) return rc;
   std::vector<WorkUnit> flat;
