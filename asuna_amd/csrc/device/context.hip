@@ -337,7 +337,7 @@ static int checkPc(ash_ctx* c, const GpuPushConstantRaytrace* pc) {
 
 // The walk of a batch's camera rays, one value where the tree or the scheme leaves no choice.
 static CameraWalk batchWalk(const ash_ctx* c, const SceneView& sc, uint32_t scheme, const BatchDesc& b) {
-  return canPacketCamera(sc, scheme) ? cameraWalk(c->numTris, b.n, b.nAcc) : kPerRay;
+  return canPacketCamera(sc, scheme) ? cameraWalk(c->numTris, b.n, b.nAcc, b.nUnits) : kPerRay;
 }
 
 // The bounce loop of a batch.  On the default traversal scheme the shadow
@@ -1453,7 +1453,7 @@ int ash_first_hit(ash_ctx* c, const GpuCamera* cam, ash_hit* out) {
   SceneView sc = viewOf(c);
   launchRaygen(b, c->wf, c->stream);
   launchResetCounters(c->wf, c->stream);
-  launchExtendCamera(sc, c->wf, kStackLds, kSchemeXcdSlices, grid, false, cameraWalk(c->numTris, P, P), c->stream);
+  launchExtendCamera(sc, c->wf, kStackLds, kSchemeXcdSlices, grid, false, cameraWalk(c->numTris, P, P, 1), c->stream);
   launchFirstHit(sc, c->shotTab.p, c->wf, dout.p, P, c->stream);
   HIPC(c, hipGetLastError());
   HIPC(c, hipMemcpyAsync(out, dout.p, P * sizeof(ash_hit), hipMemcpyDeviceToHost, c->stream));

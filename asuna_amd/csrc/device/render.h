@@ -154,24 +154,43 @@ void launchExtend(const SceneView& sc, const Wavefront& w, int cur, uint32_t lds
 // Closest hit of the camera rays (queue 0 after raygen).  On the float 4-wide
 // tree with XCD slices, cameraWalk picks the walk:
 //  - per wave (kExtendPacket), when a wave's 64 rays lie close together: from
-//    kPacketFrames frames per pixel (8 pixels per wave), or on a tree of at
-//    most kPacketTris triangles, which every wave walks whole.  kCoarse: a wave
-//    fetches 256 rays per atomic instead of 64 (for trees of at most
-//    kCoarseFetchTris triangles, whose cheap rays would otherwise wait on the
-//    fetch atomics);
+//    kPacketFrames frames per pixel (8 pixels per wave), on a tree of at most
+//    kPacketTris triangles, which every wave walks whole, and otherwise where a
+//    view is fine enough (below).  kCoarse: a wave fetches 256 rays per atomic
+//    instead of 64 (for trees of at most kCoarseFetchTris triangles, whose cheap
+//    rays would otherwise wait on the fetch atomics);
 //  - per ray (launchExtend), otherwise: with few frames a wave's rays belong to
 //    up to 64 pixels, reach different leaves, and the wave visits the union.
-// Whole render, per wave / per ray: 5.2 M triangles, 1080p: 1 frame 4.70 / 3.99
-// ms, 2: 6.32 / 5.88, 4: 9.79 / 9.61, 8: 16.85 / 16.83, 16: 30.4 / 31.2; ten
-// 256 x 256 views of a 5,450-triangle scene: 1 frame 3.21 / 2.47, 4: 3.84 /
-// 3.39; the 36-triangle box, 512 x 512: 1 frame 0.88 / 0.91, 4: 2.06 / 2.13.
 // Other schemes and trees: launchExtend.
+//
+// Fine enough: below kPacketFrames frames, fewer than 1/3 of a triangle per
+// wave's share of its view (64 / (pixels x frames) of it), or 16 of a tree above
+// kCoarseFetchTris, most of whose triangles hide one another; and more than
+// kPacketRays rays, since fewer leave most waves without a 256-ray fetch.
+// Whole render, per wave / per ray, frames in brackets:
+//   732 triangles, 96 x 64 [1] .344 / .336 ms, 512 x 512 [1] .531 / .509, [2] .694 /
+//     .763, 1280 x 720 [2] 1.456 / 1.503
+//   5,126, 512 x 512 [4] 1.308 / 1.266, 1280 x 720 [1] 1.308 / 1.339, 1920 x 1080 [7]
+//     7.50 / 7.83
+//   14,724, 160 x 120 [2] 1.130 / .728, ten views of 256 x 256 [4] 2.211 / 1.765,
+//     1920 x 1080 [1] 1.665 / 1.571, [4] 3.276 / 3.384
+//   81,926, 160 x 120 [4] 1.243 / 1.141, 1280 x 720 [1] 1.701 / 1.842
+//   5.2 M, 1920 x 1080 [1] 4.70 / 3.99, [4] 9.79 / 9.61, [8] 16.85 / 16.83, [16] 30.4 /
+//     31.2
+// Of 338 such pairs the rule takes the slower by more than 2 % in 13, by 4.6 % at
+// most (5,768 triangles, 512 x 512 [7]); always per ray below 8 frames and above
+// 512 triangles: 93 and 10 %, always per wave: 184 and 131 %.
 enum CameraWalk : uint32_t { kPerRay, kPacket, kCoarse };
-constexpr uint32_t kPacketFrames = 8, kPacketTris = 512;
+constexpr uint32_t kPacketFrames = 8, kPacketTris = 512, kPacketRays = 1u << 18;
 constexpr uint32_t kCoarseFetchTris = 1u << 16;
-inline CameraWalk cameraWalk(uint32_t numTris, uint64_t paths, uint64_t pixels) {
-  if (numTris > kPacketTris && paths < kPacketFrames * pixels) return kPerRay;
-  return numTris <= kCoarseFetchTris ? kCoarse : kPacket;
+// paths of a batch, over `pixels` pixels of `views` views together
+inline CameraWalk cameraWalk(uint32_t numTris, uint64_t paths, uint64_t pixels, uint64_t views) {
+  const bool coarse = numTris <= kCoarseFetchTris;
+  if (numTris > kPacketTris && paths < kPacketFrames * pixels) {
+    const uint64_t perShare = coarse ? 3 * 64 : 64 / 16;  // times triangles: paths of a view that is fine enough
+    if (paths <= kPacketRays || perShare * numTris * views >= paths) return kPerRay;
+  }
+  return coarse ? kCoarse : kPacket;
 }
 bool canPacketCamera(const SceneView& sc, uint32_t scheme);
 void launchExtendCamera(const SceneView& sc, const Wavefront& w, uint32_t ldsStack, uint32_t scheme, uint32_t grid,

@@ -238,3 +238,26 @@ def test_small_films_share_one_captured_loop(renderer, box_scene):
     turns = np.min([[once(w, h) for w, h in sizes] for _ in range(15)], 0)
     log(f"12 film sizes: {np.mean(alone) * 1e6:.0f} us a render alone, {np.mean(turns) * 1e6:.0f} in turns")
     assert np.mean(turns) <= 1.25 * np.mean(alone)
+
+
+@pytest.mark.parametrize("w,h,frames,views", [(1280, 802, 1, 1), (641, 480, 1, 1), (720, 401, 4, 1), (400, 300, 4, 3), (200, 100, 4, 4)])
+def test_camera_walk_by_view_size_does_not_change_images(renderer, spheres_small, w, h, frames, views):
+    """Fewer than 8 frames of 5,126 triangles on both sides of the rule's lines
+    (a third of a triangle per wave's share of a view, 2^18 rays; a view's own
+    paths count where there are several): the images are the queue-order
+    scheme's, which has one walk."""
+    s = _load(renderer, spheres_small)
+    assert s.state.num_triangles == 5126
+    _, pc = s.shot(0)
+    cams = [A.camera_lookat(w, h, 55.0, (3.0 * np.sin(k), 1.6, 3.0 * np.cos(k)), (0.0, 0.3, 0.0)) for k in range(views)]
+    out = []
+    for trav in (0, 1):
+        renderer.set_film(w, h)
+        if views == 1:
+            renderer.render(cams[0], pc, 0, frames, traversal=trav)
+            out.append([renderer.read(i) for i in (0, 8)])
+        else:
+            renderer.render_shots(cams, [pc] * views, frames, traversal=trav)
+            out.append([renderer.read_shot(k, i) for k in range(views) for i in (0, 8)])
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
