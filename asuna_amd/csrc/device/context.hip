@@ -582,7 +582,11 @@ static int renderCommon(ash_ctx* c, uint32_t nShots, const ShotParams* hostShots
   }
   int rc = ensureWavefront(c, cap);
   if (rc) return rc;
-  uint32_t grid = uint32_t(std::max(1, c->numCU)) * bpc;
+  // No more blocks than give every 4 rays of the wavefront's capacity a wave (whole sets of XCDs): the traversal's spill
+  // space is sized by the grid, and a new context's first 96 x 64 render takes 590 us in place of 690 (later ones the
+  // same).  The capacity, not this batch: the grid is part of a captured loop's key, and batches of other sizes share it.
+  const uint64_t need = (16 * ((uint64_t(c->wf.capacity) + kTraceBlock - 1) / kTraceBlock) + kXcds - 1) / kXcds * kXcds;
+  uint32_t grid = uint32_t(std::min<uint64_t>(uint64_t(std::max(1, c->numCU)) * bpc, need));
   rc = ensureSpill(c, grid);
   if (rc) return rc;
   std::vector<WorkUnit> flat;

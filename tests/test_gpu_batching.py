@@ -217,11 +217,11 @@ def test_shot_tables_of_any_size(renderer, box_scene, shots):
         np.testing.assert_array_equal(renderer.read_shot(i, 0), ref[i % 3])
 
 
-def test_small_films_share_one_captured_loop(renderer, box_scene):
+def test_small_films_share_one_captured_loop(box_scene):
     """Twelve film sizes, more than a context keeps captured loops for: a
     multi-shot render of each in turn takes no longer than the same one again
     and again.  (With a capture on every call: 516 us in place of 384, bar 480.)"""
-    s = _load(renderer, box_scene)
+    s = _load(box_scene)
     _, pc = s.shot(0)
     sizes = [(16 + 8 * k, 24) for k in range(12)]
 
@@ -237,6 +237,7 @@ def test_small_films_share_one_captured_loop(renderer, box_scene):
     alone = [min(once(w, h) for _ in range(15)) for w, h in sizes]
     turns = np.min([[once(w, h) for w, h in sizes] for _ in range(15)], 0)
     log(f"12 film sizes: {np.mean(alone) * 1e6:.0f} us a render alone, {np.mean(turns) * 1e6:.0f} in turns")
+    renderer.close()
     assert np.mean(turns) <= 1.25 * np.mean(alone)
 
 
