@@ -221,7 +221,8 @@ def test_small_films_share_one_captured_loop(box_scene):
     """Twelve film sizes, more than a context keeps captured loops for: a
     multi-shot render of each in turn takes no longer than the same one again
     and again.  (With a capture on every call: 516 us in place of 384, bar 480.)"""
-    s = _load(box_scene)
+    renderer = A.Renderer(0)  # of its own: shading launches follow the largest wavefront a context has held
+    s = _load(renderer, box_scene)
     _, pc = s.shot(0)
     sizes = [(16 + 8 * k, 24) for k in range(12)]
 
