@@ -335,3 +335,39 @@ def test_features_of_any_magnitude_reach_the_network():
     np.testing.assert_array_equal(r.read(7)[..., :3], out[0])
     r.close()
     d.close()
+
+
+@pytest.mark.parametrize("n,h,w", [(8, 272, 144), (12, 208, 176)])
+def test_cut_tiles_of_large_batches_equal_their_images(n, h, w):
+    """Batches whose two finest levels run on the 16-row tiles (16 x 32 pixels,
+    and 16 x 16 by two output groups) and the next on 8 x 32, with remainders in
+    both directions, against their images one by one, which run on the small
+    tiles that are checked against the oracle.  Bars as for the large batch; the
+    biases, summed tile by tile in the convolutions, per layer: 0.01, and two
+    pre-activations of a level's n h w co units rounded to the other side of zero."""
+    d = A.Denoiser(0, seed=37)
+    rng = np.random.default_rng(n + h + w)
+    raw = _raw(rng, n, h, w)
+    target = np.exp(rng.normal(-1.0, 1.0, size=(n, h, w, 3))).astype(np.float32)
+    out = np.log1p(d.forward(raw))
+    one = np.log1p(np.concatenate([d.forward(raw[i:i + 1]) for i in range(n)]))
+    ferr = np.linalg.norm(out - one) / np.linalg.norm(one)
+    worst = max(np.linalg.norm(out[i] - one[i]) / np.linalg.norm(one[i]) for i in range(n))
+    edge = np.linalg.norm(out[:, -16:, -32:] - one[:, -16:, -32:]) / np.linalg.norm(one[:, -16:, -32:])
+    loss, g = d.gradient(raw, target)
+    parts = [d.gradient(raw[i:i + 1], target[i:i + 1]) for i in range(n)]
+    mean = np.mean([p[1].astype(np.float64) for p in parts], 0)
+    gerr = np.linalg.norm(g - mean) / np.linalg.norm(mean)
+    log(f"{n} x {h} x {w}: forward {ferr:.5f}, worst image {worst:.5f}, last corner {edge:.5f}, gradient {gerr:.5f}")
+    assert ferr <= 0.01 and worst <= 0.01 and edge <= 0.01 and gerr <= 0.01
+    assert abs(loss - np.mean([p[0] for p in parts])) <= 1e-4 * loss
+    k = 0
+    levels = [0, 0, 1, 1, 2, 2, 3, 3, 4, 4, 3, 3, 2, 2, 1, 1, 0, 0, 0]
+    for lv, (name, a, b, o, relu) in zip(levels, U.layer_shapes()):
+        m = 9 * (a + b) * o
+        for what, s in (("weights", slice(k, k + m)), ("biases", slice(k + m, k + m + o))):
+            e = np.linalg.norm(g[s] - mean[s]) / np.linalg.norm(mean[s])
+            log(f"  {name} {what}: {e:.5f}")
+            assert e <= 0.01 + np.sqrt(8.0 / (n * (h >> lv) * (w >> lv) * o)), (name, what, e)
+        k += m + o
+    d.close()

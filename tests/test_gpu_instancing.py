@@ -188,3 +188,99 @@ def test_large_instance_grid_matches_flat(tmp_path):
     finally:
         flat.close()
         two.close()
+
+
+def _obj(path, verts):
+    with open(path, "w") as f:
+        f.write("".join("v %.9f %.9f %.9f\n" % tuple(p) for p in verts.reshape(-1, 3)))
+        f.write("".join(f"f {3 * i + 1} {3 * i + 2} {3 * i + 3}\n" for i in range(len(verts))))
+
+
+def uneven_scene(d, layout, deep):
+    """Instances of the four spheres on the ground and lights of a generated 2 x 2
+    scene.  "spread": geometrically spaced and scaled, so that the best splits
+    peel off a few boxes each; "centred": one centre, other sizes, which no
+    plane parts.  deep: one more mesh whose own tree is 49 wide levels deep
+    (150 nested triangles)."""
+    p = A.generate_scene(4, d, scale=1286)
+    j = json.load(open(p))
+    rng = np.random.default_rng(7)
+    spheres = [m["name"] for m in j["meshes"] if m["name"].startswith("sphere")]
+    inst = [i for i in j["instances"] if not i["mesh"].startswith("sphere")]
+    for k in range(160):
+        if layout == "spread":
+            r = 0.02 * 1.045 ** k  # 0.02 to 22
+            at = [r * float(v) for v in rng.uniform(-6, 6, 3)]
+            at[1] = abs(at[1])
+            s = 0.8 * r
+        else:
+            at, s = [0.0, 1.5, 0.0], 0.05 * 1.03 ** k
+        m = spheres[k % len(spheres)]
+        inst.append({"mesh": m, "material": f"m_{m}",
+                     "toworld": [{"type": "scale", "value": [s, s, s]},
+                                 {"type": "rotate", "value": [float(v) for v in rng.uniform(-180, 180, 3)]},
+                                 {"type": "translate", "value": at}]})
+    if deep:
+        n = np.arange(150)
+        v = np.array([[-1, -1, 0], [1, -1, 0], [0, 1, 0]]) * (0.001 * 1.02 ** n)[:, None, None]
+        v[..., 2] = -1e-7 * n[:, None]
+        _obj(os.path.join(d, "nested.obj"), v)
+        j["meshes"].append({"name": "nested", "path": "nested.obj"})
+        inst.append({"mesh": "nested", "material": f"m_{spheres[0]}",
+                     "toworld": [{"type": "scale", "value": [20.0, 20.0, 20.0]}, {"type": "translate", "value": [1.0, 1.0, 4.0]}]})
+    j["instances"] = inst
+    q = os.path.join(d, "uneven.json")
+    with open(q, "w") as f:
+        json.dump(j, f)
+    return q
+
+
+@pytest.mark.parametrize("deep", [False, True])
+@pytest.mark.parametrize("layout", ["spread", "centred"])
+def test_uneven_instances_match_flat(tmp_path, layout, deep):
+    """Layouts on which the tree over the instances falls back: to median splits
+    where no plane parts the centres, to the balanced tree's depth and to two
+    children per node over a BLAS deeper than the smallest stacks.  A stack entry
+    too many would be dropped: first hits and a render equal the flat tree's as
+    on the large grid."""
+    s = A.HostScene(uneven_scene(str(tmp_path), layout, deep))
+    w, h = 640, 360
+    flat, two = A.Renderer(0), A.Renderer(0)
+    try:
+        info = []
+        for r, t in ((flat, False), (two, True)):
+            r.upload(s)
+            info.append(r.build(two_level=t))
+            r.set_film(w, h)
+        n = s.desc.num_instances
+        depth = info[1]["max_depth"] - info[1]["wide_depth"]  # of the tree over the instances
+        nodes = info[1]["num_nodes"] - info[1]["num_wide_nodes"]
+        log(f"{layout}, deep {deep}: {n} instances, depth {depth}, {nodes} nodes, BLAS levels {info[1]['wide_depth']}")
+        balanced = int(np.ceil(np.log2(n)))
+        if deep:
+            assert info[1]["wide_depth"] >= 40 and depth == balanced and nodes == n - 1  # two children per node
+        else:
+            assert balanced <= depth <= balanced + 16 and nodes < n - 1
+            assert layout != "spread" or depth > balanced
+        for eye in ((0.0, 3.0, 14.0), (30.0, 25.0, 30.0)):
+            cam = A.camera_lookat(w, h, 50.0, eye, (0.0, 1.0, 0.0))
+            f, g = flat.first_hit(cam), two.first_hit(cam)
+            same = (f["prim_id"] == g["prim_id"]) & (f["inst_id"] == g["inst_id"])
+            hit = same & (f["inst_id"] >= 0)
+            tie = ~same & (f["inst_id"] >= 0) & (g["inst_id"] >= 0) & (np.abs(f["t"] - g["t"]) <= 1e-4 * np.abs(f["t"]))
+            other = ~same & ~tie
+            log(f"  same ids {same.mean():.6f}, hits {hit.mean():.4f}, {int(tie.sum())} ties, {int(other.sum())} other")
+            assert same.mean() >= 0.9995 and other.mean() <= 2e-4 and hit.mean() > 0.2
+            np.testing.assert_array_equal(f["t"][hit], g["t"][hit])
+            np.testing.assert_array_equal(f["normal"][hit], g["normal"][hit])
+            _, pc = s.shot(0)
+            img = []
+            for r in (flat, two):
+                r.set_film(w, h)
+                r.render(cam, pc, 0, 4)
+                img.append(r.read(0)[..., :3])
+            assert abs(img[0].mean() - img[1].mean()) <= 2e-3 * img[0].mean()
+            assert np.mean(np.abs(img[0] - img[1]).max(-1) > 1e-3) <= 0.02
+    finally:
+        flat.close()
+        two.close()
