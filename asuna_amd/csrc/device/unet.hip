@@ -283,10 +283,10 @@ __device__ __forceinline__ void tileBias(const ConvArgs& a, uint32_t cg, uint32_
 // Each wave computes R rows x 16 columns x 32 channels: an input fragment
 // (one row, one column shift) is read once and feeds the three taps of its
 // column shift, i.e. up to 6 MFMAs, so that per chunk a wave reads 3 (R + 2)
-// input and 18 weight fragments for 18 R MFMAs and the matrix cores, not
-// the LDS, are the limit (R = 8: 48 KB of LDS reads, 384 cycles of the CU's
-// 128 bytes per cycle, against 576 matrix cycles per SIMD).  The loads of the
-// next chunk (or the next tile's first) are in flight in registers during
+// input and 18 weight fragments for 18 R MFMAs and the LDS asks for less time
+// than the matrix cores (R = 8: the block's four waves read 192 KB, 1536 cycles of
+// the CU's 128 bytes per cycle, against 2304 cycles of 16 per MFMA on each SIMD).
+// The loads of the next chunk (or the next tile's first) are in flight in registers during
 // the MFMAs.  Blocks are persistent; with one chunk the weights stay in LDS.
 //
 // A pixel's four 16-byte slots are swizzled by its column (slot ^ column / 4),
@@ -449,7 +449,7 @@ __global__ __launch_bounds__(256, R == 8 ? 2 : 3) void kConvLds(ConvArgs a, uint
 // the image) and computes the 14 x 30 pixels of the second whose neighbours it
 // holds: 1.22 times the MFMAs for one read and one write less.  Both layers'
 // weights stay in LDS.  1080p film: features and the two layers 60 + 80 + 85 us
-// before, the last two 88 + 68; 129 and 113 us in one.
+// before, the last two 88 + 68; 133 and 112 us in one.
 struct FilmSrc {
   const float4 *rad, *alb, *nrm, *dep;  // planes of W x H pixels; all but rad may be null
   uint32_t W, H;
@@ -918,7 +918,7 @@ __global__ __launch_bounds__(256) void kPackW(LayerTab T, const float* theta, ui
 // Parameter gradients from the partial sums, and (ADAM) the optimiser step
 // and the packed weights, for 32 parameters per block: eight groups of 32
 // threads each add an eighth of a parameter's partial sums in order, then the
-// groups' sums are added in group order.  One launch of 70 us for a batch of
+// groups' sums are added in group order.  One launch of 45 us for a batch of
 // 8 x 128 x 128, where per-layer reductions of weights (8 us) and biases (one
 // block, 41 us), the Adam pass and 19 packing launches took 1.1 ms.
 struct AdamArgs {
