@@ -40,8 +40,8 @@ inline int32_t bitsRef(float f) {
 //
 // Items are moved instead of pointed to, all three axes are binned with one vector
 // operation each, and a node of few items gets few bins.  2,304 and 100,000
-// instances in a field: 0.8 and 47 ms on the build machine's CPU, as long as the
-// median splits took (0.9 and 47); with index lists, 32 bins at every node and two
+// instances in a field: 0.8 and 47 ms on a 2.7 GHz Xeon, as long as the median
+// splits took (0.9 and 47); with index lists, 32 bins at every node and two
 // bin computations per item and axis it was 2.4 and 131.
 class TlasBuilder {
  public:
